@@ -115,6 +115,14 @@ int matgptq_reorder_scales_host(const uint16_t *in_host, int64_t N, int64_t K, i
  * Asynchronous on `stream`. */
 int matgptq_pack_device(const uint8_t *codes_dev, int64_t N, int64_t K, int bitwidth,
                         int slice_from_master, uint32_t *out_dev, void *stream);
+/* A whole layer in one launch: the codes and the per-group tensors [N, K/g] (scales, optionally zeros;
+ * any 16-bit type) into the kernels' order.  source: 0 = codes already sliced to `bitwidth`, 1 = 8-bit
+ * master codes to be sliced, 2 = master codes to resident planes (packed_dev: matgptq_master_words).
+ * Same results as matgptq_pack_device / matgptq_pack_master_device and matgptq_reorder_scales_device. */
+int matgptq_pack_layer_device(const uint8_t *codes_dev, int64_t N, int64_t K, int bitwidth, int group_size,
+                              int source, const uint16_t *scales_dev, const uint16_t *zeros_dev_or_null,
+                              uint32_t *packed_dev, uint16_t *scales_out_dev, uint16_t *zeros_out_dev_or_null,
+                              void *stream);
 int matgptq_unpack_device(const uint32_t *packed_dev, int64_t N, int64_t K, int bitwidth,
                           uint8_t *codes_dev, void *stream);
 int matgptq_reorder_scales_device(const uint16_t *in_dev, int64_t N, int64_t K, int group_size,

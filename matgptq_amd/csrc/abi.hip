@@ -41,10 +41,10 @@ MATGPTQ_DECL(6)
 MATGPTQ_DECL(8)
 #undef MATGPTQ_DECL
 
-hipError_t launch_pack(const uint8_t*, int64_t, int64_t, int, int, uint32_t*, hipStream_t);
+hipError_t launch_pack_layer(const uint8_t*, int64_t, int64_t, int, int, int, const uint16_t*, const uint16_t*, uint32_t*,
+                             uint16_t*, uint16_t*, hipStream_t);
 hipError_t launch_unpack(const uint32_t*, int64_t, int64_t, int, uint8_t*, hipStream_t);
 hipError_t launch_slice(const uint8_t*, int64_t, int, uint8_t*, hipStream_t);
-hipError_t launch_pack_master(const uint8_t*, int64_t, int64_t, uint32_t*, hipStream_t);
 hipError_t launch_master_slice(const uint32_t*, int64_t, int64_t, int, bool, void*, hipStream_t);
 hipError_t launch_reorder(const uint16_t*, int64_t, int64_t, uint16_t*, hipStream_t);
 hipError_t launch_tail_gemm(int bits, bool bf16, const GemmArgs&, int group_size, hipStream_t);
@@ -812,8 +812,8 @@ int matgptq_pack_master_device(const uint8_t* codes_dev, int64_t N, int64_t K, u
   if (int e = check_problem(8, -1, N, K)) return e;
   if (K % 128 != 0) return MATGPTQ_ESHAPE;
   if (!codes_dev || !planes_dev) return MATGPTQ_ENULL;
-  return launch_pack_master(codes_dev, N, K, planes_dev, static_cast<hipStream_t>(stream)) == hipSuccess
-             ? MATGPTQ_OK : MATGPTQ_ELAUNCH;
+  return launch_pack_layer(codes_dev, N, K, 8, -1, 2, nullptr, nullptr, planes_dev, nullptr, nullptr,
+                           static_cast<hipStream_t>(stream)) == hipSuccess ? MATGPTQ_OK : MATGPTQ_ELAUNCH;
 }
 
 int matgptq_unpack_master_device(const uint32_t* planes_dev, int64_t N, int64_t K, int bitwidth,
@@ -859,8 +859,20 @@ int matgptq_pack_device(const uint8_t* codes_dev, int64_t N, int64_t K, int bitw
                         int slice_from_master, uint32_t* out_dev, void* stream) {
   if (int e = check_problem(bitwidth, -1, N, K)) return e;
   if (!codes_dev || !out_dev) return MATGPTQ_ENULL;
-  return launch_pack(codes_dev, N, K, bitwidth, slice_from_master, out_dev,
-                     static_cast<hipStream_t>(stream)) == hipSuccess ? MATGPTQ_OK : MATGPTQ_ELAUNCH;
+  return launch_pack_layer(codes_dev, N, K, bitwidth, -1, slice_from_master != 0 ? 1 : 0, nullptr, nullptr, out_dev, nullptr,
+                           nullptr, static_cast<hipStream_t>(stream)) == hipSuccess ? MATGPTQ_OK : MATGPTQ_ELAUNCH;
+}
+
+int matgptq_pack_layer_device(const uint8_t* codes_dev, int64_t N, int64_t K, int bitwidth, int group_size, int source,
+                              const uint16_t* scales_dev, const uint16_t* zeros_dev, uint32_t* packed_dev,
+                              uint16_t* scales_out_dev, uint16_t* zeros_out_dev, void* stream) {
+  if (int e = check_problem(bitwidth, group_size, N, K)) return e;
+  if (source < 0 || source > 2) return MATGPTQ_EVARIANT;
+  if (source == 2 && K % 128 != 0) return MATGPTQ_ESHAPE;
+  if (!codes_dev || !packed_dev || !scales_dev || !scales_out_dev || (zeros_dev == nullptr) != (zeros_out_dev == nullptr))
+    return MATGPTQ_ENULL;
+  return launch_pack_layer(codes_dev, N, K, bitwidth, group_size, source, scales_dev, zeros_dev, packed_dev, scales_out_dev,
+                           zeros_out_dev, static_cast<hipStream_t>(stream)) == hipSuccess ? MATGPTQ_OK : MATGPTQ_ELAUNCH;
 }
 
 int matgptq_unpack_device(const uint32_t* packed_dev, int64_t N, int64_t K, int bitwidth,

@@ -4,43 +4,80 @@
 // device-side view of the packed codes.  All are byte/integer work, HBM-bound.
 #include "device_common.h"
 #include "master_layout.h"
+#include "swar_codec.h"
 
 namespace matgptq {
 
 namespace {
 
-// One thread = one lane slot of one tile: 32 codes in, BITS words out.
-template <int BITS>
+// Per-group tensors a pack launch puts into the kernels' order along with the codes (null outputs: none).
+struct PackAux {
+  const uint16_t *s_in, *z_in;  // [N, G]
+  uint16_t *s_out, *z_out;      // [N/16][G][16]
+  int G, groups_per_tile;       // groups_per_tile 0: one group per row
+};
+
+// tiles of K a workgroup of the packing kernel takes
+constexpr int kPackTiles = 8;
+
+// Codes [N, K] -> packed tiles (PLANES false: the b-bit layout, SLICE: from 8-bit master codes; PLANES
+// true: the master-resident planes).  A thread packs two neighbouring lane slots (k-quarters 2p and 2p + 1
+// of a row: 16 bytes of each octet), half a wave a tile; a workgroup takes eight neighbouring tiles of a
+// row block and, when asked, reorders the scales and zeros of their groups, so that loading a layer is
+// one launch.
+// Bound: HBM (1 byte per code in, b/8 out).  The codes are sliced and packed four at a time on the
+// bytes of a word (swar_codec.h): about 70 vector instructions per slot where one code after another
+// took some 300 and the kernel was bound by them, and a tile is found without a 64-bit division
+// (28672 x 4096 from master codes, us before / now: 2 bits 42 / 26, 3 bits 46 / 27, 4 bits 38 / 29, 6 bits
+// 47 / 35, 8 bits 36 / 37, planes 61 / 37; a copy moves the 4-bit case's 176 MB in 36).
+template <int BITS, bool SLICE, bool PLANES>
 __global__ void __launch_bounds__(256)
-pack_kernel(const uint8_t* __restrict__ codes, uint32_t* __restrict__ out, int k_tiles,
-            int64_t K, int64_t total_slots, int slice) {
-  const int64_t slot = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (slot >= total_slots) return;
-  const int lane = (int)(slot & 63);
-  const int64_t tile = slot >> 6;
-  const int64_t rb = tile / k_tiles, kb = tile - rb * k_tiles;
-  const int r = lane & 15, q = lane >> 4;
-  const uint8_t* row = codes + (rb * 16 + r) * K + kb * 128 + q * 8;
-  uint8_t c[32];
+pack_kernel(const uint8_t* __restrict__ codes, uint32_t* __restrict__ out, int k_tiles, int64_t K, int row_blocks,
+            PackAux aux) {
+  const int r = threadIdx.x & 15, p = (threadIdx.x >> 4) & 1;
+  const int kb = blockIdx.x * kPackTiles + (threadIdx.x >> 5);
+  for (int rb = blockIdx.y; rb < row_blocks; rb += gridDim.y) {
+    if (kb < k_tiles) {
+      const uint8_t* slot = codes + ((int64_t)rb * 16 + r) * K + kb * 128 + p * 16;
+      uint4 v[4];
 #pragma unroll
-  for (int j = 0; j < 4; j++) {
-    const uint2 v = *reinterpret_cast<const uint2*>(row + j * 32);
-    const uint32_t lo = v.x, hi = v.y;
+      for (int j = 0; j < 4; j++) v[j] = *reinterpret_cast<const uint4*>(slot + j * 32);
+      const int64_t tile = (int64_t)rb * k_tiles + kb;
 #pragma unroll
-    for (int e = 0; e < 4; e++) {
-      c[j * 8 + e] = (uint8_t)(lo >> (8 * e));
-      c[j * 8 + 4 + e] = (uint8_t)(hi >> (8 * e));
+      for (int h = 0; h < 2; h++) {
+        const int lane = (2 * p + h) * 16 + r;
+        uint2 c[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) c[j] = h == 0 ? make_uint2(v[j].x, v[j].y) : make_uint2(v[j].z, v[j].w);
+        if constexpr (PLANES) {
+          uint32_t w[8];
+          pack_slot_planes(c, w);
+          uint32_t* t = out + tile * kMasterTileWords;
+          *reinterpret_cast<uint3*>(t + lane * 3) = make_uint3(w[0], w[1], w[2]);
+          t[192 + lane] = w[3];
+          t[256 + lane] = w[4];
+          *reinterpret_cast<uint3*>(t + 320 + lane * 3) = make_uint3(w[5], w[6], w[7]);
+        } else {
+          uint32_t w[BITS];
+          pack_slot<BITS, SLICE>(c, w);
+          store_tile_words<BITS>(out + tile * tile_words(BITS), lane, w);
+        }
+      }
+    }
+    if (aux.s_out != nullptr) {
+      // the groups of this workgroup's tiles; the last workgroup of a row block also takes those of a
+      // tail of 64 columns
+      const int per = kPackTiles * aux.groups_per_tile;
+      const int g0 = blockIdx.x * per;
+      const int g1 = per == 0 ? (blockIdx.x == 0 ? 1 : 0) : blockIdx.x + 1 == gridDim.x ? aux.G : g0 + per;
+      for (int i = threadIdx.x; i < (g1 - g0) * 16; i += 256) {
+        const int g = g0 + (i >> 4);
+        const int64_t from = ((int64_t)rb * 16 + (i & 15)) * aux.G + g, to = ((int64_t)rb * aux.G + g) * 16 + (i & 15);
+        aux.s_out[to] = aux.s_in[from];
+        if (aux.z_out != nullptr) aux.z_out[to] = aux.z_in[from];
+      }
     }
   }
-  if (slice) {
-#pragma unroll
-    for (int i = 0; i < 32; i++) c[i] = slice_code(c[i], BITS);
-  }
-  uint32_t w[BITS];
-  Codec<BITS>::encode_lane(c, w);
-  uint32_t* t = out + tile * tile_words(BITS);
-#pragma unroll
-  for (int i = 0; i < BITS; i++) t[word_offset(BITS, lane, i)] = w[i];
 }
 
 template <int BITS>
@@ -75,17 +112,20 @@ unpack_kernel(const uint32_t* __restrict__ packed, uint8_t* __restrict__ codes, 
   emit(std::integral_constant<int, 3>{});
 }
 
+// one thread = 16 codes, sliced four at a time on the bytes of a word (117 M codes: 55 -> 33 us)
+template <int BITS>
 __global__ void __launch_bounds__(256)
-slice_kernel(const uint8_t* __restrict__ in, uint8_t* __restrict__ out, int64_t count, int bits) {
-  const int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 4;
-  if (i + 4 <= count && ((reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(out)) & 3) == 0) {
-    const uint32_t v = *reinterpret_cast<const uint32_t*>(in + i);
-    uint32_t o = 0;
-#pragma unroll
-    for (int e = 0; e < 4; e++) o |= (uint32_t)slice_code((uint8_t)(v >> (8 * e)), bits) << (8 * e);
-    *reinterpret_cast<uint32_t*>(out + i) = o;
+slice_kernel(const uint8_t* __restrict__ in, uint8_t* __restrict__ out, int64_t count) {
+  const int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 16;
+  if (i + 16 <= count && ((reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(out)) & 15) == 0) {
+    uint4 v = *reinterpret_cast<const uint4*>(in + i);
+    v.x = slice_bytes<BITS>(v.x);
+    v.y = slice_bytes<BITS>(v.y);
+    v.z = slice_bytes<BITS>(v.z);
+    v.w = slice_bytes<BITS>(v.w);
+    *reinterpret_cast<uint4*>(out + i) = v;
   } else {
-    for (int64_t e = i; e < count && e < i + 4; e++) out[e] = slice_code(in[e], bits);
+    for (int64_t e = i; e < count && e < i + 16; e++) out[e] = slice_code(in[e], BITS);
   }
 }
 
@@ -143,73 +183,49 @@ dequant_kernel(const uint32_t* __restrict__ packed, const uint16_t* __restrict__
 }
 
 // ---- master-resident bit planes (master_layout.h) --------------------------------------
-// 32 codes of a lane slot from row-major uint8 [N, K]
-__device__ __forceinline__ void read_lane_codes(const uint8_t* __restrict__ row, uint8_t (&c)[32]) {
-#pragma unroll
-  for (int j = 0; j < 4; j++) {
-    const uint2 v = *reinterpret_cast<const uint2*>(row + j * 32);
-#pragma unroll
-    for (int e = 0; e < 4; e++) {
-      c[j * 8 + e] = (uint8_t)(v.x >> (8 * e));
-      c[j * 8 + 4 + e] = (uint8_t)(v.y >> (8 * e));
-    }
-  }
-}
-
-// master codes [N, K] -> bit planes; one thread = one lane slot of one tile
-__global__ void __launch_bounds__(256)
-pack_master_kernel(const uint8_t* __restrict__ codes, uint32_t* __restrict__ out, int k_tiles,
-                   int64_t K, int64_t total_slots) {
-  const int64_t slot = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (slot >= total_slots) return;
-  const int lane = (int)(slot & 63);
-  const int64_t tile = slot >> 6;
-  const int64_t rb = tile / k_tiles, kb = tile - rb * k_tiles;
-  uint8_t c[32];
-  read_lane_codes(codes + (rb * 16 + (lane & 15)) * K + kb * 128 + (lane >> 4) * 8, c);
-  uint32_t w[8];
-  master_encode_lane(c, w);
-  uint32_t* t = out + tile * kMasterTileWords;
-#pragma unroll
-  for (int i = 0; i < 8; i++) t[master_word_offset(lane, i)] = w[i];
-}
-
 // bit planes -> codes sliced to BITS with the sequence the GEMM kernels run:
 // SLICED_PACKED false: uint8 [N, K] (bit-exactness checks);
 // SLICED_PACKED true : the pre-sliced tile layout of layout.h (input of the kernels that do not
 //                      read the planes themselves)
+// Bound: HBM.  A nibble word of the planes is a nibble word of the packed layout, so nothing is unpacked
+// to single codes on the way (28672 x 4096, us before / now: 2 bits 23 / 13, 3 bits 34 / 18, 4 bits 26 / 21,
+// 6 bits 50 / 34, 8 bits 42 / 35).
 template <int BITS, bool SLICED_PACKED>
 __global__ void __launch_bounds__(256)
-master_slice_kernel(const uint32_t* __restrict__ planes, void* __restrict__ out, int k_tiles,
-                    int64_t K, int64_t total_slots) {
-  const int64_t slot = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (slot >= total_slots) return;
-  const int lane = (int)(slot & 63);
-  const int64_t tile = slot >> 6;
-  const int64_t rb = tile / k_tiles, kb = tile - rb * k_tiles;
-  const uint32_t* t = planes + tile * kMasterTileWords;
-  uint32_t w[8];
+master_slice_kernel(const uint32_t* __restrict__ planes, void* __restrict__ out, int k_tiles, int64_t K, int row_blocks) {
+  const int lane = threadIdx.x & 63;
+  const int kb = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (kb >= k_tiles) return;
+  for (int rb = blockIdx.y; rb < row_blocks; rb += gridDim.y) {
+    const int64_t tile = (int64_t)rb * k_tiles + kb;
+    const uint32_t* t = planes + tile * kMasterTileWords;
+    uint32_t w[8] = {};
+    const uint3 s0 = *reinterpret_cast<const uint3*>(t + lane * 3);
+    w[0] = s0.x; w[1] = s0.y; w[2] = s0.z;
+    if constexpr (BITS >= 3) w[3] = t[192 + lane];
+    if constexpr (BITS >= 4) w[4] = t[256 + lane];
+    if constexpr (BITS >= 6) {
+      const uint3 s3 = *reinterpret_cast<const uint3*>(t + 320 + lane * 3);
+      w[5] = s3.x; w[6] = s3.y; w[7] = s3.z;
+    }
+    if constexpr (SLICED_PACKED) {
+      uint32_t pw[BITS];
+      pack_slot_from_planes<BITS>(w, pw);
+      store_tile_words<BITS>(static_cast<uint32_t*>(out) + tile * tile_words(BITS), lane, pw);
+    } else {
+      uint8_t c[32];
+      master_decode_lane<BITS>(w, c);
+      uint8_t* row = static_cast<uint8_t*>(out) + ((int64_t)rb * 16 + (lane & 15)) * K + kb * 128 + (lane >> 4) * 8;
 #pragma unroll
-  for (int i = 0; i < 8; i++) w[i] = i < master_words(BITS) ? t[master_word_offset(lane, i)] : 0u;
-  uint8_t c[32];
-  master_decode_lane<BITS>(w, c);
-  if constexpr (SLICED_PACKED) {
-    uint32_t pw[BITS];
-    Codec<BITS>::encode_lane(c, pw);
-    uint32_t* o = static_cast<uint32_t*>(out) + tile * tile_words(BITS);
+      for (int j = 0; j < 4; j++) {
+        uint32_t lo = 0, hi = 0;
 #pragma unroll
-    for (int i = 0; i < BITS; i++) o[word_offset(BITS, lane, i)] = pw[i];
-  } else {
-    uint8_t* row = static_cast<uint8_t*>(out) + (rb * 16 + (lane & 15)) * K + kb * 128 + (lane >> 4) * 8;
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-      uint32_t lo = 0, hi = 0;
-#pragma unroll
-      for (int e = 0; e < 4; e++) {
-        lo |= (uint32_t)c[j * 8 + e] << (8 * e);
-        hi |= (uint32_t)c[j * 8 + 4 + e] << (8 * e);
+        for (int e = 0; e < 4; e++) {
+          lo |= (uint32_t)c[j * 8 + e] << (8 * e);
+          hi |= (uint32_t)c[j * 8 + 4 + e] << (8 * e);
+        }
+        *reinterpret_cast<uint2*>(row + j * 32) = make_uint2(lo, hi);
       }
-      *reinterpret_cast<uint2*>(row + j * 32) = make_uint2(lo, hi);
     }
   }
 }
@@ -378,21 +394,44 @@ hipError_t launch_tail_gemm(int bits, bool bf16, const GemmArgs& a, int group_si
   return hipGetLastError();
 }
 
-hipError_t launch_pack(const uint8_t* codes, int64_t N, int64_t K, int bits, int slice,
-                       uint32_t* out, hipStream_t s) {
+// grid of the kernels in which a workgroup takes `per` neighbouring tiles of a row block
+static dim3 tile_grid(int k_tiles, int64_t row_blocks, int per) {
+  return dim3((unsigned)((k_tiles + per - 1) / per), (unsigned)(row_blocks < 65535 ? row_blocks : 65535));
+}
+
+// source: 0 = codes already sliced, 1 = 8-bit master codes to be sliced, 2 = master codes to resident
+// planes.  s_out (with s_in; z_out with z_in): also reorder the per-group tensors of the layer.
+hipError_t launch_pack_layer(const uint8_t* codes, int64_t N, int64_t K, int bits, int group_size, int source,
+                             const uint16_t* s_in, const uint16_t* z_in, uint32_t* out, uint16_t* s_out,
+                             uint16_t* z_out, hipStream_t s) {
   const int k_tiles = (int)(K / 128);
-  const int64_t slots = (N / 16) * (int64_t)k_tiles * 64;
-  const dim3 grid(blocks_for(slots, 256)), block(256);
-  switch (bits) {
-    case 2: hipLaunchKernelGGL(pack_kernel<2>, grid, block, 0, s, codes, out, k_tiles, K, slots, slice); break;
-    case 3: hipLaunchKernelGGL(pack_kernel<3>, grid, block, 0, s, codes, out, k_tiles, K, slots, slice); break;
-    case 4: hipLaunchKernelGGL(pack_kernel<4>, grid, block, 0, s, codes, out, k_tiles, K, slots, slice); break;
-    case 6: hipLaunchKernelGGL(pack_kernel<6>, grid, block, 0, s, codes, out, k_tiles, K, slots, slice); break;
-    default: hipLaunchKernelGGL(pack_kernel<8>, grid, block, 0, s, codes, out, k_tiles, K, slots, slice); break;
+  const int64_t row_blocks = N / 16;
+  const PackAux aux{s_in, z_in, s_out, z_out, group_size == -1 ? 1 : (int)(K / group_size),
+                    group_size == -1 ? 0 : 128 / group_size};
+  const dim3 grid = tile_grid(k_tiles, row_blocks, kPackTiles), block(256);
+#define MATGPTQ_PACK(B)                                                                                              \
+  case B:                                                                                                            \
+    if (source != 0) hipLaunchKernelGGL((pack_kernel<B, true, false>), grid, block, 0, s, codes, out, k_tiles, K,     \
+                                        (int)row_blocks, aux);                                                       \
+    else hipLaunchKernelGGL((pack_kernel<B, false, false>), grid, block, 0, s, codes, out, k_tiles, K, (int)row_blocks, aux); \
+    break;
+  if (source == 2) {
+    hipLaunchKernelGGL((pack_kernel<8, false, true>), grid, block, 0, s, codes, out, k_tiles, K, (int)row_blocks, aux);
+  } else {
+    switch (bits) {
+      MATGPTQ_PACK(2)
+      MATGPTQ_PACK(3)
+      MATGPTQ_PACK(4)
+      MATGPTQ_PACK(6)
+      default:
+        hipLaunchKernelGGL((pack_kernel<8, false, false>), grid, block, 0, s, codes, out, k_tiles, K, (int)row_blocks, aux);
+        break;
+    }
+    if (K % 128 != 0)
+      hipLaunchKernelGGL(pack_tail_kernel, dim3(blocks_for(N, 256)), block, 0, s, codes,
+                         out + tail_offset_words(N, K, bits), N, K, bits, source);
   }
-  if (K % 128 != 0)
-    hipLaunchKernelGGL(pack_tail_kernel, dim3(blocks_for(N, 256)), block, 0, s, codes, out + tail_offset_words(N, K, bits),
-                       N, K, bits, slice);
+#undef MATGPTQ_PACK
   return hipGetLastError();
 }
 
@@ -414,23 +453,15 @@ hipError_t launch_unpack(const uint32_t* packed, int64_t N, int64_t K, int bits,
   return hipGetLastError();
 }
 
-hipError_t launch_pack_master(const uint8_t* codes, int64_t N, int64_t K, uint32_t* out, hipStream_t s) {
-  const int k_tiles = (int)(K / 128);
-  const int64_t slots = (N / 16) * (int64_t)k_tiles * 64;
-  hipLaunchKernelGGL(pack_master_kernel, dim3(blocks_for(slots, 256)), dim3(256), 0, s, codes, out, k_tiles, K, slots);
-  return hipGetLastError();
-}
-
 // sliced_packed: write the pre-sliced tile layout instead of uint8 [N, K]
 hipError_t launch_master_slice(const uint32_t* planes, int64_t N, int64_t K, int bits, bool sliced_packed,
                                void* out, hipStream_t s) {
-  const int k_tiles = (int)(K / 128);
-  const int64_t slots = (N / 16) * (int64_t)k_tiles * 64;
-  const dim3 grid(blocks_for(slots, 256)), block(256);
+  const int k_tiles = (int)(K / 128), row_blocks = (int)(N / 16);
+  const dim3 grid = tile_grid(k_tiles, row_blocks, 4), block(256);
 #define MATGPTQ_MS(B)                                                                                         \
   case B:                                                                                                     \
-    if (sliced_packed) hipLaunchKernelGGL((master_slice_kernel<B, true>), grid, block, 0, s, planes, out, k_tiles, K, slots); \
-    else hipLaunchKernelGGL((master_slice_kernel<B, false>), grid, block, 0, s, planes, out, k_tiles, K, slots);  \
+    if (sliced_packed) hipLaunchKernelGGL((master_slice_kernel<B, true>), grid, block, 0, s, planes, out, k_tiles, K, row_blocks); \
+    else hipLaunchKernelGGL((master_slice_kernel<B, false>), grid, block, 0, s, planes, out, k_tiles, K, row_blocks);  \
     break;
   switch (bits) {
     MATGPTQ_MS(2)
@@ -438,8 +469,8 @@ hipError_t launch_master_slice(const uint32_t* planes, int64_t N, int64_t K, int
     MATGPTQ_MS(4)
     MATGPTQ_MS(6)
     default:
-      if (sliced_packed) hipLaunchKernelGGL((master_slice_kernel<8, true>), grid, block, 0, s, planes, out, k_tiles, K, slots);
-      else hipLaunchKernelGGL((master_slice_kernel<8, false>), grid, block, 0, s, planes, out, k_tiles, K, slots);
+      if (sliced_packed) hipLaunchKernelGGL((master_slice_kernel<8, true>), grid, block, 0, s, planes, out, k_tiles, K, row_blocks);
+      else hipLaunchKernelGGL((master_slice_kernel<8, false>), grid, block, 0, s, planes, out, k_tiles, K, row_blocks);
       break;
   }
 #undef MATGPTQ_MS
@@ -447,8 +478,14 @@ hipError_t launch_master_slice(const uint32_t* planes, int64_t N, int64_t K, int
 }
 
 hipError_t launch_slice(const uint8_t* in, int64_t count, int bits, uint8_t* out, hipStream_t s) {
-  const dim3 grid(blocks_for((count + 3) / 4, 256)), block(256);
-  hipLaunchKernelGGL(slice_kernel, grid, block, 0, s, in, out, count, bits);
+  const dim3 grid(blocks_for((count + 15) / 16, 256)), block(256);
+  switch (bits) {
+    case 2: hipLaunchKernelGGL(slice_kernel<2>, grid, block, 0, s, in, out, count); break;
+    case 3: hipLaunchKernelGGL(slice_kernel<3>, grid, block, 0, s, in, out, count); break;
+    case 4: hipLaunchKernelGGL(slice_kernel<4>, grid, block, 0, s, in, out, count); break;
+    case 6: hipLaunchKernelGGL(slice_kernel<6>, grid, block, 0, s, in, out, count); break;
+    default: hipLaunchKernelGGL(slice_kernel<8>, grid, block, 0, s, in, out, count); break;
+  }
   return hipGetLastError();
 }
 

@@ -136,6 +136,41 @@ Tensor reorder_matgptq_scales(const Tensor& scales, int64_t n_out_features, int6
   return out;
 }
 
+// A layer on the GPU in one launch: codes packed, scales and zeros reordered.  source: 0 = sliced codes,
+// 1 = 8-bit master codes, 2 = master codes to resident planes.  Returns (packed, scales[, zeros]).
+std::vector<Tensor> pack_matgptq_layer(const Tensor& qweights, const Tensor& scales, const c10::optional<Tensor>& zeros,
+                                       int64_t bitwidth, int64_t group_size, int64_t source) {
+  TORCH_CHECK(qweights.is_cuda(), "pack_matgptq_layer: qweights must be on the GPU");
+  TORCH_CHECK(qweights.dtype() == torch::kUInt8, "qweights must be uint8");
+  TORCH_CHECK(qweights.dim() == 2 && qweights.is_contiguous(), "qweights must be contiguous and 2D (n_out_features, n_in_features)");
+  const int64_t n = qweights.size(0), k = qweights.size(1);
+  check_bits_group(bitwidth, group_size, k);
+  check_tiling(n, k, source == 2);
+  const int64_t groups = group_size == -1 ? 1 : k / group_size;
+  auto check_per_group = [&](const Tensor& t) {
+    TORCH_CHECK(t.device() == qweights.device() && t.is_contiguous(), "scales and zeros must be contiguous and on the GPU of qweights");
+    TORCH_CHECK(t.dtype() == torch::kFloat16 || t.dtype() == torch::kBFloat16, "scales must be float16 or bfloat16");
+    TORCH_CHECK(t.dim() == 2 && t.size(0) == n && t.size(1) == groups,
+                "scales must have shape (n_out_features, n_in_features / group_size)");
+  };
+  check_per_group(scales);
+  if (zeros.has_value()) check_per_group(*zeros);
+  const at::Device dev = qweights.device();
+  c10::hip::HIPGuardMasqueradingAsCUDA guard(dev);
+  std::vector<Tensor> out;
+  out.push_back(torch::empty({(source == 2 ? 8 : bitwidth) * n * k / 32}, qweights.options().dtype(torch::kUInt32)));
+  out.push_back(torch::empty_like(scales));
+  if (zeros.has_value()) out.push_back(torch::empty_like(*zeros));
+  check_abi(matgptq_pack_layer_device(
+                qweights.data_ptr<uint8_t>(), n, k, (int)bitwidth, (int)group_size, (int)source,
+                static_cast<const uint16_t*>(scales.data_ptr()),
+                zeros.has_value() ? static_cast<const uint16_t*>(zeros->data_ptr()) : nullptr,
+                static_cast<uint32_t*>(out[0].data_ptr()), static_cast<uint16_t*>(out[1].data_ptr()),
+                zeros.has_value() ? static_cast<uint16_t*>(out[2].data_ptr()) : nullptr, stream_of(dev)),
+            "pack_matgptq_layer");
+  return out;
+}
+
 // matmul_matgptq (bindings.cpp:146-191) and its zero-point extension.
 // `master`: `weights` are master-resident bit planes (N*K/4 words) instead of a pre-sliced tensor
 Tensor matmul_impl(const Tensor& input, const Tensor& weights, const Tensor& scales,
@@ -378,6 +413,7 @@ TORCH_LIBRARY(matgptq_cuda, m) {
   m.def("matmul_matgptq_zp(Tensor input, Tensor matgptq_weights, Tensor matgptq_scales, "
         "Tensor matgptq_zeros, int n_out_features, int n_in_features, int bitwidth, int group_size, "
         "int feature_flag) -> Tensor");
+  m.def("pack_matgptq_layer(Tensor qweights, Tensor scales, Tensor? zeros, int bitwidth, int group_size, int source) -> Tensor[]");
   m.def("unpack_matgptq_qweights(Tensor matgptq_weights, int n_out_features, int n_in_features, "
         "int bitwidth) -> Tensor");
   m.def("slice_matgptq_master(Tensor master, int bitwidth) -> Tensor");
@@ -407,6 +443,7 @@ TORCH_LIBRARY_IMPL(matgptq_cuda, CUDA, m) {
   m.impl("matmul_matgptq", TORCH_FN(matmul_matgptq));
   m.impl("matmul_matgptq_zp", TORCH_FN(matmul_matgptq_zp));
   m.impl("matmul_matgptq_master", TORCH_FN(matmul_matgptq_master));
+  m.impl("pack_matgptq_layer", TORCH_FN(pack_matgptq_layer));
   m.impl("slice_matgptq_master", TORCH_FN(slice_matgptq_master));
   m.impl("dequantize_matgptq", TORCH_FN(dequantize_matgptq));
 }

@@ -14,6 +14,8 @@ Additive operators of this implementation (all under torch.ops.matgptq_cuda):
                              codes and slices them to `bitwidth` while packing
     matmul_matgptq_zp        matmul_matgptq with a per-group zero tensor (reordered with
                              reorder_matgptq_scales) after matgptq_scales
+    pack_matgptq_layer       codes, scales and zeros of a layer that is on the GPU into the kernels' order
+                             in one launch
     unpack_matgptq_qweights  packed -> uint8 codes (tests, bit-exactness checks)
     slice_matgptq_master     rounded MSB slice of master codes on the GPU
     dequantize_matgptq       packed -> dense fp16 weight, rounded like the reference's dequantize
@@ -36,6 +38,7 @@ _ops = torch.ops.matgptq_cuda
 
 pack_matgptq_qweights = _ops.pack_matgptq_qweights
 pack_matgptq_master = _ops.pack_matgptq_master
+pack_matgptq_layer = _ops.pack_matgptq_layer
 reorder_matgptq_scales = _ops.reorder_matgptq_scales
 matmul_matgptq = _ops.matmul_matgptq
 matmul_matgptq_zp = _ops.matmul_matgptq_zp

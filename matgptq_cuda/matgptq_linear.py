@@ -46,12 +46,17 @@ class MatGPTQLinear(torch.nn.Module):
         def frozen(t: torch.Tensor) -> torch.nn.Parameter:
             return torch.nn.Parameter(t, requires_grad=False)
 
-        def per_group(t: torch.Tensor) -> torch.Tensor:  # scales and zeros share one device layout
-            return ops.reorder_matgptq_scales(t, *shape, self.group_size)
+        zeros = None if zeros is None else zeros.to(scales.dtype).contiguous()
+        if qweight.is_cuda and scales.device == qweight.device and (zeros is None or zeros.device == qweight.device):
+            packed = ops.pack_matgptq_layer(qweight, scales, zeros, bitwidth, group_size, 0)  # one launch
+        else:
+            def per_group(t: torch.Tensor) -> torch.Tensor:  # scales and zeros share one device layout
+                return ops.reorder_matgptq_scales(t, *shape, self.group_size)
 
-        self.matgptq_qweight = frozen(ops.pack_matgptq_qweights(qweight, *shape, self.bitwidth, self.group_size, self.flag))
-        self.matgptq_scales = frozen(per_group(scales))
-        self.matgptq_zeros = None if zeros is None else frozen(per_group(zeros.to(scales.dtype).contiguous()))
+            packed = [ops.pack_matgptq_qweights(qweight, *shape, self.bitwidth, self.group_size, self.flag),
+                      per_group(scales)] + ([] if zeros is None else [per_group(zeros)])
+        self.matgptq_qweight, self.matgptq_scales = frozen(packed[0]), frozen(packed[1])
+        self.matgptq_zeros = None if zeros is None else frozen(packed[2])
         if perm is None:
             self.matgptq_perm = None
         else:

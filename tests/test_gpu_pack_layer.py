@@ -1,0 +1,42 @@
+"""The one-launch packing of a layer (codes, scales, zeros) against the separate host packers, word for
+word, at the edges of its tiling: a workgroup takes eight tiles of K, half a wave one tile."""
+import numpy as np
+import pytest
+import torch
+
+import matgptq_cuda  # noqa: F401  (registers the operators)
+from matgptq_amd import _lib
+from oracle import matgptq_oracle as o
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("source", (0, 1, 2))
+@pytest.mark.parametrize("b", (2, 3, 4, 6, 8))
+@pytest.mark.parametrize("n,k,g", ((16, 128, 128), (48, 7 * 128, 32), (32, 8 * 128, -1), (80, 9 * 128, 128),
+                                   (32, 8 * 128 + 64, 32), (16, 192, -1), (48, 17 * 128 + 64, 32)))
+def test_layer_in_one_launch_equals_host_packers(n, k, g, b, source):
+    if source == 2 and k % 128 != 0:
+        pytest.skip("the planes have whole tiles only")
+    L = _lib.load()
+    rng = np.random.default_rng(n + k + b)
+    q = rng.integers(0, 256, (n, k), dtype=np.uint8)
+    codes = o.slice_codes(q, b) if source == 0 else q
+    groups = 1 if g == -1 else k // g
+    per_group = [rng.integers(0, 1 << 16, (n, groups), dtype=np.uint16) for _ in range(2)]
+    dev = [torch.from_numpy(t.view(np.float16)).cuda() for t in per_group]
+    packed, scales, zeros = torch.ops.matgptq_cuda.pack_matgptq_layer(
+        torch.from_numpy(codes).cuda(), dev[0], dev[1], b, g, source)
+    if source == 2:
+        host = np.zeros(L.matgptq_master_words(n, k), dtype=np.uint32)
+        _lib.check(L.matgptq_pack_master_host(q.ctypes.data, n, k, host.ctypes.data))
+    else:
+        host = np.zeros(L.matgptq_packed_words(b, n, k), dtype=np.uint32)
+        _lib.check(L.matgptq_pack_host(q.ctypes.data, n, k, b, 1, host.ctypes.data))
+    assert np.array_equal(packed.cpu().numpy(), host)
+    for got, src in ((scales, per_group[0]), (zeros, per_group[1])):
+        want = np.zeros_like(src)
+        _lib.check(L.matgptq_reorder_scales_host(src.ctypes.data, n, k, g, want.ctypes.data))
+        assert np.array_equal(got.cpu().numpy().view(np.uint16), want)
+    without = torch.ops.matgptq_cuda.pack_matgptq_layer(torch.from_numpy(codes).cuda(), dev[0], None, b, g, source)
+    assert len(without) == 2 and torch.equal(without[0].view(torch.int32), packed.view(torch.int32))

@@ -244,48 +244,59 @@ class MatGPTQLinearMethod(LinearMethodBase):
             self.n_out_features, self.n_in_features, bitwidth,
             self.config.group_size, self.config.flag)
 
-    def process_weights_after_loading(self, layer: torch.nn.Module) -> None:
-        with torch.no_grad():
-            qweight = layer.qweight.data
-            if self.config.resident_master_planes:
-                layer.matgptq_planes = Parameter(
-                    torch.ops.matgptq_cuda.pack_matgptq_master_resident(qweight.contiguous()), requires_grad=False)
-                layer.matgptq_weights = None
-            else:
-                layer.matgptq_planes = None
-                layer.matgptq_weights = Parameter(self._pack_at(layer, qweight, self.bitwidth), requires_grad=False)
-            layer.matgptq_bitwidth = self.bitwidth
-            layer.matgptq_scales = Parameter(
-                torch.ops.matgptq_cuda.reorder_matgptq_scales(
-                    layer.scales.data.contiguous(), self.n_out_features, self.n_in_features,
-                    self.config.group_size),
-                requires_grad=False)
-            zeros = getattr(layer, "zeros", None)
-            if zeros is not None:
-                layer.matgptq_zeros = Parameter(
-                    torch.ops.matgptq_cuda.reorder_matgptq_scales(
-                        zeros.data.to(layer.scales.dtype).contiguous(), self.n_out_features,
-                        self.n_in_features, self.config.group_size),
-                    requires_grad=False)
-                del layer.zeros
-            else:
-                layer.matgptq_zeros = None
-            perm = getattr(layer, "perm", None)
-            if perm is not None:
-                # act-order: the codes are stored in permuted column order and the input features
-                # are gathered with the permutation (src/quant_utils_matgpqt.py:218-220)
-                layer.matgptq_perm = Parameter(perm.data.to(device=layer.matgptq_scales.device,
-                                                            dtype=torch.int64).reshape(-1), requires_grad=False)
-                del layer.perm
-            else:
-                layer.matgptq_perm = None
+    def _pack_all(self, layer: torch.nn.Module) -> List[torch.Tensor]:
+        """Packed codes (or resident planes), scales and, if the layer has them, zeros in the kernels' order."""
+        ops, config = torch.ops.matgptq_cuda, self.config
+        params = layer._parameters
+        qweight, scales, zeros = params["qweight"].data, params["scales"].data.contiguous(), params.get("zeros")
+        zeros = None if zeros is None else zeros.data.to(scales.dtype).contiguous()
+        planes = config.resident_master_planes
+        if (qweight.is_cuda and config.master_bitwidth == 8 and scales.device == qweight.device
+                and tuple(qweight.shape) == (self.n_out_features, self.n_in_features)
+                and (zeros is None or zeros.device == qweight.device)):
+            # on the GPU already: one pass over the master codes, one launch for all of it
+            return ops.pack_matgptq_layer(qweight.contiguous(), scales, zeros, self.bitwidth, config.group_size,
+                                          2 if planes else 1)
+        packed = [ops.pack_matgptq_master_resident(qweight.contiguous()) if planes
+                  else self._pack_at(layer, qweight, self.bitwidth)]
+        for t in (scales, zeros):
+            if t is not None:
+                packed.append(ops.reorder_matgptq_scales(t, self.n_out_features, self.n_in_features, config.group_size))
+        return packed
 
-            if self.config.keep_master_codes and not self.config.resident_master_planes:
+    def process_weights_after_loading(self, layer: torch.nn.Module) -> None:
+        # A model has hundreds of layers: names are put into the module's own tables, which is what
+        # Module.__setattr__ comes to after about 2 us of look-ups per name.
+        params, plain = layer._parameters, layer.__dict__
+
+        def put(name: str, value: Optional[torch.Tensor]) -> None:
+            if value is None:
+                params.pop(name, None)
+                plain[name] = None
+            else:
+                plain.pop(name, None)
+                params[name] = Parameter(value, requires_grad=False)
+
+        with torch.no_grad():
+            qweight = params["qweight"].data
+            packed = self._pack_all(layer)
+            planes = self.config.resident_master_planes
+            put("matgptq_planes", packed[0] if planes else None)
+            put("matgptq_weights", None if planes else packed[0])
+            plain["matgptq_bitwidth"] = self.bitwidth
+            put("matgptq_scales", packed[1])
+            put("matgptq_zeros", packed[2] if len(packed) > 2 else None)
+            perm = params.pop("perm", None)
+            # act-order: the codes are stored in permuted column order and the input features
+            # are gathered with the permutation (src/quant_utils_matgpqt.py:218-220)
+            put("matgptq_perm", None if perm is None else
+                perm.data.to(device=packed[1].device, dtype=torch.int64).reshape(-1))
+            if self.config.keep_master_codes and not planes:
                 # The reference deletes the master codes here (inference_lib/vllm_matgptq.py:177-178);
                 # kept, a layer can be re-sliced to another bitwidth without the checkpoint.
-                layer.matgptq_master = Parameter(qweight.to(layer.matgptq_scales.device), requires_grad=False)
-            del layer.qweight
-            del layer.scales
+                put("matgptq_master", qweight.to(packed[1].device))
+            for name in ("qweight", "scales", "zeros"):
+                params.pop(name, None)
 
     def set_bitwidth(self, layer: torch.nn.Module, bitwidth: int) -> None:
         """Moves a loaded layer to `bitwidth`.  With `resident_master_planes` nothing is touched but
