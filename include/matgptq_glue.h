@@ -74,6 +74,19 @@ int matgptq_glue_attention_split(const void *qkv, const void *cos_table, const v
                                  void *workspace, int64_t M, int heads, int kv_heads,
                                  int head_dim, int64_t max_ctx, int fuse_rotary, void *stream);
 
+/* Operators of a prompt (many rows), each bit for bit the sequence of fp16 element-wise operators it stands for;
+ * heads of 128 elements, F % 8 == 0, pointers on 16 bytes, M <= 65535 for the first two.
+ * rope_prompt: t cos + rotate_half(t) sin of the query heads of qkv[M, (heads + 2 kv_heads) * 128] into
+ * q_out[heads, M, 128] and of the key heads into row pos[m] of k_cache[kv_heads, max_ctx, 128]; the value heads go to
+ * the same row of v_cache.  cos_rows / sin_rows [M, 128]: the table rows of the positions.  qkv is read only.
+ * heads_to_rows: out[m, head, :] = x[head, m, :].
+ * silu_mul_prompt: matgptq_glue_silu_mul with the exponential and quotient of the separate operators. */
+int matgptq_glue_rope_prompt(const void *qkv, const void *cos_rows, const void *sin_rows,
+                             const int64_t *pos, void *q_out, void *k_cache, void *v_cache, int64_t M,
+                             int heads, int kv_heads, int head_dim, int64_t max_ctx, void *stream);
+int matgptq_glue_heads_to_rows(const void *x, void *out, int64_t M, int heads, int head_dim, void *stream);
+int matgptq_glue_silu_mul_prompt(const void *gate_up, void *out, int64_t M, int64_t F, void *stream);
+
 /* out[m] (int64) = index of the largest of x[m, 0:n] (fp32, rows contiguous): the first among equals, a NaN
  * counts as the largest (torch.argmax).  One launch, no workspace.  M <= 65535, n < 2^31. */
 int matgptq_glue_argmax(const void *x, void *out, int64_t M, int64_t n, void *stream);

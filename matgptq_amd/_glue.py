@@ -18,7 +18,8 @@ MAX_CONTEXT = 8192
 
 EXPORTS = ("matgptq_glue_strerror", "matgptq_glue_add_rmsnorm", "matgptq_glue_rope_cache",
            "matgptq_glue_attention", "matgptq_glue_rope_attention", "matgptq_glue_attention_workspace_floats",
-           "matgptq_glue_attention_split", "matgptq_glue_silu_mul", "matgptq_glue_argmax")
+           "matgptq_glue_attention_split", "matgptq_glue_rope_prompt", "matgptq_glue_heads_to_rows",
+           "matgptq_glue_silu_mul_prompt", "matgptq_glue_silu_mul", "matgptq_glue_argmax")
 
 _lib = None
 
@@ -41,6 +42,9 @@ def load() -> ctypes.CDLL:
     L.matgptq_glue_add_rmsnorm.argtypes = [vp, vp, vp, vp, i64, i64, f32, vp]
     L.matgptq_glue_rope_cache.argtypes = [vp, vp, vp, vp, vp, vp, i64, ci, ci, ci, i64, vp]
     L.matgptq_glue_attention.argtypes = [vp, vp, vp, vp, vp, i64, ci, ci, ci, i64, vp]
+    L.matgptq_glue_rope_prompt.argtypes = [vp, vp, vp, vp, vp, vp, vp, i64, ci, ci, ci, i64, vp]
+    L.matgptq_glue_heads_to_rows.argtypes = [vp, vp, i64, ci, ci, vp]
+    L.matgptq_glue_silu_mul_prompt.argtypes = [vp, vp, i64, i64, vp]
     L.matgptq_glue_rope_attention.argtypes = [vp, vp, vp, vp, vp, vp, vp, ci, ci, ci, i64, vp]
     L.matgptq_glue_silu_mul.argtypes = [vp, vp, i64, i64, vp]
     L.matgptq_glue_argmax.argtypes = [vp, vp, i64, i64, vp]
@@ -152,13 +156,38 @@ def attention_split(qkv, cos, sin, pos, k_cache, v_cache, out, workspace, heads:
         m, heads, kv_heads, d, max_ctx, int(fuse_rotary), _stream()))
 
 
-def silu_mul(gate_up, out) -> None:
-    """out[M, F] = silu(gate_up[:, :F]) * gate_up[:, F:]."""
+def rope_prompt(qkv, cos_rows, sin_rows, pos, q_out, k_cache, v_cache, heads: int, kv_heads: int) -> None:
+    """Rotated queries of qkv [M, (heads + 2 kv_heads) * 128] into q_out [heads, M, 128], rotated keys and the values
+    into row pos[m] of the caches; cos_rows / sin_rows [M, 128] are the table rows of pos."""
+    _f16(qkv, cos_rows, sin_rows, q_out, k_cache, v_cache)
+    m = qkv.shape[0]
+    _pos_ok(pos, m)
+    kv, max_ctx, d = k_cache.shape
+    if (kv != kv_heads or v_cache.shape != k_cache.shape or qkv.shape[1] != (heads + 2 * kv_heads) * d
+            or cos_rows.shape != (m, d) or sin_rows.shape != (m, d) or q_out.shape != (heads, m, d)):
+        raise GlueError("rope_prompt: shapes differ")
+    _check(load().matgptq_glue_rope_prompt(qkv.data_ptr(), cos_rows.data_ptr(), sin_rows.data_ptr(), pos.data_ptr(),
+                                           q_out.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), m, heads,
+                                           kv_heads, d, max_ctx, _stream()))
+
+
+def heads_to_rows(x, out) -> None:
+    """out [M, heads * 128] = x [heads, M, 128] with rows first."""
+    _f16(x, out)
+    heads, m, d = x.shape
+    if out.shape != (m, heads * d):
+        raise GlueError("heads_to_rows: shapes differ")
+    _check(load().matgptq_glue_heads_to_rows(x.data_ptr(), out.data_ptr(), m, heads, d, _stream()))
+
+
+def silu_mul(gate_up, out, prompt: bool = False) -> None:
+    """out[M, F] = silu(gate_up[:, :F]) * gate_up[:, F:]; with `prompt` bit for bit as torch's two operators."""
     _f16(gate_up, out)
     m, f = out.shape
     if gate_up.shape != (m, 2 * f):
         raise GlueError("silu_mul: shapes differ")
-    _check(load().matgptq_glue_silu_mul(gate_up.data_ptr(), out.data_ptr(), m, f, _stream()))
+    fn = load().matgptq_glue_silu_mul_prompt if prompt else load().matgptq_glue_silu_mul
+    _check(fn(gate_up.data_ptr(), out.data_ptr(), m, f, _stream()))
 
 
 def argmax(x, out) -> None:
