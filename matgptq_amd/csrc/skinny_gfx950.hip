@@ -28,6 +28,10 @@
 //    tiles) and what hides the memory latency is the number of waves, not the depth of a
 //    ring (a four-deep ring at 128 KB per workgroup measured 10-30 % slower).  There is no
 //    barrier in the loop;
+//  * with two buffers (BUFS = 2) tile t + 2 is requested while t is multiplied and t + 1 is on its way, and the
+//    codes have two register sets that are refilled behind the multiplication.  That pays where a wave alone on its
+//    SIMD waits for its copies, and where several rounds of workgroups keep the copies queued; the rule is at
+//    two_buffers below;
 //  * every load is branch-free (tiles beyond K, rows beyond M or N go through a zero-length
 //    buffer descriptor or an out-of-range offset);
 //  * the eight partial sums meet in LDS once, at the end; the threads add them and store four
@@ -58,7 +62,7 @@ constexpr int skinny_lds_bytes(int r, int mb) {
 
 // MASTER: `a.packed` holds the master-resident bit planes (master_layout.h); the slice to BITS,
 // rounding and saturation happen in registers on the way to the raw fp16 pairs.
-template <int BITS, int GROUP, bool ZP, int R, int MB, bool MASTER>
+template <int BITS, int GROUP, bool ZP, int R, int MB, bool MASTER, int BUFS>
 __global__ void __launch_bounds__(64 * kWaves, 2)
 skinny_kernel(const GemmArgs a, int n_tiles, int m_tiles) {
   using Fmt = TileFormat<BITS, MASTER>;
@@ -66,6 +70,8 @@ skinny_kernel(const GemmArgs a, int n_tiles, int m_tiles) {
   constexpr int kStage = MB * 16 * 256;  // bytes of one activation buffer
   constexpr int NS = 2;  // register sets of codes, scales, zeros
   __shared__ __align__(16) unsigned char smem[skinny_lds_bytes(R, MB)];
+  // (an array of its own: the compiler orders LDS copies and reads per variable)
+  __shared__ __align__(16) unsigned char smem_odd[BUFS == 2 ? kWaves * kStage : 16];
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -124,6 +130,7 @@ skinny_kernel(const GemmArgs a, int n_tiles, int m_tiles) {
   // Copy of one tile's activations: instruction i moves rows 4i .. 4i+3 (lane l: row 4i + l/16,
   // LDS position l%16, which holds chunk (l%16) ^ (row & 15) of the row's 256 bytes).
   unsigned char* const stage = smem + wave * kStage;
+  unsigned char* const stage_odd = smem_odd + (BUFS == 2 ? wave * kStage : 0);
   uint32_t dma_voff[4 * MB];
 #pragma unroll
   for (int i = 0; i < 4 * MB; i++) {
@@ -132,18 +139,18 @@ skinny_kernel(const GemmArgs a, int n_tiles, int m_tiles) {
     const uint32_t m = (uint32_t)(m0 + row);
     dma_voff[i] = m < (uint32_t)a.M ? m * (uint32_t)a.K * 2u + c * 16 : x_bytes;
   }
-  auto dma = [&](int kb) {
+  auto dma = [&](unsigned char* to, int kb) {
     const BufRsrc xres = make_rsrc(a.x, kb < a.k_tiles ? x_bytes : 0u);
 #pragma unroll
     for (int i = 0; i < 4 * MB; i++)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(
-          xres, (__attribute__((address_space(3))) void*)(stage + i * 1024), 16, (int)dma_voff[i],
+          xres, (__attribute__((address_space(3))) void*)(to + i * 1024), 16, (int)dma_voff[i],
           (int)((uint32_t)kb * 256u), 0, 0);  // (int: the builtin's own parameter type)
     __builtin_amdgcn_sched_barrier(0);
   };
   // operand of batch rows i*16 + r16, columns [j*32 + q*8, +8) of the tile: chunk 4j + q
-  auto read_frag = [&](int i, int j) {
-    return *reinterpret_cast<const half8*>(stage + (i * 16 + r16) * 256 + (((4 * j + q) ^ r16) * 16));
+  auto read_frag = [&](const unsigned char* from, int i, int j) {
+    return *reinterpret_cast<const half8*>(from + (i * 16 + r16) * 256 + (((4 * j + q) ^ r16) * 16));
   };
 
   auto dequant_step = [&](Frag (&aw)[R], const uint32_t (&w)[R][Fmt::kWords], const uint32_t (&s)[R][GPT],
@@ -173,6 +180,30 @@ skinny_kernel(const GemmArgs a, int n_tiles, int m_tiles) {
     }
   };
 
+  auto multiply = [&](const half8 (&xf)[4][MB], const uint32_t (&w)[R][Fmt::kWords], const uint32_t (&s)[R][GPT],
+                      const uint32_t (&z)[R][GPT]) {
+    auto one = [&](auto jtag) {
+      constexpr int J = decltype(jtag)::value;
+      Frag aw[R];
+      dequant_step(aw, w, s, z, jtag);
+#pragma unroll
+      for (int i = 0; i < MB; i++) {
+#pragma unroll
+        for (int rr = 0; rr < R; rr++) {
+          if constexpr (kBf16)
+            acc[rr][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, aw[rr].h),
+                                                                __builtin_bit_cast(bf16x8, xf[J][i]), acc[rr][i], 0, 0, 0);
+          else
+            acc[rr][i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(aw[rr].h, xf[J][i], acc[rr][i], 0, 0, 0);
+        }
+      }
+    };
+    one(std::integral_constant<int, 0>{});
+    one(std::integral_constant<int, 1>{});
+    one(std::integral_constant<int, 2>{});
+    one(std::integral_constant<int, 3>{});
+  };
+
   // Tile t of the walk (K tile kb = wave + 8 t), codes in register set `btag`.
   auto tile = [&](int t, auto btag) {
     constexpr int B = decltype(btag)::value;
@@ -186,45 +217,68 @@ skinny_kernel(const GemmArgs a, int n_tiles, int m_tiles) {
 #pragma unroll
     for (int j = 0; j < 4; j++)
 #pragma unroll
-      for (int i = 0; i < MB; i++) xf[j][i] = read_frag(i, j);
+      for (int i = 0; i < MB; i++) xf[j][i] = read_frag(stage, i, j);
     // the buffer is free once these reads have returned: request the next tile
     __builtin_amdgcn_sched_barrier(0);
     __builtin_amdgcn_s_waitcnt(15 | (7 << 4) | (0 << 8) | (3 << 14));  // lgkmcnt(0)
     __builtin_amdgcn_sched_barrier(0);
-    dma(kb + kWaves);
+    dma(stage, kb + kWaves);
     load_weights(wr[B ^ 1], sr[B ^ 1], zr[B ^ 1], kb + kWaves);
-    if (kb < a.k_tiles) {
-      auto one = [&](auto jtag) {
-        constexpr int J = decltype(jtag)::value;
-        Frag aw[R];
-        dequant_step(aw, wr[B], sr[B], zr[B], jtag);
-#pragma unroll
-        for (int i = 0; i < MB; i++) {
-#pragma unroll
-          for (int rr = 0; rr < R; rr++) {
-            if constexpr (kBf16)
-              acc[rr][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, aw[rr].h),
-                                                                  __builtin_bit_cast(bf16x8, xf[J][i]), acc[rr][i], 0, 0, 0);
-            else
-              acc[rr][i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(aw[rr].h, xf[J][i], acc[rr][i], 0, 0, 0);
-          }
-        }
-      };
-      one(std::integral_constant<int, 0>{});
-      one(std::integral_constant<int, 1>{});
-      one(std::integral_constant<int, 2>{});
-      one(std::integral_constant<int, 3>{});
-    }
+    if (kb < a.k_tiles) multiply(xf, wr[B], sr[B], zr[B]);
     __builtin_amdgcn_sched_barrier(0);
   };
 
+  // The same with two buffers: tile t in buffer and register set `btag`.  `moretag`: tile t + 2 is requested;
+  // without it (the last two tiles) set 0 leaves set 1's requests in flight, set 1 none.
+  constexpr int kTileLoads = 4 * MB + R * ((MASTER ? master_load_count(BITS) : tile_load_count(BITS)) + GPT * (ZP ? 2 : 1));
+  static_assert(BUFS == 1 || kTileLoads < 64, "vmcnt counts up to 63");
+  auto tile_of_two = [&](int t, auto btag, auto moretag) {
+    constexpr int B = decltype(btag)::value;
+    constexpr bool kMore = decltype(moretag)::value;
+    constexpr int kYounger = kMore || B == 0 ? kTileLoads : 0;  // requests of the tile behind this one
+    const int kb = wave + t * kWaves;
+    unsigned char* const buf = B == 0 ? stage : stage_odd;
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_waitcnt((kYounger & 15) | (7 << 4) | (15 << 8) | ((kYounger >> 4) << 14));
+    __builtin_amdgcn_sched_barrier(0);
+    half8 xf[4][MB];
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+#pragma unroll
+      for (int i = 0; i < MB; i++) xf[j][i] = read_frag(buf, i, j);
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (kMore) {
+      __builtin_amdgcn_s_waitcnt(15 | (7 << 4) | (0 << 8) | (3 << 14));  // lgkmcnt(0): the buffer is free
+      __builtin_amdgcn_sched_barrier(0);
+      dma(buf, kb + 2 * kWaves);
+    }
+    // (only the last tile of a walk can lie beyond K; its buffer may hold anything)
+    if (kMore || kb < a.k_tiles) multiply(xf, wr[B], sr[B], zr[B]);
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (kMore) load_weights(wr[B], sr[B], zr[B], kb + 2 * kWaves);
+  };
+
   const int walk = (a.k_tiles + kWaves - 1) / kWaves;  // tiles of the longest walk
+  using Even = std::integral_constant<int, 0>;
+  using Odd = std::integral_constant<int, 1>;
   __builtin_amdgcn_sched_barrier(0);
-  dma(wave);
+  dma(stage, wave);
   load_weights(wr[0], sr[0], zr[0], wave);
-  for (int t = 0; t < walk; t += 2) {
-    tile(t, std::integral_constant<int, 0>{});
-    tile(t + 1, std::integral_constant<int, 1>{});
+  if constexpr (BUFS == 2) {
+    dma(stage_odd, wave + kWaves);
+    load_weights(wr[1], sr[1], zr[1], wave + kWaves);
+    int t = 0;
+    for (; t + 2 < walk; t += 2) {
+      tile_of_two(t, Even{}, std::true_type{});
+      tile_of_two(t + 1, Odd{}, std::true_type{});
+    }
+    tile_of_two(t, Even{}, std::false_type{});
+    if (t + 1 < walk) tile_of_two(t + 1, Odd{}, std::false_type{});
+  } else {
+    for (int t = 0; t < walk; t += 2) {
+      tile(t, Even{});
+      tile(t + 1, Odd{});
+    }
   }
 
   // The eight partial sums of every output meet in LDS (over the activation buffers: every
@@ -256,12 +310,36 @@ skinny_kernel(const GemmArgs a, int n_tiles, int m_tiles) {
   }
 }
 
+// Two buffers, on pre-sliced codes and up to 32 batch rows per workgroup (the second buffer is another 32 KB per 16
+// batch rows).  us, one -> two buffers, 4 bits where nothing else is said:
+//  * a walk of one tile, whose second tile the loop of pairs would wait for: 8192 x 1024 at M = 16 / 32 / 64
+//    4.29 -> 3.98 / 5.28 -> 4.77 / 6.30 -> 5.69, 8192 x 512 at M = 10 3.74 -> 3.36, 8192 x 1024 at 6 bits and M = 51 7.91 -> 6.48;
+//  * one row block per workgroup: 2048 x 4096 at M = 12 / 32 / 64 5.16 -> 4.82 / 6.93 -> 6.61 / 6.79 -> 6.57, 4096 x 4096 at M = 12
+//    5.53 -> 5.28 (several blocks of 32 batch rows and a longer walk: 1280 x 8192 at M = 49, 6 bits, 9.98 against 10.69);
+//  * 16 batch rows and more workgroups than CUs, fp16 storage: 28672 x 4096 at M = 8 / 12 / 16 16.3 -> 15.5 / 17.6 -> 16.0 / 17.6 -> 16.6,
+//    12288 x 2560 at M = 6 and 8 bits 11.1 -> 10.0, 57344 x 8192 at M = 10 49.0 -> 47.9 (the weights of bf16 storage, and 8 bits with
+//    their four scales per tile at group size 32, take more registers: 28672 x 4096 at M = 13 17.3 against 19.3,
+//    16384 x 2048 at M = 12 11.2 against 12.3).
+// Elsewhere one buffer is as fast or ahead by up to 5 % (8192 x 3584 at M = 16: 6.74 against 7.02, 7168 x 8192 at M = 22 and 2
+// bits 11.2 against 11.8).
+template <int GROUP, int R, int MB, bool MASTER>
+bool two_buffers(const GemmArgs& a, int workgroups) {
+  if (MASTER || R > 4 || MB > 2) return false;
+  if (a.k_tiles <= kWaves) return true;
+  if (R == 1) return a.M <= 32 || a.k_tiles <= 4 * kWaves;
+  return MB == 1 && !kBf16 && !(GROUP == 32 && kBits == 8) && workgroups > 256;
+}
+
 template <int GROUP, bool ZP, int R, int MB, bool MASTER>
 hipError_t launch_r(const GemmArgs& a, hipStream_t stream) {
   const int n_tiles = (a.row_blocks + R - 1) / R;
   const int m_tiles = (a.M + 16 * MB - 1) / (16 * MB);
   const dim3 grid(n_tiles * m_tiles), block(64 * kWaves);
-  hipLaunchKernelGGL((skinny_kernel<kBits, GROUP, ZP, R, MB, MASTER>), grid, block, 0, stream, a, n_tiles, m_tiles);
+  constexpr int kTwo = !MASTER && R <= 4 && MB <= 2 ? 2 : 1;
+  if (kTwo == 2 && two_buffers<GROUP, R, MB, MASTER>(a, n_tiles * m_tiles))
+    hipLaunchKernelGGL((skinny_kernel<kBits, GROUP, ZP, R, MB, MASTER, kTwo>), grid, block, 0, stream, a, n_tiles, m_tiles);
+  else
+    hipLaunchKernelGGL((skinny_kernel<kBits, GROUP, ZP, R, MB, MASTER, 1>), grid, block, 0, stream, a, n_tiles, m_tiles);
   return hipGetLastError();
 }
 

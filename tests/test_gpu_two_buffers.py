@@ -1,0 +1,33 @@
+"""The mid-batch kernel's walk with two activation buffers (skinny_gfx950.hip) at the edges of its range: walks of one,
+two, three and an odd number of tiles, waves without a tile, more workgroups than CUs, ragged batches."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import matgptq_oracle as o
+from tests import _gpu_util as G
+
+pytestmark = pytest.mark.gpu
+
+# (N, K, M, flags variant: 80 + rsel + 3 msel, 0 = the planner's own)
+CASES = [(32, 128, 9, 80), (64, 384, 16, 80), (48, 1024, 17, 83), (48, 1152, 33, 83), (64, 2048, 12, 80), (32, 3200, 16, 80),
+         (96, 1024, 16, 81), (160, 896, 40, 85), (112, 3072, 23, 84), (8256, 2176, 16, 81), (16640, 1280, 7, 82)]
+
+
+@pytest.mark.parametrize("bits,group,bf16", [(4, 128, False), (3, 128, True), (8, 128, False), (2, -1, False), (6, 32, True)])
+@pytest.mark.parametrize("n,k,m,variant", CASES)
+def test_two_buffers(n, k, m, variant, bits, group, bf16):
+    q, s, z = o.make_layer(n, k, group, seed=n + k + bits)
+    dt = torch.bfloat16 if bf16 else torch.float16
+    st, zt = torch.from_numpy(s).to(dt), torch.from_numpy(z).to(dt)
+    x = torch.from_numpy(o.make_activations(m, k, seed=m)).to(dt)
+    bits_of = lambda t: t.view(torch.float16).numpy()  # (the reordering moves 16-bit values, whatever they are)
+    y = G.gemm(bits, group, n, k, x.cuda(), G.pack_device(q, bits, True), G.reorder_device(bits_of(st), n, k, group),
+               G.reorder_device(bits_of(zt), n, k, group), flags=1 | (2 if bf16 else 0) | (variant << 8)).view(dt)
+    if bf16:  # the weights are the oracle's; one rounding of the result (half a step of 2^-7), sums in fp32 (a hundredth of it)
+        w = o.dequantize_bf16(q, st.float().numpy(), zt.float().numpy(), bits, group)
+        ref = x.double().numpy() @ w.astype(np.float64).T
+        assert np.max(np.abs(y.double().cpu().numpy() - ref)) <= 1.01 * 2.0 ** -8 * np.max(np.abs(ref))
+    else:
+        G.assert_close_to_oracle(y.cpu().numpy(), x.numpy(), o.dequantize(q, s, z, bits, group),
+                                 f"{n}x{k} m{m} b{bits} g{group} v{variant}")
