@@ -59,9 +59,8 @@ int matgptq_glue_rope_attention(const void *qkv, const void *cos_table, const vo
                                 int heads, int kv_heads, int head_dim, int64_t max_ctx,
                                 void *stream);
 
-/* The same attention with the context split over workgroups (one per key/value head and 64
- * cache rows, serving all query heads of that key/value head) and a second small launch that
- * combines their partial results: for short batches, where a workgroup per query head leaves
+/* The same attention with the context split over workgroups (one per one or two query heads and
+ * 64 cache rows) and a second small launch that combines their partial results: for short batches, where a workgroup per query head leaves
  * most of the GPU idle.  Query heads per key/value head: 1, 2, 4 or 8.  fuse_rotary != 0 (M = 1
  * only) also does what matgptq_glue_rope_cache does, like matgptq_glue_rope_attention;
  * otherwise qkv holds rotated queries and the caches are read only (cos_table / sin_table may

@@ -313,31 +313,37 @@ attention_kernel(const _Float16* __restrict__ qkv, _Float16* k_cache, _Float16* 
   }
 }
 
-// The same attention with the context split over workgroups: grid (kv_heads, splits, M), one
-// workgroup per key/value head and 64 cache rows, which serves all REP query heads of that
-// key/value head from one read of the rows (a workgroup per query head reads them REP times, and
-// a single CU can pull only so much).  Every workgroup with rows to look at leaves its partial
-// result - the maximum score, the sum of the exponentials and the weighted values, per query
-// head - in `ws`; attention_combine_kernel, launched behind it, puts the partial results of the
+// The same attention with the context split over workgroups: grid (heads / HEADS, splits, M), one
+// workgroup per HEADS query heads of one key/value head and 64 cache rows (with eight key/value heads the
+// workgroups that share rows share an XCD's L2).  Every workgroup with rows to look at leaves its partial
+// result - the maximum score, the sum of the exponentials and the weighted values, per query head -
+// in `ws`; attention_combine_kernel, launched behind it, puts the partial results of the
 // splits up to pos[m] together.  (One kernel whose last workgroup combines was measured slower:
 // the fences that publish the partial results across the L2 caches of the XCDs cost more than
 // the second launch.)
+// A workgroup's time is its arithmetic, one head after the other: up to four rows take one head per workgroup up to
+// 1024 cache rows, everything else two, where reading the rows again starts to count.  One row, us with 1 / 2 / all query heads
+// of a key/value head per workgroup: 32 / 8 heads, 513 rows of 584 6.5 / 6.7 / 8.0, 1001 of 1024 7.5 / 7.5 / 8.8, 4097 of 4168 16.4 /
+// 16.0 / 17.0; 64 / 8 heads, 513 of 584 7.3 / 7.6 / 10.6, 4097 of 4168 22.1 / 20.6 / 30.7; four rows, 32 / 8 heads, 513 of 584
+// 7.3 / 8.1 / 8.9; 16 rows, 64 / 8 heads, 900 of 1000 30.8 / 29.5 / 33.6.  (One workgroup per head, unsplit: 513 of 584 rows 8.3.)
 // ws: M x heads x splits x 130 floats.
+constexpr int kOneHeadContext = 1024;
 constexpr int kSplitRows = 64;
 constexpr int kSplitStride = 130;  // 128 values, maximum, sum
 
-template <bool ROPE, int REP>
+template <bool ROPE, int HEADS>
 __global__ void __launch_bounds__(256)
 attention_split_kernel(const _Float16* __restrict__ qkv, _Float16* k_cache, _Float16* v_cache,
                        const int64_t* __restrict__ pos, _Float16* __restrict__ out,
                        const _Float16* __restrict__ cos_t, const _Float16* __restrict__ sin_t,
                        float* __restrict__ ws, int heads, int kv_heads, int64_t max_ctx, int splits, float scale) {
   constexpr int d = 128;
-  __shared__ float sc[REP][kSplitRows];  // scores, then exponentials
-  __shared__ float part[4][REP][d];      // weighted values per wave
-  __shared__ float mx_s[REP], sum_s[REP];
-  const int kvh = blockIdx.x, split = blockIdx.y, m = blockIdx.z;
+  __shared__ float sc[HEADS][kSplitRows];  // scores, then exponentials
+  __shared__ float part[4][HEADS][d];      // weighted values per wave
+  __shared__ float mx_s[HEADS], sum_s[HEADS];
+  const int kvh = (int)(blockIdx.x % (unsigned)kv_heads), split = blockIdx.y, m = blockIdx.z;
   const int tid = threadIdx.x, sub = tid & 15, grp = tid >> 4, wave = tid >> 6, lane = tid & 63;
+  const int head0 = kvh * (heads / kv_heads) + (int)(blockIdx.x / (unsigned)kv_heads) * HEADS;  // this workgroup's heads
   const int row0 = split * kSplitRows;
   const int last = (int)max_ctx - 1;
   auto row_of = [&](int t) { return (size_t)(t < last ? t : last) * d; };
@@ -350,9 +356,9 @@ attention_split_kernel(const _Float16* __restrict__ qkv, _Float16* k_cache, _Flo
 #pragma unroll
   for (int u = 0; u < 4; u++) vr[u] = *reinterpret_cast<const half8*>(vb + row_of(row0 + grp + 16 * u));
   const _Float16* row = qkv + (size_t)m * (heads + 2 * kv_heads) * d + sub * 8;
-  half8 qv[REP];
+  half8 qv[HEADS];
 #pragma unroll
-  for (int r = 0; r < REP; r++) qv[r] = *reinterpret_cast<const half8*>(row + (size_t)(kvh * REP + r) * d);
+  for (int r = 0; r < HEADS; r++) qv[r] = *reinterpret_cast<const half8*>(row + (size_t)(head0 + r) * d);
   half8 k_cur = qv[0], v_cur = qv[0];
   if constexpr (ROPE) {
     k_cur = *reinterpret_cast<const half8*>(row + (size_t)(heads + kvh) * d);
@@ -371,14 +377,15 @@ attention_split_kernel(const _Float16* __restrict__ qkv, _Float16* k_cache, _Flo
       const float kp = row_ror<8>(ko);
       k_cur[e] = rotary(ko, sub < 8 ? -kp : kp, cv[e], sv[e]);
 #pragma unroll
-      for (int r = 0; r < REP; r++) {
+      for (int r = 0; r < HEADS; r++) {
         const float qo = (float)qv[r][e];
         const float qp = row_ror<8>(qo);
         qv[r][e] = rotary(qo, sub < 8 ? -qp : qp, cv[e], sv[e]);
       }
     }
-    // the workgroup whose rows include the new one writes it to the caches
-    if ((int)p >= row0 && (int)p < row0 + kSplitRows && grp == 0) {
+    // the (first) workgroup whose rows include the new one writes it to the caches; the others do not use what
+    // they read of that row
+    if (blockIdx.x < (unsigned)kv_heads && (int)p >= row0 && (int)p < row0 + kSplitRows && grp == 0) {
       *reinterpret_cast<half8*>(k_cache + ((size_t)kvh * max_ctx + p) * d + sub * 8) = k_cur;
       *reinterpret_cast<half8*>(v_cache + ((size_t)kvh * max_ctx + p) * d + sub * 8) = v_cur;
     }
@@ -388,7 +395,7 @@ attention_split_kernel(const _Float16* __restrict__ qkv, _Float16* k_cache, _Flo
     const int t = row0 + grp + 16 * u;
     const half8 kk = ROPE && t == (int)p ? k_cur : kr[u];
 #pragma unroll
-    for (int r = 0; r < REP; r++) {
+    for (int r = 0; r < HEADS; r++) {
       float dot = 0.f;
 #pragma unroll
       for (int e = 0; e < 8; e++) dot += (float)qv[r][e] * scale * (float)kk[e];
@@ -398,7 +405,7 @@ attention_split_kernel(const _Float16* __restrict__ qkv, _Float16* k_cache, _Flo
   }
   __syncthreads();
   // maximum and sum of exponentials per query head: wave w takes heads w, w + 4; lane = row
-  for (int r = wave; r < REP; r += 4) {
+  for (int r = wave; r < HEADS; r += 4) {
     const float v = sc[r][lane];
     const float mx = wave_max(v);
     const float e = mx == -INFINITY ? 0.f : __expf(v - mx);
@@ -407,9 +414,9 @@ attention_split_kernel(const _Float16* __restrict__ qkv, _Float16* k_cache, _Flo
     if (lane == 0) { mx_s[r] = mx; sum_s[r] = sum; }
   }
   __syncthreads();
-  float acc[REP][8];
+  float acc[HEADS][8];
 #pragma unroll
-  for (int r = 0; r < REP; r++)
+  for (int r = 0; r < HEADS; r++)
 #pragma unroll
     for (int e = 0; e < 8; e++) acc[r][e] = 0.f;
 #pragma unroll
@@ -418,7 +425,7 @@ attention_split_kernel(const _Float16* __restrict__ qkv, _Float16* k_cache, _Flo
     if (t < n) {  // (an unused row may hold anything, also NaN)
       const half8 vv = ROPE && t == (int)p ? v_cur : vr[u];
 #pragma unroll
-      for (int r = 0; r < REP; r++) {
+      for (int r = 0; r < HEADS; r++) {
         const float pr = sc[r][grp + 16 * u];
 #pragma unroll
         for (int e = 0; e < 8; e++) acc[r][e] += pr * (float)vv[e];
@@ -427,20 +434,19 @@ attention_split_kernel(const _Float16* __restrict__ qkv, _Float16* k_cache, _Flo
   }
   // the four row groups of a wave by shuffles, the four waves through LDS
 #pragma unroll
-  for (int r = 0; r < REP; r++)
+  for (int r = 0; r < HEADS; r++)
 #pragma unroll
     for (int e = 0; e < 8; e++) {
       acc[r][e] = sum_of_rows(acc[r][e]);
     }
   if (lane < 16) {
 #pragma unroll
-    for (int r = 0; r < REP; r++)
+    for (int r = 0; r < HEADS; r++)
 #pragma unroll
       for (int e = 0; e < 8; e++) part[wave][r][sub * 8 + e] = acc[r][e];
   }
   __syncthreads();
-  const int head0 = kvh * REP;
-  for (int idx = tid; idx < REP * d; idx += 256) {
+  for (int idx = tid; idx < HEADS * d; idx += 256) {
     const int r = idx >> 7, dim = idx & 127;
     float* dst = ws + ((size_t)(m * heads + head0 + r) * splits + split) * kSplitStride;
     dst[dim] = part[0][r][dim] + part[1][r][dim] + part[2][r][dim] + part[3][r][dim];
@@ -495,20 +501,20 @@ int launch_attention_split(const void* qkv, void* k_cache, void* v_cache, const 
                            const void* cos_table, const void* sin_table, void* ws, int64_t M, int heads,
                            int kv_heads, int64_t max_ctx, void* stream) {
   const int splits = (int)((max_ctx + kSplitRows - 1) / kSplitRows);
-  const dim3 grid((unsigned)kv_heads, (unsigned)splits, (unsigned)M), block(256);
+  const dim3 block(256);
   const float scale = 1.0f / sqrtf(128.0f);
-#define MATGPTQ_GLUE_SPLIT(REP)                                                                              \
-  hipLaunchKernelGGL((attention_split_kernel<ROPE, REP>), grid, block, 0, (hipStream_t)stream,                \
+#define MATGPTQ_GLUE_SPLIT(HEADS)                                                                            \
+  hipLaunchKernelGGL((attention_split_kernel<ROPE, HEADS>),                                                   \
+                     dim3((unsigned)(heads / HEADS), (unsigned)splits, (unsigned)M), block, 0, (hipStream_t)stream, \
                      (const _Float16*)qkv, (_Float16*)k_cache, (_Float16*)v_cache, pos, (_Float16*)out,       \
                      (const _Float16*)cos_table, (const _Float16*)sin_table, (float*)ws, heads, kv_heads,   \
                      max_ctx, splits, scale)
   switch (heads / kv_heads) {
-    case 1: MATGPTQ_GLUE_SPLIT(1); break;
-    case 2: MATGPTQ_GLUE_SPLIT(2); break;
-    case 4: MATGPTQ_GLUE_SPLIT(4); break;
-    case 8: MATGPTQ_GLUE_SPLIT(8); break;
+    case 1: case 2: case 4: case 8: break;
     default: return MATGPTQ_GLUE_ESHAPE;
   }
+  if (heads == kv_heads || (M <= 4 && max_ctx <= kOneHeadContext)) MATGPTQ_GLUE_SPLIT(1);
+  else MATGPTQ_GLUE_SPLIT(2);
 #undef MATGPTQ_GLUE_SPLIT
   if (int e = launch_status()) return e;
   hipLaunchKernelGGL(attention_combine_kernel, dim3((unsigned)heads, (unsigned)M), dim3(128), 0,

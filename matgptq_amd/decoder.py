@@ -156,14 +156,14 @@ class Block(torch.nn.Module):
         is updated in place with `delta` (the previous block's last linear output, or None) and this
         block's attention output; returns the output of `down`, which the next block (or the final
         norm) adds.  `x` [M, hidden] is scratch, `attn_workspace` the workspace of the split attention
-        or None for the unsplit one.  Five launches for a single row (six with the split attention),
+        or None for the unsplit one.  Six launches for a single row (five with the unsplit attention),
         eight or nine where the linears cannot take their prologues in the kernel."""
         from . import _glue
         from .ops import PRE_ADD_RMSNORM, PRE_SILU_MUL
 
         cfg = self.cfg
         m = h.shape[0]
-        # Up to four rows the two norms and the SiLU gate ride in the linears behind them (five launches
+        # Up to four rows the two norms and the SiLU gate ride in the linears behind them (six launches
         # per block instead of eight): the residual stream goes h -> x (= h + delta) in the qkv launch
         # and x -> h (= x + attention output) in the gate_up launch, so it is back in `h` at the end.
         in_kernel = self.prologues_apply(m)
@@ -173,9 +173,9 @@ class Block(torch.nn.Module):
             _glue.add_rmsnorm(h, delta, self.input_norm, x, cfg.rms_eps)
             qkv = self.qkv(x)
         attn = torch.empty(m, cfg.hidden, dtype=h.dtype, device=h.device)
-        # For a single row the rotary embedding and the cache write ride in the attention launch.
-        # A long cache is split over workgroups (two launches; measured on MI355X with 32 / 8 heads,
-        # one row: 10.9 against 12.6 us at 1024 rows, 28.9 against 60 us at 8192, 9.7 against 9.4 at 512).
+        # For a single row the rotary embedding and the cache write ride in the attention launch, and the
+        # context is split over workgroups (two launches; measured on MI355X with 32 / 8 heads, split against
+        # unsplit: 5.3 against 6.8 us at 64 rows, 6.5 against 8.3 at 512, 7.5 against 10.9 at 1000, 24.5 against 58.5 at 7900).
         if m > 1:
             _glue.rope_cache(qkv, cos_table, sin_table, pos, k_cache, v_cache, cfg.heads, cfg.kv_heads)
         if attn_workspace is not None:
@@ -235,8 +235,10 @@ class Decoder(torch.nn.Module):
         self.register_buffer("arange", torch.arange(max_context, device=embed.device), persistent=False)
         self.max_context = max_context
         self.fused = True  # decode steps of a few rows use the fused operators between the linears
-        # long caches: context split over workgroups (1, 2, 4 or 8 query heads per key/value head)
-        self.split_attention = max_context > 768 and cfg.heads // cfg.kv_heads in (1, 2, 4, 8)
+        # context split over workgroups (1, 2, 4 or 8 query heads per key/value head): for a single row always, for
+        # several on long caches
+        self.split_single_row = cfg.heads // cfg.kv_heads in (1, 2, 4, 8)
+        self.split_attention = max_context > 768 and self.split_single_row
         self._attn_workspace = None
 
     def new_cache(self):
@@ -269,14 +271,19 @@ class Decoder(torch.nn.Module):
         if self.fused_applies(h.shape[0]):
             from . import _glue
 
-            if self.split_attention and self._attn_workspace is None:
-                # shared by all blocks: their launches follow one another
-                self._attn_workspace = _glue.attention_workspace(16, self.cfg.heads, self.max_context, h.device)
+            # shared by all blocks: their launches follow one another
+            workspace = None
+            if h.shape[0] == 1 and self.split_single_row:
+                # (a step's own, so that sessions on several streams do not share it)
+                workspace = _glue.attention_workspace(1, self.cfg.heads, self.max_context, h.device)
+            elif self.split_attention:
+                if self._attn_workspace is None:
+                    self._attn_workspace = _glue.attention_workspace(16, self.cfg.heads, self.max_context, h.device)
+                workspace = self._attn_workspace
             x = torch.empty_like(h)
             delta = None
             for i, block in enumerate(self.blocks):
-                delta = block.forward_fused(h, delta, x, self.cos, self.sin, pos, cache[i, 0], cache[i, 1],
-                                            self._attn_workspace if self.split_attention else None)
+                delta = block.forward_fused(h, delta, x, self.cos, self.sin, pos, cache[i, 0], cache[i, 1], workspace)
             _glue.add_rmsnorm(h, delta, self.final_norm, x, self.cfg.rms_eps)
             return torch.nn.functional.linear(x[-1:], self.head).float()
         cos, sin = self.cos.index_select(0, pos), self.sin.index_select(0, pos)
