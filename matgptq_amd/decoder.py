@@ -164,7 +164,7 @@ class Block(torch.nn.Module):
         cfg = self.cfg
         m = h.shape[0]
         # Up to four rows the two norms and the SiLU gate ride in the linears behind them (six launches
-        # per block instead of eight): the residual stream goes h -> x (= h + delta) in the qkv launch
+        # per block instead of nine): the residual stream goes h -> x (= h + delta) in the qkv launch
         # and x -> h (= x + attention output) in the gate_up launch, so it is back in `h` at the end.
         in_kernel = self.prologues_apply(m)
         if in_kernel:
