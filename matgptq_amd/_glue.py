@@ -1,8 +1,8 @@
 """ctypes face of the decode-time operators between the linears (include/matgptq_glue.h).
 
 Loaded from `matgptq_amd/lib/libmatgptq_glue.so`, built by `matgptq_amd._build.build_glue()`.
-The functions below take torch tensors on the GPU, launch on torch's current stream and
-return nothing: outputs are written into the tensors passed in.  There is no fallback:
+The functions below take torch tensors on one GPU, launch there on torch's current stream of that
+GPU and return nothing: outputs are written into the tensors passed in.  There is no fallback:
 a missing library raises.
 """
 from __future__ import annotations
@@ -68,8 +68,15 @@ def _f16(*tensors) -> None:
             raise GlueError("expected contiguous float16 tensors on the GPU")
 
 
-def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+def _launch(name: str, tensors, *args) -> None:
+    """Calls `name` with `args` and the stream, on the GPU that all of `tensors` (None: not given) are on,
+    whichever GPU is the current one."""
+    device = tensors[0].device
+    for t in tensors:
+        if t is not None and t.device != device:
+            raise GlueError("the tensors are on different GPUs")
+    with torch.cuda.device(device):
+        _check(getattr(load(), name)(*args, torch.cuda.current_stream().cuda_stream))
 
 
 def add_rmsnorm(h, delta, weight, x, eps: float) -> None:
@@ -78,8 +85,8 @@ def add_rmsnorm(h, delta, weight, x, eps: float) -> None:
     m, hidden = h.shape
     if x.shape != h.shape or weight.numel() != hidden or (delta is not None and delta.shape != h.shape):
         raise GlueError("add_rmsnorm: shapes differ")
-    _check(load().matgptq_glue_add_rmsnorm(h.data_ptr(), None if delta is None else delta.data_ptr(),
-                                           weight.data_ptr(), x.data_ptr(), m, hidden, eps, _stream()))
+    _launch("matgptq_glue_add_rmsnorm", (h, delta, weight, x), h.data_ptr(),
+            None if delta is None else delta.data_ptr(), weight.data_ptr(), x.data_ptr(), m, hidden, eps)
 
 
 def _pos_ok(pos, m: int) -> None:
@@ -97,9 +104,8 @@ def rope_cache(qkv, cos, sin, pos, k_cache, v_cache, heads: int, kv_heads: int) 
     if (kv != kv_heads or v_cache.shape != k_cache.shape or qkv.shape[1] != (heads + 2 * kv_heads) * d
             or cos.shape != (max_ctx, d) or sin.shape != (max_ctx, d)):
         raise GlueError("rope_cache: shapes differ")
-    _check(load().matgptq_glue_rope_cache(qkv.data_ptr(), cos.data_ptr(), sin.data_ptr(), pos.data_ptr(),
-                                          k_cache.data_ptr(), v_cache.data_ptr(), m, heads, kv_heads, d, max_ctx,
-                                          _stream()))
+    _launch("matgptq_glue_rope_cache", (qkv, cos, sin, pos, k_cache, v_cache), qkv.data_ptr(), cos.data_ptr(),
+            sin.data_ptr(), pos.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), m, heads, kv_heads, d, max_ctx)
 
 
 def attention(qkv, k_cache, v_cache, pos, out, heads: int, kv_heads: int) -> None:
@@ -111,8 +117,8 @@ def attention(qkv, k_cache, v_cache, pos, out, heads: int, kv_heads: int) -> Non
     if (kv != kv_heads or v_cache.shape != k_cache.shape or qkv.shape[1] != (heads + 2 * kv_heads) * d
             or out.shape != (m, heads * d)):
         raise GlueError("attention: shapes differ")
-    _check(load().matgptq_glue_attention(qkv.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), pos.data_ptr(),
-                                         out.data_ptr(), m, heads, kv_heads, d, max_ctx, _stream()))
+    _launch("matgptq_glue_attention", (qkv, k_cache, v_cache, pos, out), qkv.data_ptr(), k_cache.data_ptr(),
+            v_cache.data_ptr(), pos.data_ptr(), out.data_ptr(), m, heads, kv_heads, d, max_ctx)
 
 
 def rope_attention(qkv, cos, sin, pos, k_cache, v_cache, out, heads: int, kv_heads: int) -> None:
@@ -124,9 +130,9 @@ def rope_attention(qkv, cos, sin, pos, k_cache, v_cache, out, heads: int, kv_hea
             or qkv.shape[1] != (heads + 2 * kv_heads) * d or cos.shape != (max_ctx, d) or sin.shape != (max_ctx, d)
             or out.shape != (1, heads * d)):
         raise GlueError("rope_attention: shapes differ")
-    _check(load().matgptq_glue_rope_attention(qkv.data_ptr(), cos.data_ptr(), sin.data_ptr(), pos.data_ptr(),
-                                              k_cache.data_ptr(), v_cache.data_ptr(), out.data_ptr(), heads,
-                                              kv_heads, d, max_ctx, _stream()))
+    _launch("matgptq_glue_rope_attention", (qkv, cos, sin, pos, k_cache, v_cache, out), qkv.data_ptr(),
+            cos.data_ptr(), sin.data_ptr(), pos.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), out.data_ptr(),
+            heads, kv_heads, d, max_ctx)
 
 
 def attention_workspace(rows: int, heads: int, max_ctx: int, device):
@@ -150,10 +156,11 @@ def attention_split(qkv, cos, sin, pos, k_cache, v_cache, out, workspace, heads:
     if (workspace.dtype != torch.float32 or not workspace.is_cuda or not workspace.is_contiguous()
             or workspace.numel() < need):
         raise GlueError("attention_split: workspace too small or of the wrong type")
-    _check(load().matgptq_glue_attention_split(
-        qkv.data_ptr(), cos.data_ptr() if fuse_rotary else None, sin.data_ptr() if fuse_rotary else None,
-        pos.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), out.data_ptr(), workspace.data_ptr(),
-        m, heads, kv_heads, d, max_ctx, int(fuse_rotary), _stream()))
+    cos, sin = (cos, sin) if fuse_rotary else (None, None)
+    _launch("matgptq_glue_attention_split", (qkv, cos, sin, pos, k_cache, v_cache, out, workspace), qkv.data_ptr(),
+            None if cos is None else cos.data_ptr(), None if sin is None else sin.data_ptr(), pos.data_ptr(),
+            k_cache.data_ptr(), v_cache.data_ptr(), out.data_ptr(), workspace.data_ptr(), m, heads, kv_heads, d, max_ctx,
+            int(fuse_rotary))
 
 
 def rope_prompt(qkv, cos_rows, sin_rows, pos, q_out, k_cache, v_cache, heads: int, kv_heads: int) -> None:
@@ -166,9 +173,9 @@ def rope_prompt(qkv, cos_rows, sin_rows, pos, q_out, k_cache, v_cache, heads: in
     if (kv != kv_heads or v_cache.shape != k_cache.shape or qkv.shape[1] != (heads + 2 * kv_heads) * d
             or cos_rows.shape != (m, d) or sin_rows.shape != (m, d) or q_out.shape != (heads, m, d)):
         raise GlueError("rope_prompt: shapes differ")
-    _check(load().matgptq_glue_rope_prompt(qkv.data_ptr(), cos_rows.data_ptr(), sin_rows.data_ptr(), pos.data_ptr(),
-                                           q_out.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), m, heads,
-                                           kv_heads, d, max_ctx, _stream()))
+    _launch("matgptq_glue_rope_prompt", (qkv, cos_rows, sin_rows, pos, q_out, k_cache, v_cache), qkv.data_ptr(),
+            cos_rows.data_ptr(), sin_rows.data_ptr(), pos.data_ptr(), q_out.data_ptr(), k_cache.data_ptr(),
+            v_cache.data_ptr(), m, heads, kv_heads, d, max_ctx)
 
 
 def heads_to_rows(x, out) -> None:
@@ -177,7 +184,7 @@ def heads_to_rows(x, out) -> None:
     heads, m, d = x.shape
     if out.shape != (m, heads * d):
         raise GlueError("heads_to_rows: shapes differ")
-    _check(load().matgptq_glue_heads_to_rows(x.data_ptr(), out.data_ptr(), m, heads, d, _stream()))
+    _launch("matgptq_glue_heads_to_rows", (x, out), x.data_ptr(), out.data_ptr(), m, heads, d)
 
 
 def silu_mul(gate_up, out, prompt: bool = False) -> None:
@@ -186,8 +193,8 @@ def silu_mul(gate_up, out, prompt: bool = False) -> None:
     m, f = out.shape
     if gate_up.shape != (m, 2 * f):
         raise GlueError("silu_mul: shapes differ")
-    fn = load().matgptq_glue_silu_mul_prompt if prompt else load().matgptq_glue_silu_mul
-    _check(fn(gate_up.data_ptr(), out.data_ptr(), m, f, _stream()))
+    _launch("matgptq_glue_silu_mul_prompt" if prompt else "matgptq_glue_silu_mul", (gate_up, out), gate_up.data_ptr(),
+            out.data_ptr(), m, f)
 
 
 def argmax(x, out) -> None:
@@ -195,4 +202,4 @@ def argmax(x, out) -> None:
     if (x.dtype != torch.float32 or out.dtype != torch.int64 or not x.is_cuda or not out.is_cuda
             or not x.is_contiguous() or not out.is_contiguous() or x.dim() != 2 or out.shape != (x.shape[0],)):
         raise GlueError("argmax: fp32 [M, n] in, int64 [M] out, contiguous, on the GPU")
-    _check(load().matgptq_glue_argmax(x.data_ptr(), out.data_ptr(), x.shape[0], x.shape[1], _stream()))
+    _launch("matgptq_glue_argmax", (x, out), x.data_ptr(), out.data_ptr(), x.shape[0], x.shape[1])
