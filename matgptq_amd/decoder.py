@@ -239,7 +239,6 @@ class Decoder(torch.nn.Module):
         # several on long caches
         self.split_single_row = cfg.heads // cfg.kv_heads in (1, 2, 4, 8)
         self.split_attention = max_context > 768 and self.split_single_row
-        self._attn_workspace = None
 
     def new_cache(self):
         cfg = self.cfg
@@ -271,15 +270,11 @@ class Decoder(torch.nn.Module):
         if self.fused_applies(h.shape[0]):
             from . import _glue
 
-            # shared by all blocks: their launches follow one another
+            # a step's own, so that sessions on several streams do not share it; shared by all blocks, whose
+            # launches follow one another
             workspace = None
-            if h.shape[0] == 1 and self.split_single_row:
-                # (a step's own, so that sessions on several streams do not share it)
-                workspace = _glue.attention_workspace(1, self.cfg.heads, self.max_context, h.device)
-            elif self.split_attention:
-                if self._attn_workspace is None:
-                    self._attn_workspace = _glue.attention_workspace(16, self.cfg.heads, self.max_context, h.device)
-                workspace = self._attn_workspace
+            if self.split_attention or (h.shape[0] == 1 and self.split_single_row):
+                workspace = _glue.attention_workspace(h.shape[0], self.cfg.heads, self.max_context, h.device)
             x = torch.empty_like(h)
             delta = None
             for i, block in enumerate(self.blocks):

@@ -272,3 +272,24 @@ def test_graph_replays_equal_eager_fused_steps():
     assert torch.equal(eager, graph)
     again = s.generate(prompt, 12, use_graph=True)  # the captured step starts over from a new prompt
     assert torch.equal(eager, again)
+
+
+def test_short_prompts_on_two_streams_equal_prompts_one_after_the_other():
+    # a long cache: the attention of 8 rows is split and leaves its partial results in a workspace
+    D, cfg, dec = _decoder(context=1100)
+    assert dec.split_attention
+    prompts = [torch.randint(0, cfg.vocab, (8,), device=DEV, generator=_gen(i)) for i in (1, 2)]
+    want = []
+    for prompt in prompts:
+        s = D.DecodeSession(dec)
+        s.prefill(prompt)
+        want.append((s.logits, s.cache))
+    sessions = [D.DecodeSession(dec) for _ in prompts]
+    torch.cuda.synchronize()
+    for _ in range(10):
+        for s, prompt in zip(sessions, prompts):
+            with torch.cuda.stream(s.stream):
+                s.prefill(prompt)
+        torch.cuda.synchronize()
+        for s, (logits, cache) in zip(sessions, want):
+            assert torch.equal(s.logits, logits) and torch.equal(s.cache, cache)
