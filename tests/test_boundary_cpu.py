@@ -113,3 +113,73 @@ def test_plugin_create_weights_shapes_and_alignment_error():
     assert (layer.scales.input_dim, layer.scales.output_dim, layer.scales.packed_dim) == (1, 0, 1)
     with pytest.raises(ValueError, match="not a multiple of the quantisation group size"):
         m.create_weights(torch.nn.Module(), 200, [32], 200, 32, torch.float16)
+
+
+def _hold(layer, name, tensor, how):
+    if how == "parameter":
+        layer.register_parameter(name, torch.nn.Parameter(tensor, requires_grad=False))
+    elif how == "buffer":
+        layer.register_buffer(name, tensor)
+    else:
+        setattr(layer, name, tensor)
+
+
+def _loaded_layer(monkeypatch, how, layer=None, **config):
+    """A layer after loading on the host, with packers that hand their input back."""
+    ops = torch.ops.matgptq_cuda
+    monkeypatch.setattr(ops, "pack_matgptq_qweights", lambda q, *_: q.clone())
+    monkeypatch.setattr(ops, "reorder_matgptq_scales", lambda t, *_: t.clone())
+    method = vllm_matgptq.MatGPTQLinearMethod(vllm_matgptq.MatGPTQConfig(128, 8, 8, "float16", **config))
+    method.n_out_features, method.n_in_features = 16, 256
+    layer = torch.nn.Module() if layer is None else layer
+    given = {"qweight": torch.arange(16 * 256).view(16, 256).to(torch.uint8), "scales": torch.rand(16, 2).half(),
+             "zeros": torch.full((16, 2), 120.0).half(), "perm": torch.randperm(256, dtype=torch.int32)}
+    for name, tensor in given.items():
+        if name in how:
+            _hold(layer, name, tensor, how[name])
+    method.process_weights_after_loading(layer)
+    return method, layer, given
+
+
+@pytest.mark.parametrize("how", ("parameter", "buffer", "attribute"))
+def test_plugin_takes_tensors_however_the_loader_left_them(monkeypatch, how):
+    names = ("qweight", "scales", "zeros", "perm")
+    _, layer, given = _loaded_layer(monkeypatch, dict.fromkeys(names, how))
+    assert torch.equal(layer.matgptq_weights, given["qweight"]) and torch.equal(layer.matgptq_scales, given["scales"])
+    assert torch.equal(layer.matgptq_zeros, given["zeros"])
+    assert torch.equal(layer.matgptq_perm, given["perm"].long())
+    assert layer.matgptq_planes is None and layer.matgptq_bitwidth == 8
+    assert not any(hasattr(layer, name) for name in names)
+    assert {"matgptq_weights", "matgptq_scales", "matgptq_zeros", "matgptq_perm"} == set(layer._parameters)
+
+
+def test_plugin_layer_without_zeros_and_perm_and_loaded_again(monkeypatch):
+    plain = {"qweight": "parameter", "scales": "parameter"}
+    _, layer, given = _loaded_layer(monkeypatch, {**plain, "zeros": "buffer"}, keep_master_codes=True)
+    assert layer.matgptq_zeros is not None and layer.matgptq_perm is None
+    assert torch.equal(layer.matgptq_master, given["qweight"])
+    _, again, given = _loaded_layer(monkeypatch, plain, layer=layer)
+    assert again is layer and layer.matgptq_zeros is None and layer.matgptq_perm is None
+    assert torch.equal(layer.matgptq_scales, given["scales"])
+
+
+def test_plugin_parameters_are_registered_the_modules_way(monkeypatch):
+    class Watched(torch.nn.Module):
+        seen = []
+
+        def __setattr__(self, name, value):
+            if name.startswith("matgptq_"):
+                self.seen.append(name)
+            super().__setattr__(name, value)
+
+    everything = dict.fromkeys(("qweight", "scales", "zeros", "perm"), "parameter")
+    _loaded_layer(monkeypatch, everything, layer=Watched())
+    assert {"matgptq_weights", "matgptq_scales", "matgptq_zeros", "matgptq_perm", "matgptq_bitwidth"} <= set(Watched.seen)
+    registered = []
+    handle = torch.nn.modules.module.register_module_parameter_registration_hook(
+        lambda module, name, value: registered.append(name))
+    try:
+        _loaded_layer(monkeypatch, everything)
+    finally:
+        handle.remove()
+    assert {"matgptq_weights", "matgptq_scales", "matgptq_zeros", "matgptq_perm"} <= set(registered)

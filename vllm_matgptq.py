@@ -180,6 +180,25 @@ class MatGPTQConfig(QuantizationConfig):
         return None
 
 
+def _setter(layer: torch.nn.Module):
+    """`setattr(layer, name, value)` for parameters and plain values.  Where nothing else takes part - Module's own
+    __setattr__, no registration hooks, a name that the module does not hold yet - this is what it comes to without
+    its look-ups (22 -> 15 us on the host per layer, of which loading has hundreds)."""
+    cls, own, params, buffers, modules = type(layer), layer.__dict__, layer._parameters, layer._buffers, layer._modules
+    hooks = getattr(torch.nn.modules.module, "_global_parameter_registration_hooks", True)
+    by_module = bool(hooks) or cls.__setattr__ is not torch.nn.Module.__setattr__
+
+    def put(name: str, value) -> None:
+        if by_module or name in own or name in params or name in buffers or name in modules or hasattr(cls, name):
+            setattr(layer, name, value)
+        elif isinstance(value, Parameter):
+            params[name] = value
+        else:
+            own[name] = value
+
+    return put
+
+
 class MatGPTQLinearMethod(LinearMethodBase):
     """Linear method (reference: inference_lib/vllm_matgptq.py:89-201)."""
 
@@ -247,8 +266,7 @@ class MatGPTQLinearMethod(LinearMethodBase):
     def _pack_all(self, layer: torch.nn.Module) -> List[torch.Tensor]:
         """Packed codes (or resident planes), scales and, if the layer has them, zeros in the kernels' order."""
         ops, config = torch.ops.matgptq_cuda, self.config
-        params = layer._parameters
-        qweight, scales, zeros = params["qweight"].data, params["scales"].data.contiguous(), params.get("zeros")
+        qweight, scales, zeros = layer.qweight.data, layer.scales.data.contiguous(), getattr(layer, "zeros", None)
         zeros = None if zeros is None else zeros.data.to(scales.dtype).contiguous()
         planes = config.resident_master_planes
         if (qweight.is_cuda and config.master_bitwidth == 8 and scales.device == qweight.device
@@ -265,38 +283,29 @@ class MatGPTQLinearMethod(LinearMethodBase):
         return packed
 
     def process_weights_after_loading(self, layer: torch.nn.Module) -> None:
-        # A model has hundreds of layers: names are put into the module's own tables, which is what
-        # Module.__setattr__ comes to after about 2 us of look-ups per name.
-        params, plain = layer._parameters, layer.__dict__
-
-        def put(name: str, value: Optional[torch.Tensor]) -> None:
-            if value is None:
-                params.pop(name, None)
-                plain[name] = None
-            else:
-                plain.pop(name, None)
-                params[name] = Parameter(value, requires_grad=False)
-
+        # (a loader may have left any of them as a parameter, a buffer or a plain tensor)
         with torch.no_grad():
-            qweight = params["qweight"].data
-            packed = self._pack_all(layer)
+            qweight = layer.qweight.data
+            packed = [Parameter(t, requires_grad=False) for t in self._pack_all(layer)]
             planes = self.config.resident_master_planes
+            put = _setter(layer)
             put("matgptq_planes", packed[0] if planes else None)
             put("matgptq_weights", None if planes else packed[0])
-            plain["matgptq_bitwidth"] = self.bitwidth
+            put("matgptq_bitwidth", self.bitwidth)
             put("matgptq_scales", packed[1])
             put("matgptq_zeros", packed[2] if len(packed) > 2 else None)
-            perm = params.pop("perm", None)
+            perm = getattr(layer, "perm", None)
             # act-order: the codes are stored in permuted column order and the input features
             # are gathered with the permutation (src/quant_utils_matgpqt.py:218-220)
-            put("matgptq_perm", None if perm is None else
-                perm.data.to(device=packed[1].device, dtype=torch.int64).reshape(-1))
+            put("matgptq_perm", None if perm is None else Parameter(
+                perm.data.to(device=packed[1].device, dtype=torch.int64).reshape(-1), requires_grad=False))
             if self.config.keep_master_codes and not planes:
                 # The reference deletes the master codes here (inference_lib/vllm_matgptq.py:177-178);
                 # kept, a layer can be re-sliced to another bitwidth without the checkpoint.
-                put("matgptq_master", qweight.to(packed[1].device))
-            for name in ("qweight", "scales", "zeros"):
-                params.pop(name, None)
+                put("matgptq_master", Parameter(qweight.to(packed[1].device), requires_grad=False))
+            for name, given in (("qweight", True), ("scales", True), ("zeros", len(packed) > 2), ("perm", perm is not None)):
+                if given:
+                    delattr(layer, name)
 
     def set_bitwidth(self, layer: torch.nn.Module, bitwidth: int) -> None:
         """Moves a loaded layer to `bitwidth`.  With `resident_master_planes` nothing is touched but
