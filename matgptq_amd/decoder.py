@@ -237,8 +237,19 @@ class Decoder(torch.nn.Module):
         self.fused = True  # decode steps of a few rows use the fused operators between the linears
         # context split over workgroups (1, 2, 4 or 8 query heads per key/value head): for a single row always, for
         # several on long caches
-        self.split_single_row = cfg.heads // cfg.kv_heads in (1, 2, 4, 8)
-        self.split_attention = max_context > 768 and self.split_single_row
+        covered = cfg.heads // cfg.kv_heads in (1, 2, 4, 8)
+        self.split_attention = max_context > 768 and covered
+        self.split_single_row = covered
+
+    @property
+    def split_attention(self) -> bool:
+        """Whether decode steps of several rows split their attention over workgroups; set, it switches the split on or
+        off for single rows (`split_single_row`) too."""
+        return self._split_rows
+
+    @split_attention.setter
+    def split_attention(self, on: bool) -> None:
+        self._split_rows = self.split_single_row = on
 
     def new_cache(self):
         cfg = self.cfg
@@ -273,7 +284,7 @@ class Decoder(torch.nn.Module):
             # a step's own, so that sessions on several streams do not share it; shared by all blocks, whose
             # launches follow one another
             workspace = None
-            if self.split_attention or (h.shape[0] == 1 and self.split_single_row):
+            if self.split_single_row if h.shape[0] == 1 else self.split_attention:
                 workspace = _glue.attention_workspace(h.shape[0], self.cfg.heads, self.max_context, h.device)
             x = torch.empty_like(h)
             delta = None

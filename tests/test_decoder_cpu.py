@@ -38,3 +38,18 @@ def test_steps_do_not_share_their_attention_workspace(monkeypatch, rows):
     assert first[0].data_ptr() != second[0].data_ptr()
     for workspace in (first[0], second[0]):
         assert workspace.numel() >= _glue.load().matgptq_glue_attention_workspace_floats(rows, 4, 1100)
+
+
+@pytest.mark.parametrize("context", (64, 1100))
+def test_split_attention_switches_the_split_for_every_number_of_rows(monkeypatch, context):
+    decoder = _decoder(monkeypatch, context)
+    assert decoder.split_attention == (context > 768)
+    assert (_step(decoder, 8)[0] is not None) == (context > 768) and _step(decoder, 1)[0] is not None
+    for on in (False, True):
+        decoder.split_attention = on
+        assert [(_step(decoder, rows)[0] is not None) for rows in (1, 8)] == [on, on]
+
+
+def test_ratios_that_the_split_does_not_cover(monkeypatch):
+    decoder = _decoder(monkeypatch, 1100, heads=6, kv_heads=2)
+    assert not decoder.split_attention and _step(decoder, 1)[0] is None and _step(decoder, 8)[0] is None
