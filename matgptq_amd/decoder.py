@@ -31,6 +31,7 @@ from dataclasses import dataclass
 from typing import Dict, List, Optional, Sequence, Union
 
 import torch
+from torch.utils._python_dispatch import is_in_torch_dispatch_mode
 
 from .checkpoint import load_quantised_layer, read_layer_bitwidths
 from .ops import matryoshka_slice
@@ -217,6 +218,14 @@ def _rotate(t, cos, sin):
     return t * cos[:, None, :] + rot * sin[:, None, :]
 
 
+def _plain_tensors(*tensors) -> bool:
+    """Whether these are tensors with memory, in code that runs as it stands: not while it is traced, exported,
+    transformed or watched by a dispatch mode, which see torch operators and not kernels called by address."""
+    return (not torch.compiler.is_compiling() and not torch.jit.is_tracing() and not is_in_torch_dispatch_mode()
+            and all(type(t) in (torch.Tensor, torch.nn.Parameter) and not torch._C._functorch.is_functorch_wrapped_tensor(t)
+                    for t in tensors))
+
+
 class Decoder(torch.nn.Module):
     def __init__(self, cfg: DecoderConfig, blocks: Sequence[Block], embed: torch.Tensor, head: torch.Tensor,
                  max_context: int):
@@ -267,12 +276,13 @@ class Decoder(torch.nn.Module):
         """A prompt's layout copies and element-wise operators as one kernel each: fp16, head dimension 128, tensors as
         those kernels address them (plain torch takes any).  512 rows of 32 Llama-3-8B blocks: 13.24 -> 11.29 ms."""
         cfg = self.cfg
-        return (self.fused and pos.numel() <= 65535 and self.embed.dtype == torch.float16 and self.embed.is_cuda
+        return (self.fused and _plain_tensors(self.embed, pos, cache) and pos.numel() <= 65535 and self.embed.dtype == torch.float16 and self.embed.is_cuda
                 and cfg.hidden == cfg.heads * 128 and cfg.heads % cfg.kv_heads == 0 and cfg.ffn % 8 == 0
                 and pos.dim() == 1 and pos.dtype == torch.int64 and pos.is_contiguous()
                 and cache.dtype == torch.float16 and cache.is_contiguous() and cache.data_ptr() % 16 == 0
                 and tuple(cache.shape) == (len(self.blocks), 2, cfg.kv_heads, self.max_context, 128)
-                and all(type(block).forward is Block.forward for block in self.blocks))
+                and all(type(block).forward is Block.forward and "forward" not in vars(block)
+                        and getattr(block, "_compiled_call_impl", None) is None for block in self.blocks))
 
     @torch.no_grad()
     def forward(self, tokens, pos, cache):
