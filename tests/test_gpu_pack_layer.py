@@ -40,3 +40,21 @@ def test_layer_in_one_launch_equals_host_packers(n, k, g, b, source):
         assert np.array_equal(got.cpu().numpy().view(np.uint16), want)
     without = torch.ops.matgptq_cuda.pack_matgptq_layer(torch.from_numpy(codes).cuda(), dev[0], None, b, g, source)
     assert len(without) == 2 and torch.equal(without[0].view(torch.int32), packed.view(torch.int32))
+
+
+@pytest.mark.parametrize("b", (2, 3, 4, 6, 8))
+@pytest.mark.parametrize("offset", (0, 1, 4, 8, 12, 16))
+@pytest.mark.parametrize("count", (1, 15, 16, 63, 4096 * 16 + 7))
+def test_slice_at_every_alignment(count, offset, b):
+    # 16 bytes per thread where the codes lie on 4 bytes, code by code elsewhere and at the end
+    L = _lib.load()
+    q = np.random.default_rng(count + offset).integers(0, 256, count, dtype=np.uint8)
+    src = torch.zeros(count + offset, dtype=torch.uint8, device="cuda")
+    src[offset:] = torch.from_numpy(q).cuda()
+    for out_offset in {0, offset}:
+        out = torch.full((count + out_offset + 16,), 255, dtype=torch.uint8, device="cuda")
+        _lib.check(L.matgptq_slice_device(src.data_ptr() + offset, count, b, out.data_ptr() + out_offset,
+                                          torch.cuda.current_stream().cuda_stream))
+        got = out.cpu().numpy()
+        assert np.array_equal(got[out_offset:out_offset + count], o.slice_codes(q, b))
+        assert (got[:out_offset] == 255).all() and (got[out_offset + count:] == 255).all()
