@@ -218,6 +218,9 @@ int matgptq_gemm_master_static(int bitwidth, int group_size, int64_t N, int64_t 
 /* Human-readable name of the kernel variant matgptq_gemm would launch. */
 int matgptq_describe_plan(int bitwidth, int group_size, int64_t N, int64_t K, int64_t M,
                           int has_zeros, uint32_t flags, char *buf, size_t buf_len);
+/* Activation buffers (1 or 2) of the mid-batch kernel that matgptq_gemm would launch; 0 where it launches another one,
+ * negative on an error. */
+int matgptq_midbatch_buffers(int bitwidth, int group_size, int64_t N, int64_t K, int64_t M, int has_zeros, uint32_t flags);
 
 #ifdef __cplusplus
 }

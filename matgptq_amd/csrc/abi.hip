@@ -10,6 +10,7 @@
 
 #include "../../include/matgptq_abi.h"
 #include "device_common.h"
+#include "midbatch_plan.h"
 #include "prefill_plan.h"
 
 // Scratch of matgptq_gemm_master_static: device memory that lives in the library's code object, so
@@ -853,6 +854,16 @@ int matgptq_describe_plan(int bitwidth, int group_size, int64_t N, int64_t K, in
     snprintf(buf, buf_len, "prefill b%d g%d zp%d cfg%d", bitwidth, group_size, has_zeros ? 1 : 0,
              p.cfg);
   return MATGPTQ_OK;
+}
+
+int matgptq_midbatch_buffers(int bitwidth, int group_size, int64_t N, int64_t K, int64_t M, int has_zeros, uint32_t flags) {
+  if (int e = check_problem(bitwidth, group_size, N, K)) return e;
+  if (M <= 0) return MATGPTQ_ESIZE;
+  Plan p;
+  if (int e = make_plan(bitwidth, group_size, N, K, M, has_zeros != 0, flags, &p)) return e;
+  if (!p.skinny) return 0;
+  return midbatch_two_buffers(bitwidth, (flags & MATGPTQ_FLAG_BF16) != 0, group_size, has_zeros != 0, p.R, p.mb, false,
+                              (int)(K / 128), (int)M, (int)(N / 16)) ? 2 : 1;
 }
 
 int matgptq_pack_device(const uint8_t* codes_dev, int64_t N, int64_t K, int bitwidth,

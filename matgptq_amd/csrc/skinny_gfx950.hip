@@ -30,8 +30,8 @@
 //    barrier in the loop;
 //  * with two buffers (BUFS = 2) tile t + 2 is requested while t is multiplied and t + 1 is on its way, and the
 //    codes have two register sets that are refilled behind the multiplication.  That pays where a wave alone on its
-//    SIMD waits for its copies, and where several rounds of workgroups keep the copies queued; the rule is at
-//    two_buffers below;
+//    SIMD waits for its copies, and where several rounds of workgroups keep the copies queued; the rule is in
+//    midbatch_plan.h;
 //  * every load is branch-free (tiles beyond K, rows beyond M or N go through a zero-length
 //    buffer descriptor or an out-of-range offset);
 //  * the eight partial sums meet in LDS once, at the end; the threads add them and store four
@@ -39,6 +39,7 @@
 //
 // The activations are re-read once per workgroup column (N / (16 R) times in total, from L2):
 // that traffic, not the weights, bounds this kernel, which is why R grows with N.
+#include "midbatch_plan.h"
 #include "tile_format.h"
 
 #ifndef MATGPTQ_BITS
@@ -310,33 +311,13 @@ skinny_kernel(const GemmArgs a, int n_tiles, int m_tiles) {
   }
 }
 
-// Two buffers, on pre-sliced codes and up to 32 batch rows per workgroup (the second buffer is another 32 KB per 16
-// batch rows).  us, one -> two buffers, 4 bits where nothing else is said:
-//  * a walk of one tile, whose second tile the loop of pairs would wait for: 8192 x 1024 at M = 16 / 32 / 64
-//    4.29 -> 3.98 / 5.28 -> 4.77 / 6.30 -> 5.69, 8192 x 512 at M = 10 3.74 -> 3.36, 8192 x 1024 at 6 bits and M = 51 7.91 -> 6.48;
-//  * one row block per workgroup: 2048 x 4096 at M = 12 / 32 / 64 5.16 -> 4.82 / 6.93 -> 6.61 / 6.79 -> 6.57, 4096 x 4096 at M = 12
-//    5.53 -> 5.28 (several blocks of 32 batch rows and a longer walk: 1280 x 8192 at M = 49, 6 bits, 9.98 against 10.69);
-//  * 16 batch rows and more workgroups than CUs, fp16 storage: 28672 x 4096 at M = 8 / 12 / 16 16.3 -> 15.5 / 17.6 -> 16.0 / 17.6 -> 16.6,
-//    12288 x 2560 at M = 6 and 8 bits 11.1 -> 10.0, 57344 x 8192 at M = 10 49.0 -> 47.9 (the weights of bf16 storage, and 8 bits with
-//    their four scales per tile at group size 32, take more registers: 28672 x 4096 at M = 13 17.3 against 19.3,
-//    16384 x 2048 at M = 12 11.2 against 12.3).
-// Elsewhere one buffer is as fast or ahead by up to 5 % (8192 x 3584 at M = 16: 6.74 against 7.02, 7168 x 8192 at M = 22 and 2
-// bits 11.2 against 11.8).
-template <int GROUP, int R, int MB, bool MASTER>
-bool two_buffers(const GemmArgs& a, int workgroups) {
-  if (MASTER || R > 4 || MB > 2) return false;
-  if (a.k_tiles <= kWaves) return true;
-  if (R == 1) return a.M <= 32 || a.k_tiles <= 4 * kWaves;
-  return MB == 1 && !kBf16 && !(GROUP == 32 && kBits == 8) && workgroups > 256;
-}
-
 template <int GROUP, bool ZP, int R, int MB, bool MASTER>
 hipError_t launch_r(const GemmArgs& a, hipStream_t stream) {
   const int n_tiles = (a.row_blocks + R - 1) / R;
   const int m_tiles = (a.M + 16 * MB - 1) / (16 * MB);
   const dim3 grid(n_tiles * m_tiles), block(64 * kWaves);
   constexpr int kTwo = !MASTER && R <= 4 && MB <= 2 ? 2 : 1;
-  if (kTwo == 2 && two_buffers<GROUP, R, MB, MASTER>(a, n_tiles * m_tiles))
+  if (kTwo == 2 && midbatch_two_buffers(kBits, kBf16, GROUP, ZP, R, MB, MASTER, a.k_tiles, a.M, a.row_blocks))
     hipLaunchKernelGGL((skinny_kernel<kBits, GROUP, ZP, R, MB, MASTER, kTwo>), grid, block, 0, stream, a, n_tiles, m_tiles);
   else
     hipLaunchKernelGGL((skinny_kernel<kBits, GROUP, ZP, R, MB, MASTER, 1>), grid, block, 0, stream, a, n_tiles, m_tiles);

@@ -446,3 +446,38 @@ def test_planner_answers_every_valid_shape_within_its_kernels_domains():
         else:
             assert kind.startswith("decode") and m <= 16, plan
     assert {"gemv", "midbatch", "prefill"} <= seen
+
+
+def test_midbatch_buffers_at_the_edges_of_the_rule():
+    buffers = _lib.load().matgptq_midbatch_buffers
+    bf16, plain = 3, 1
+
+    def forced(row_blocks_sel, batch_sel):
+        return (80 + row_blocks_sel + 3 * batch_sel) << 8
+
+    assert buffers(4, 128, 4096, 4096, 1, 1, plain) == 0        # another kernel
+    assert buffers(5, 128, 4096, 4096, 16, 1, plain) < 0 and buffers(4, 128, 4096, 4096, 0, 1, plain) < 0
+    # a walk of one tile: every format and shape that has the second buffer at all (up to 32 batch rows, four row blocks)
+    for bits, flags in ((2, plain), (4, bf16), (6, plain), (8, bf16)):
+        assert buffers(bits, 128, 256, 1024, 16, 1, flags | forced(1, 0)) == 2
+        assert buffers(bits, 32, 256, 1024, 30, 1, flags | forced(0, 1)) == 2
+    assert buffers(4, 128, 256, 1024, 60, 1, plain | forced(0, 2)) == 1   # 64 batch rows
+    assert buffers(4, 128, 256, 1024, 30, 1, plain | (91 << 8)) == 1      # eight row blocks
+    # one row block, 16 batch rows: 3 | 4 tiles with zero points at group 32, 5 | 6 at 6 bits
+    one = forced(0, 0)
+    assert [buffers(4, 32, 256, k, 16, 1, plain | one) for k in (3072, 3200)] == [2, 1]
+    assert [buffers(4, 32, 256, k, 16, 0, plain | one) for k in (3072, 3200)] == [2, 2]
+    assert [buffers(6, 128, 256, k, 16, 1, plain | one) for k in (3072, 3200, 4096, 4224, 5120, 5248)] == [2, 1, 1, 2, 2, 1]
+    # one row block, 32 batch rows: two tiles in at most 256 workgroups, three, then odd walks of fp16 storage
+    two = forced(0, 1)
+    assert [buffers(4, 128, 16 * w, 2048, 32, 1, plain | two) for w in (256, 257)] == [2, 1]
+    assert [buffers(4, 128, 16 * 300, 3072, 32, 1, f | two) for f in (plain, bf16)] == [2, 2]
+    assert [buffers(4, 128, 256, 5120, 32, 1, f | two) for f in (plain, bf16)] == [2, 1]
+    assert [buffers(4, 128, 256, 4096, 32, 1, f | two) for f in (plain, bf16)] == [1, 1]
+    assert buffers(4, 128, 256, 5120, 33, 1, plain | two) == 1            # more than 32 batch rows, a long walk
+    # several row blocks: fp16 storage, 16 batch rows, more than 256 workgroups
+    assert [buffers(4, 128, 32 * w, 2048, 16, 1, plain | forced(1, 0)) for w in (256, 257)] == [1, 2]
+    assert buffers(4, 128, 32 * 257, 2048, 16, 1, bf16 | forced(1, 0)) == 1
+    assert [buffers(8, g, 32 * 257, 2048, 16, 1, plain | forced(1, 0)) for g in (128, 32)] == [2, 1]
+    assert [buffers(6, 128, 64 * 257, 2048, 16, z, plain | forced(2, 0)) for z in (0, 1)] == [2, 1]
+    assert buffers(4, 128, 64 * 257, 2048, 16, 1, plain | forced(2, 0)) == 2
