@@ -241,7 +241,7 @@ def _decoder(context=80, seed=5):
     return D, cfg, dec
 
 
-@pytest.mark.parametrize("context", (80, 1100))  # short cache: one attention launch; long: split over workgroups
+@pytest.mark.parametrize("context", (80, 1100))  # three rows: one attention launch on the short cache; all others are split
 @pytest.mark.parametrize("rows", (1, 3))
 def test_fused_step_matches_step_of_torch_operators(rows, context):
     D, cfg, dec = _decoder(context)
