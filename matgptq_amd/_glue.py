@@ -12,6 +12,8 @@ import os
 
 import torch
 
+from .ops import raw_stream
+
 _HERE = os.path.dirname(os.path.abspath(__file__))
 GLUE_PATH = os.path.join(_HERE, "lib", "libmatgptq_glue.so")
 MAX_CONTEXT = 8192
@@ -71,12 +73,16 @@ def _f16(*tensors) -> None:
 def _launch(name: str, tensors, *args) -> None:
     """Calls `name` with `args` and the stream, on the GPU that all of `tensors` (None: not given) are on,
     whichever GPU is the current one."""
-    device = tensors[0].device
+    index = tensors[0].get_device()
     for t in tensors:
-        if t is not None and t.device != device:
+        if t is not None and t.get_device() != index:
             raise GlueError("the tensors are on different GPUs")
-    with torch.cuda.device(device):
-        _check(getattr(load(), name)(*args, torch.cuda.current_stream().cuda_stream))
+    fn, stream = getattr(load(), name), raw_stream(index)
+    if index == torch.cuda.current_device():
+        _check(fn(*args, stream))
+    else:
+        with torch.cuda.device(index):
+            _check(fn(*args, stream))
 
 
 def add_rmsnorm(h, delta, weight, x, eps: float) -> None:

@@ -3,7 +3,6 @@ header declares, and rejects bad arguments before anything is launched."""
 import ctypes
 import os
 import re
-import types
 
 import pytest
 import torch
@@ -70,6 +69,9 @@ class _GpuTensor:
     def data_ptr(self):
         return 4096
 
+    def get_device(self):
+        return self.device.index
+
 
 class _Gpus:
     """A library whose calls return 0 and note the GPU that was current and the stream they were given; the
@@ -81,7 +83,7 @@ class _Gpus:
 
         class Device:
             def __init__(self, device):
-                self.index = torch.device(device).index
+                self.index = device
 
             def __enter__(self):
                 self.before, gpus.current = gpus.current, self.index
@@ -99,15 +101,11 @@ class _Gpus:
                     return 0
                 return call
 
-        def current_stream(device=None):
-            index = gpus.current if device is None else torch.device(device).index
-            return types.SimpleNamespace(cuda_stream=100 + index)
-
         library = Library()
         monkeypatch.setattr(_glue, "load", lambda: library)
         monkeypatch.setattr(torch.cuda, "device", Device)
         monkeypatch.setattr(torch.cuda, "current_device", lambda: gpus.current)
-        monkeypatch.setattr(torch.cuda, "current_stream", current_stream)
+        monkeypatch.setattr(_glue, "raw_stream", lambda index: 100 + index)
 
 
 def _operator_calls(device, other=None):
