@@ -183,7 +183,7 @@ class MatGPTQConfig(QuantizationConfig):
 def _setter(layer: torch.nn.Module):
     """`setattr(layer, name, value)` for parameters and plain values.  Where nothing else takes part - Module's own
     __setattr__, no registration hooks, a name that the module does not hold yet - this is what it comes to without
-    its look-ups (22 -> 15 us on the host per layer, of which loading has hundreds)."""
+    its look-ups (22 -> 15 us on the host per layer)."""
     cls, own, params, buffers, modules = type(layer), layer.__dict__, layer._parameters, layer._buffers, layer._modules
     hooks = getattr(torch.nn.modules.module, "_global_parameter_registration_hooks", True)
     by_module = bool(hooks) or cls.__setattr__ is not torch.nn.Module.__setattr__
@@ -263,11 +263,12 @@ class MatGPTQLinearMethod(LinearMethodBase):
             self.n_out_features, self.n_in_features, bitwidth,
             self.config.group_size, self.config.flag)
 
-    def _pack_all(self, layer: torch.nn.Module) -> List[torch.Tensor]:
+    def _pack_all(self, layer: torch.nn.Module, qweight: torch.Tensor, scales: torch.Tensor,
+                  zeros: Optional[torch.Tensor]) -> List[torch.Tensor]:
         """Packed codes (or resident planes), scales and, if the layer has them, zeros in the kernels' order."""
         ops, config = torch.ops.matgptq_cuda, self.config
-        qweight, scales, zeros = layer.qweight.data, layer.scales.data.contiguous(), getattr(layer, "zeros", None)
-        zeros = None if zeros is None else zeros.data.to(scales.dtype).contiguous()
+        scales = scales.contiguous()
+        zeros = None if zeros is None else zeros.to(scales.dtype).contiguous()
         planes = config.resident_master_planes
         if (qweight.is_cuda and config.master_bitwidth == 8 and scales.device == qweight.device
                 and tuple(qweight.shape) == (self.n_out_features, self.n_in_features)
@@ -284,28 +285,29 @@ class MatGPTQLinearMethod(LinearMethodBase):
 
     def process_weights_after_loading(self, layer: torch.nn.Module) -> None:
         # (a loader may have left any of them as a parameter, a buffer or a plain tensor)
-        with torch.no_grad():
-            qweight = layer.qweight.data
-            packed = [Parameter(t, requires_grad=False) for t in self._pack_all(layer)]
-            planes = self.config.resident_master_planes
-            put = _setter(layer)
-            put("matgptq_planes", packed[0] if planes else None)
-            put("matgptq_weights", None if planes else packed[0])
-            put("matgptq_bitwidth", self.bitwidth)
-            put("matgptq_scales", packed[1])
-            put("matgptq_zeros", packed[2] if len(packed) > 2 else None)
-            perm = getattr(layer, "perm", None)
-            # act-order: the codes are stored in permuted column order and the input features
-            # are gathered with the permutation (src/quant_utils_matgpqt.py:218-220)
-            put("matgptq_perm", None if perm is None else Parameter(
-                perm.data.to(device=packed[1].device, dtype=torch.int64).reshape(-1), requires_grad=False))
-            if self.config.keep_master_codes and not planes:
-                # The reference deletes the master codes here (inference_lib/vllm_matgptq.py:177-178);
-                # kept, a layer can be re-sliced to another bitwidth without the checkpoint.
-                put("matgptq_master", Parameter(qweight.to(packed[1].device), requires_grad=False))
-            for name, given in (("qweight", True), ("scales", True), ("zeros", len(packed) > 2), ("perm", perm is not None)):
-                if given:
-                    delattr(layer, name)
+        qweight, zeros, perm = layer.qweight.data, getattr(layer, "zeros", None), getattr(layer, "perm", None)
+        packed = [Parameter(t, requires_grad=False)
+                  for t in self._pack_all(layer, qweight, layer.scales.data, None if zeros is None else zeros.data)]
+        planes = self.config.resident_master_planes
+        put = _setter(layer)
+        put("matgptq_planes", packed[0] if planes else None)
+        put("matgptq_weights", None if planes else packed[0])
+        put("matgptq_bitwidth", self.bitwidth)
+        put("matgptq_scales", packed[1])
+        put("matgptq_zeros", None if zeros is None else packed[2])
+        # act-order: the codes are stored in permuted column order and the input features
+        # are gathered with the permutation (src/quant_utils_matgpqt.py:218-220)
+        put("matgptq_perm", None if perm is None else Parameter(
+            perm.data.to(device=packed[1].device, dtype=torch.int64).reshape(-1), requires_grad=False))
+        if self.config.keep_master_codes and not planes:
+            # The reference deletes the master codes here (inference_lib/vllm_matgptq.py:177-178);
+            # kept, a layer can be re-sliced to another bitwidth without the checkpoint.
+            put("matgptq_master", Parameter(qweight.to(packed[1].device), requires_grad=False))
+        del layer.qweight, layer.scales
+        if zeros is not None:
+            del layer.zeros
+        if perm is not None:
+            del layer.perm
 
     def set_bitwidth(self, layer: torch.nn.Module, bitwidth: int) -> None:
         """Moves a loaded layer to `bitwidth`.  With `resident_master_planes` nothing is touched but
