@@ -17,60 +17,68 @@ struct PackAux {
   int G, groups_per_tile;       // groups_per_tile 0: one group per row
 };
 
-// tiles of K a workgroup of the packing kernel takes
+// tiles a workgroup of the packing kernel takes
 constexpr int kPackTiles = 8;
+
+// A workgroup's tiles: 2^tx_log neighbours along K (a power of two that divides the tiles of a row block) by the rest
+// of the workgroup's tiles in row blocks, so that no lane is idle whatever K is.  us, eight (four) neighbours of one row block /
+// this: packing 28672 x 1152 at 4 / 8 bits 13.5 / 10.5 and 17.1 / 13.7, 262144 x 128 at 2 bits 13.6 / 9.5; planes to codes
+// 262144 x 640 at 8 bits 116 / 81.
+struct TilePos {
+  int kb, rb;
+};
+__device__ __forceinline__ TilePos tile_of(int slot, int rb0, int tx_log) {
+  return {((int)blockIdx.x << tx_log) + (slot & ((1 << tx_log) - 1)), rb0 + (slot >> tx_log)};
+}
 
 // Codes [N, K] -> packed tiles (PLANES false: the b-bit layout, SLICE: from 8-bit master codes; PLANES
 // true: the master-resident planes).  A thread packs two neighbouring lane slots (k-quarters 2p and 2p + 1
-// of a row: 16 bytes of each octet), half a wave a tile; a workgroup takes eight neighbouring tiles of a
-// row block and, when asked, reorders the scales and zeros of their groups, so that loading a layer is
-// one launch.
+// of a row: 16 bytes of each octet), half a wave a tile and, when asked, the scales and zeros of the tile's
+// groups, so that loading a layer is one launch.
 // Bound: HBM (1 byte per code in, b/8 out).  The codes are sliced and packed four at a time on the
 // bytes of a word (swar_codec.h): about 70 vector instructions per slot where one code after another
-// took some 300 and the kernel was bound by them, and a tile is found without a 64-bit division
+// took some 300 and the kernel was bound by them, and a tile is found without a division
 // (28672 x 4096 from master codes, us before / now: 2 bits 42 / 26, 3 bits 46 / 27, 4 bits 38 / 29, 6 bits
 // 47 / 35, 8 bits 36 / 37, planes 61 / 37; a copy moves the 4-bit case's 176 MB in 36).
 template <int BITS, bool SLICE, bool PLANES>
 __global__ void __launch_bounds__(256)
-pack_kernel(const uint8_t* __restrict__ codes, uint32_t* __restrict__ out, int k_tiles, int64_t K, int row_blocks,
+pack_kernel(const uint8_t* __restrict__ codes, uint32_t* __restrict__ out, int k_tiles, int64_t K, int row_blocks, int tx_log,
             PackAux aux) {
   const int r = threadIdx.x & 15, p = (threadIdx.x >> 4) & 1;
-  const int kb = blockIdx.x * kPackTiles + (threadIdx.x >> 5);
-  for (int rb = blockIdx.y; rb < row_blocks; rb += gridDim.y) {
-    if (kb < k_tiles) {
-      const uint8_t* slot = codes + ((int64_t)rb * 16 + r) * K + kb * 128 + p * 16;
-      uint4 v[4];
+  const int ty = kPackTiles >> tx_log;
+  for (int rb0 = blockIdx.y * ty; rb0 < row_blocks; rb0 += gridDim.y * ty) {
+    const auto [kb, rb] = tile_of(threadIdx.x >> 5, rb0, tx_log);
+    if (rb >= row_blocks) continue;
+    const uint8_t* slot = codes + ((int64_t)rb * 16 + r) * K + kb * 128 + p * 16;
+    uint4 v[4];
 #pragma unroll
-      for (int j = 0; j < 4; j++) v[j] = *reinterpret_cast<const uint4*>(slot + j * 32);
-      const int64_t tile = (int64_t)rb * k_tiles + kb;
+    for (int j = 0; j < 4; j++) v[j] = *reinterpret_cast<const uint4*>(slot + j * 32);
+    const int64_t tile = (int64_t)rb * k_tiles + kb;
 #pragma unroll
-      for (int h = 0; h < 2; h++) {
-        const int lane = (2 * p + h) * 16 + r;
-        uint2 c[4];
+    for (int h = 0; h < 2; h++) {
+      const int lane = (2 * p + h) * 16 + r;
+      uint2 c[4];
 #pragma unroll
-        for (int j = 0; j < 4; j++) c[j] = h == 0 ? make_uint2(v[j].x, v[j].y) : make_uint2(v[j].z, v[j].w);
-        if constexpr (PLANES) {
-          uint32_t w[8];
-          pack_slot_planes(c, w);
-          uint32_t* t = out + tile * kMasterTileWords;
-          *reinterpret_cast<uint3*>(t + lane * 3) = make_uint3(w[0], w[1], w[2]);
-          t[192 + lane] = w[3];
-          t[256 + lane] = w[4];
-          *reinterpret_cast<uint3*>(t + 320 + lane * 3) = make_uint3(w[5], w[6], w[7]);
-        } else {
-          uint32_t w[BITS];
-          pack_slot<BITS, SLICE>(c, w);
-          store_tile_words<BITS>(out + tile * tile_words(BITS), lane, w);
-        }
+      for (int j = 0; j < 4; j++) c[j] = h == 0 ? make_uint2(v[j].x, v[j].y) : make_uint2(v[j].z, v[j].w);
+      if constexpr (PLANES) {
+        uint32_t w[8];
+        pack_slot_planes(c, w);
+        uint32_t* t = out + tile * kMasterTileWords;
+        *reinterpret_cast<uint3*>(t + lane * 3) = make_uint3(w[0], w[1], w[2]);
+        t[192 + lane] = w[3];
+        t[256 + lane] = w[4];
+        *reinterpret_cast<uint3*>(t + 320 + lane * 3) = make_uint3(w[5], w[6], w[7]);
+      } else {
+        uint32_t w[BITS];
+        pack_slot<BITS, SLICE>(c, w);
+        store_tile_words<BITS>(out + tile * tile_words(BITS), lane, w);
       }
     }
     if (aux.s_out != nullptr) {
-      // the groups of this workgroup's tiles; the last workgroup of a row block also takes those of a
-      // tail of 64 columns
-      const int per = kPackTiles * aux.groups_per_tile;
-      const int g0 = blockIdx.x * per;
-      const int g1 = per == 0 ? (blockIdx.x == 0 ? 1 : 0) : blockIdx.x + 1 == gridDim.x ? aux.G : g0 + per;
-      for (int i = threadIdx.x; i < (g1 - g0) * 16; i += 256) {
+      // the groups of this tile; the last tile of a row block also takes those of a tail of 64 columns
+      const int g0 = kb * aux.groups_per_tile;
+      const int g1 = aux.groups_per_tile == 0 ? (kb == 0 ? 1 : 0) : kb + 1 == k_tiles ? aux.G : g0 + aux.groups_per_tile;
+      for (int i = threadIdx.x & 31; i < (g1 - g0) * 16; i += 32) {
         const int g = g0 + (i >> 4);
         const int64_t from = ((int64_t)rb * 16 + (i & 15)) * aux.G + g, to = ((int64_t)rb * aux.G + g) * 16 + (i & 15);
         aux.s_out[to] = aux.s_in[from];
@@ -190,13 +198,17 @@ dequant_kernel(const uint32_t* __restrict__ packed, const uint16_t* __restrict__
 // Bound: HBM.  A nibble word of the planes is a nibble word of the packed layout, so nothing is unpacked
 // to single codes on the way (28672 x 4096, us before / now: 2 bits 23 / 13, 3 bits 34 / 18, 4 bits 26 / 21,
 // 6 bits 50 / 34, 8 bits 42 / 35).
+constexpr int kSliceTiles = 4;  // tiles of a workgroup, one a wave
 template <int BITS, bool SLICED_PACKED>
 __global__ void __launch_bounds__(256)
-master_slice_kernel(const uint32_t* __restrict__ planes, void* __restrict__ out, int k_tiles, int64_t K, int row_blocks) {
+master_slice_kernel(const uint32_t* __restrict__ planes, void* __restrict__ out, int k_tiles, int64_t K, int row_blocks,
+                    int tx_log) {
   const int lane = threadIdx.x & 63;
-  const int kb = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  if (kb >= k_tiles) return;
-  for (int rb = blockIdx.y; rb < row_blocks; rb += gridDim.y) {
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int ty = kSliceTiles >> tx_log;
+  for (int rb0 = blockIdx.y * ty; rb0 < row_blocks; rb0 += gridDim.y * ty) {
+    const auto [kb, rb] = tile_of(wave, rb0, tx_log);
+    if (rb >= row_blocks) continue;
     const int64_t tile = (int64_t)rb * k_tiles + kb;
     const uint32_t* t = planes + tile * kMasterTileWords;
     uint32_t w[8] = {};
@@ -394,9 +406,12 @@ hipError_t launch_tail_gemm(int bits, bool bf16, const GemmArgs& a, int group_si
   return hipGetLastError();
 }
 
-// grid of the kernels in which a workgroup takes `per` neighbouring tiles of a row block
-static dim3 tile_grid(int k_tiles, int64_t row_blocks, int per) {
-  return dim3((unsigned)((k_tiles + per - 1) / per), (unsigned)(row_blocks < 65535 ? row_blocks : 65535));
+// grid of the kernels in which a workgroup takes `per` (a power of two) tiles; tx_log: see tile_of
+static dim3 tile_grid(int k_tiles, int64_t row_blocks, int per, int* tx_log) {
+  int tx = 1;
+  for (*tx_log = 0; tx < per && k_tiles % (2 * tx) == 0; tx *= 2) ++*tx_log;
+  const int64_t rows = (row_blocks * tx + per - 1) / per;
+  return dim3((unsigned)(k_tiles / tx), (unsigned)(rows < 65535 ? rows : 65535));
 }
 
 // source: 0 = codes already sliced, 1 = 8-bit master codes to be sliced, 2 = master codes to resident
@@ -408,15 +423,18 @@ hipError_t launch_pack_layer(const uint8_t* codes, int64_t N, int64_t K, int bit
   const int64_t row_blocks = N / 16;
   const PackAux aux{s_in, z_in, s_out, z_out, group_size == -1 ? 1 : (int)(K / group_size),
                     group_size == -1 ? 0 : 128 / group_size};
-  const dim3 grid = tile_grid(k_tiles, row_blocks, kPackTiles), block(256);
+  int tx_log;
+  const dim3 grid = tile_grid(k_tiles, row_blocks, kPackTiles, &tx_log), block(256);
 #define MATGPTQ_PACK(B)                                                                                              \
   case B:                                                                                                            \
     if (source != 0) hipLaunchKernelGGL((pack_kernel<B, true, false>), grid, block, 0, s, codes, out, k_tiles, K,     \
-                                        (int)row_blocks, aux);                                                       \
-    else hipLaunchKernelGGL((pack_kernel<B, false, false>), grid, block, 0, s, codes, out, k_tiles, K, (int)row_blocks, aux); \
+                                        (int)row_blocks, tx_log, aux);                                               \
+    else hipLaunchKernelGGL((pack_kernel<B, false, false>), grid, block, 0, s, codes, out, k_tiles, K,               \
+                            (int)row_blocks, tx_log, aux);                                                           \
     break;
   if (source == 2) {
-    hipLaunchKernelGGL((pack_kernel<8, false, true>), grid, block, 0, s, codes, out, k_tiles, K, (int)row_blocks, aux);
+    hipLaunchKernelGGL((pack_kernel<8, false, true>), grid, block, 0, s, codes, out, k_tiles, K, (int)row_blocks, tx_log,
+                       aux);
   } else {
     switch (bits) {
       MATGPTQ_PACK(2)
@@ -424,7 +442,8 @@ hipError_t launch_pack_layer(const uint8_t* codes, int64_t N, int64_t K, int bit
       MATGPTQ_PACK(4)
       MATGPTQ_PACK(6)
       default:
-        hipLaunchKernelGGL((pack_kernel<8, false, false>), grid, block, 0, s, codes, out, k_tiles, K, (int)row_blocks, aux);
+        hipLaunchKernelGGL((pack_kernel<8, false, false>), grid, block, 0, s, codes, out, k_tiles, K, (int)row_blocks, tx_log,
+                           aux);
         break;
     }
     if (K % 128 != 0)
@@ -457,11 +476,12 @@ hipError_t launch_unpack(const uint32_t* packed, int64_t N, int64_t K, int bits,
 hipError_t launch_master_slice(const uint32_t* planes, int64_t N, int64_t K, int bits, bool sliced_packed,
                                void* out, hipStream_t s) {
   const int k_tiles = (int)(K / 128), row_blocks = (int)(N / 16);
-  const dim3 grid = tile_grid(k_tiles, row_blocks, 4), block(256);
+  int tx_log;
+  const dim3 grid = tile_grid(k_tiles, row_blocks, kSliceTiles, &tx_log), block(256);
 #define MATGPTQ_MS(B)                                                                                         \
   case B:                                                                                                     \
-    if (sliced_packed) hipLaunchKernelGGL((master_slice_kernel<B, true>), grid, block, 0, s, planes, out, k_tiles, K, row_blocks); \
-    else hipLaunchKernelGGL((master_slice_kernel<B, false>), grid, block, 0, s, planes, out, k_tiles, K, row_blocks);  \
+    if (sliced_packed) hipLaunchKernelGGL((master_slice_kernel<B, true>), grid, block, 0, s, planes, out, k_tiles, K, row_blocks, tx_log); \
+    else hipLaunchKernelGGL((master_slice_kernel<B, false>), grid, block, 0, s, planes, out, k_tiles, K, row_blocks, tx_log);  \
     break;
   switch (bits) {
     MATGPTQ_MS(2)
@@ -469,8 +489,8 @@ hipError_t launch_master_slice(const uint32_t* planes, int64_t N, int64_t K, int
     MATGPTQ_MS(4)
     MATGPTQ_MS(6)
     default:
-      if (sliced_packed) hipLaunchKernelGGL((master_slice_kernel<8, true>), grid, block, 0, s, planes, out, k_tiles, K, row_blocks);
-      else hipLaunchKernelGGL((master_slice_kernel<8, false>), grid, block, 0, s, planes, out, k_tiles, K, row_blocks);
+      if (sliced_packed) hipLaunchKernelGGL((master_slice_kernel<8, true>), grid, block, 0, s, planes, out, k_tiles, K, row_blocks, tx_log);
+      else hipLaunchKernelGGL((master_slice_kernel<8, false>), grid, block, 0, s, planes, out, k_tiles, K, row_blocks, tx_log);
       break;
   }
 #undef MATGPTQ_MS
