@@ -326,9 +326,12 @@ attention_kernel(const _Float16* __restrict__ qkv, _Float16* k_cache, _Float16* 
 // of a key/value head per workgroup: 32 / 8 heads, 513 rows of 584 6.5 / 6.7 / 8.0, 1001 of 1024 7.5 / 7.5 / 8.8, 4097 of 4168 16.4 /
 // 16.0 / 17.0; 64 / 8 heads, 513 of 584 7.3 / 7.6 / 10.6, 4097 of 4168 22.1 / 20.6 / 30.7; four rows, 32 / 8 heads, 513 of 584
 // 7.3 / 8.1 / 8.9; 16 rows, 64 / 8 heads, 900 of 1000 30.8 / 29.5 / 33.6.  (One workgroup per head, unsplit: 513 of 584 rows 8.3.)
+// Several rows, 64 / 8 heads, 1 / 2 / 4 / 8 heads per workgroup: 5 rows, 2048 of 2048 24.7 / 23.9 / 24.0 / 25.9, position 64 6.9 / 7.3 / 10.8 /
+// 14.5; 16 rows, 8192 of 8192 219 / 203 / 195 / 219, position 64 31.5 / 19.2 / 15.6 / 19.2: two is within 5 % of the best of a full cache
+// and in the middle of an empty one.
 // Every workgroup requests its rows before it knows pos[m], so a long cache is read whatever the position; short contexts in
 // one are still ahead of the unsplit form, one row, split / unsplit: 32 / 8 heads, 8192 rows, position 5 5.8 / 7.0, 64 6.0 / 7.3,
-// 512 6.9 / 8.3, 2000 10.1 / 17.6; 64 / 8 heads, 2048 rows, position 512 8.1 / 8.5 (the closest of 120 shapes), 8192 rows, 64 6.1 /
+// 512 6.9 / 8.3, 2000 10.1 / 17.6; 64 / 8 heads, 4096 rows, position 512 8.2 / 8.5 (the closest of 135 shapes), 8192 rows, 64 6.1 /
 // 8.1.  Errors against 64 bits are the same in both (2.0e-4, the rounding of the result).
 // ws: M x heads x splits x 130 floats.
 constexpr int kOneHeadContext = 1024;
