@@ -142,13 +142,15 @@ std::vector<Tensor> pack_matgptq_layer(const Tensor& qweights, const Tensor& sca
                                        int64_t bitwidth, int64_t group_size, int64_t source) {
   TORCH_CHECK(qweights.is_cuda(), "pack_matgptq_layer: qweights must be on the GPU");
   TORCH_CHECK(qweights.dtype() == torch::kUInt8, "qweights must be uint8");
-  TORCH_CHECK(qweights.dim() == 2 && qweights.is_contiguous(), "qweights must be contiguous and 2D (n_out_features, n_in_features)");
+  TORCH_CHECK(qweights.is_contiguous(), "qweights must be contiguous");
+  TORCH_CHECK(qweights.dim() == 2, "qweights must be 2D (n_out_features, n_in_features)");
   const int64_t n = qweights.size(0), k = qweights.size(1);
   check_bits_group(bitwidth, group_size, k);
   check_tiling(n, k, source == 2);
   const int64_t groups = group_size == -1 ? 1 : k / group_size;
   auto check_per_group = [&](const Tensor& t) {
-    TORCH_CHECK(t.device() == qweights.device() && t.is_contiguous(), "scales and zeros must be contiguous and on the GPU of qweights");
+    TORCH_CHECK(t.device() == qweights.device(), "scales and zeros must be on the GPU of qweights");
+    TORCH_CHECK(t.is_contiguous(), "scales must be contiguous");
     TORCH_CHECK(t.dtype() == torch::kFloat16 || t.dtype() == torch::kBFloat16, "scales must be float16 or bfloat16");
     TORCH_CHECK(t.dim() == 2 && t.size(0) == n && t.size(1) == groups,
                 "scales must have shape (n_out_features, n_in_features / group_size)");

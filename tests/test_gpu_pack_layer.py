@@ -58,3 +58,17 @@ def test_slice_at_every_alignment(count, offset, b):
         got = out.cpu().numpy()
         assert np.array_equal(got[out_offset:out_offset + count], o.slice_codes(q, b))
         assert (got[:out_offset] == 255).all() and (got[out_offset + count:] == 255).all()
+
+
+def test_layer_on_the_gpu_is_refused_in_the_words_of_the_separate_packers():
+    from matgptq_cuda.matgptq_linear import MatGPTQLinear
+
+    q = torch.zeros(32, 256, dtype=torch.uint8, device="cuda")
+    s = torch.ones(32, 2, dtype=torch.float16, device="cuda")
+    for codes, scales, message in ((torch.zeros(256, 32, dtype=torch.uint8, device="cuda").t(), s, "qweights must be contiguous"),
+                                   (q.int(), s, "qweights must be uint8"),
+                                   (q, torch.ones(2, 32, dtype=torch.float16, device="cuda").t(), "scales must be contiguous"),
+                                   (q, s.float(), "scales must be float16 or bfloat16"),
+                                   (q, s[:16].contiguous(), "scales must have shape")):
+        with pytest.raises(RuntimeError, match=message):
+            MatGPTQLinear(codes, scales, 4, 128)
