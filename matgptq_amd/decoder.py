@@ -98,6 +98,12 @@ class DecoderConfig:
                 "down": (self.hidden, self.ffn)}
 
 
+def _addressable(t: torch.Tensor) -> torch.Tensor:
+    """Contiguous on 16 bytes, as the fused operators of a prompt read; a linear may return a view of another buffer."""
+    t = t.contiguous()
+    return t if t.data_ptr() % 16 == 0 else t.clone()
+
+
 class Block(torch.nn.Module):
     """One decoder block.  The linears may be any module mapping `[M, K] -> [M, N]`."""
 
@@ -124,7 +130,7 @@ class Block(torch.nn.Module):
         qkv = self.qkv(x)
         if fused:
             qg = torch.empty(cfg.heads, m, d, dtype=h.dtype, device=h.device)
-            _glue.rope_prompt(qkv.contiguous(), cos, sin, pos, qg, k_cache, v_cache, cfg.heads, cfg.kv_heads)
+            _glue.rope_prompt(_addressable(qkv), cos, sin, pos, qg, k_cache, v_cache, cfg.heads, cfg.kv_heads)
             qg = qg.view(cfg.kv_heads, rep * m, d)
         else:
             qkv = qkv.view(m, cfg.heads + 2 * cfg.kv_heads, d)
@@ -147,7 +153,7 @@ class Block(torch.nn.Module):
         gu = self.gate_up(x)
         if fused:
             act = torch.empty(m, cfg.ffn, dtype=h.dtype, device=h.device)
-            _glue.silu_mul(gu.contiguous(), act, prompt=True)
+            _glue.silu_mul(_addressable(gu), act, prompt=True)
         else:
             act = torch.nn.functional.silu(gu[:, :cfg.ffn]) * gu[:, cfg.ffn:]
         return h + self.down(act)

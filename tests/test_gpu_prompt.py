@@ -74,3 +74,31 @@ def test_fused_prompt_equals_prompt_of_torch_operators(heads, kv, rows, start, c
     dec.fused = False
     b = dec(tokens, pos, cache_b)
     assert torch.equal(a, b) and torch.equal(_bits(cache_a), _bits(cache_b))
+
+
+def test_fused_prompt_takes_linears_that_return_views():
+    # a linear may be any module: one that hands out part of a larger buffer, off 16 bytes or with longer rows
+    from matgptq_amd import decoder as D
+
+    class Part(torch.nn.Module):
+        def __init__(self, linear, offset, pad):
+            super().__init__()
+            self.linear, self.offset, self.pad = linear, offset, pad
+
+        def forward(self, x):
+            y = self.linear(x)
+            buffer = torch.zeros(self.offset + y.shape[0] * (y.shape[1] + self.pad), dtype=y.dtype, device=y.device)
+            part = buffer[self.offset:].view(y.shape[0], -1)[:, :y.shape[1]]
+            return part.copy_(y)
+
+    cfg = D.DecoderConfig(hidden=512, ffn=768, layers=2, heads=4, kv_heads=2, vocab=512)
+    dec = D.random_mixnmatch_decoder(cfg, 80, seed=3)[0]
+    for block, (offset, pad) in zip(dec.blocks, ((4, 0), (8, 24))):
+        block.qkv, block.gate_up = Part(block.qkv, offset, pad), Part(block.gate_up, offset, pad)
+    tokens, pos = torch.randint(0, cfg.vocab, (33,), device=DEV, generator=_gen(4)), torch.arange(33, device=DEV)
+    caches = [dec.new_cache() for _ in range(2)]
+    assert dec.fused_prompt_applies(pos, caches[0])
+    a = dec(tokens, pos, caches[0])
+    dec.fused = False
+    b = dec(tokens, pos, caches[1])
+    assert torch.equal(a, b) and torch.equal(_bits(caches[0]), _bits(caches[1]))
