@@ -215,12 +215,16 @@ int matgptq_gemm_master_static(int bitwidth, int group_size, int64_t N, int64_t 
                                const void *planes_dev, const void *scales_dev, const void *zeros_dev,
                                const void *x_dev, void *y_dev, void *stream, uint32_t flags);
 
-/* Human-readable name of the kernel variant matgptq_gemm would launch. */
+/* Human-readable name of the kernel variant matgptq_gemm would launch; where matgptq_few_rows() is not 0 that kernel runs
+ * instead, and the name is the one of the forced variant next to it. */
 int matgptq_describe_plan(int bitwidth, int group_size, int64_t N, int64_t K, int64_t M,
                           int has_zeros, uint32_t flags, char *buf, size_t buf_len);
 /* Activation buffers (1 or 2) of the mid-batch kernel that matgptq_gemm would launch; 0 where it launches another one,
  * negative on an error. */
 int matgptq_midbatch_buffers(int bitwidth, int group_size, int64_t N, int64_t K, int64_t M, int has_zeros, uint32_t flags);
+/* Row blocks of 16 weight rows per workgroup (1, 2 or 4) of the few-rows kernel (up to 16 batch rows) where matgptq_gemm, or
+ * with master != 0 matgptq_gemm_master, launches it; 0 where it launches another one, negative on an error. */
+int matgptq_few_rows(int bitwidth, int group_size, int64_t N, int64_t K, int64_t M, uint32_t flags, int master);
 
 #ifdef __cplusplus
 }

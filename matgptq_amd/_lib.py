@@ -24,7 +24,7 @@ EXPORTS = (
     "matgptq_master_words", "matgptq_pack_master_host", "matgptq_pack_master_device",
     "matgptq_unpack_master_host", "matgptq_unpack_master_device",
     "matgptq_gemm_master_workspace_bytes", "matgptq_gemm_master", "matgptq_gemm_master_static",
-    "matgptq_probe_read", "matgptq_pack_layer_device", "matgptq_midbatch_buffers",
+    "matgptq_probe_read", "matgptq_pack_layer_device", "matgptq_midbatch_buffers", "matgptq_few_rows",
 )
 
 _lib = None
@@ -92,6 +92,8 @@ def load() -> ctypes.CDLL:
     L.matgptq_pack_layer_device.restype = ci
     L.matgptq_midbatch_buffers.argtypes = [ci, ci, i64, i64, i64, ci, u32]
     L.matgptq_midbatch_buffers.restype = ci
+    L.matgptq_few_rows.argtypes = [ci, ci, i64, i64, i64, u32, ci]
+    L.matgptq_few_rows.restype = ci
     L.matgptq_probe_read.argtypes = [vp, ctypes.c_size_t, vp]
     L.matgptq_probe_read.restype = ci
     _lib = L

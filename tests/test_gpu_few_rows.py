@@ -1,0 +1,119 @@
+"""The few-rows kernel (fewrows_gfx950.hip): one to sixteen batch rows, at the edges of its walks (waves without a tile, one,
+two and three tiles per wave, odd and even), of its row blocks (ragged for two and four per workgroup) and of its batches, on
+pre-sliced codes and on planes."""
+import numpy as np
+import pytest
+import torch
+
+from matgptq_amd import _lib
+from oracle import matgptq_oracle as o
+from tests import _gpu_util as G
+
+pytestmark = pytest.mark.gpu
+
+# (N, K, M, row blocks per workgroup of 4-bit codes, of 4-bit planes)
+CASES = [(16, 128, 1, 1, 1), (48, 1024, 2, 1, 1), (304, 1152, 2, 1, 1), (48, 8192, 4, 1, 1), (5136, 384, 3, 2, 2), (32, 2048, 5, 1, 1),
+         (5136, 1152, 8, 2, 2), (8208, 2944, 7, 2, 2), (10256, 3072, 8, 4, 4), (80, 4224, 9, 1, 1), (5136, 896, 16, 2, 2),
+         (10256, 1024, 13, 4, 4), (10288, 2176, 16, 4, 4)]
+FORMATS = [(2, 128, False), (3, 128, False), (4, 128, False), (6, 128, False), (8, 128, False), (2, -1, True), (3, -1, True),
+           (4, 128, True), (6, 128, True), (8, -1, True), (8, 128, True), (4, -1, False)]
+
+
+def layer(bits, group, bf16, zeros, n, k, seed):
+    dt = torch.bfloat16 if bf16 else torch.float16
+    q, s, z = o.make_layer(n, k, group, seed=seed, symmetric=not zeros)
+    st, zt = torch.from_numpy(s).to(dt), torch.from_numpy(z).to(dt)
+    reorder = lambda t: G.reorder_device(t.view(torch.float16).numpy(), n, k, group)  # (moves 16-bit values, whatever they are)
+    return q, st, zt, reorder(st), reorder(zt) if zeros else None
+
+
+def exact_weights(q, s, z, bits, group):
+    """scale * (code - zero) in 64 bits: the kernel multiplies codes as they are and rounds no weight."""
+    n, k = q.shape
+    spread = lambda t: np.repeat(t.double().numpy(), k if group == -1 else group, axis=1)
+    return spread(s) * ((o.slice_codes(q, bits).astype(np.float64) * (1 << (8 - bits))) - spread(z))
+
+
+def run(bits, group, n, k, x, packed, scales, zeros, flags, planes):
+    y = torch.full((x.shape[0], n), float("nan"), dtype=x.dtype, device=G.DEV)
+    z = zeros.data_ptr() if zeros is not None else None
+    if planes:
+        _lib.check(G.lib().matgptq_gemm_master(bits, group, n, k, x.shape[0], packed.data_ptr(), scales.data_ptr(), z, x.data_ptr(),
+                                               y.data_ptr(), None, 0, G.stream(), flags))
+    else:
+        _lib.check(G.lib().matgptq_gemm(bits, group, n, k, x.shape[0], packed.data_ptr(), scales.data_ptr(), z, x.data_ptr(),
+                                        y.data_ptr(), G.stream(), flags))
+    return y
+
+
+def packed_of(q, bits, planes):
+    if not planes:
+        return G.pack_device(q, bits, True)
+    n, k = q.shape
+    out = torch.empty(G.lib().matgptq_master_words(n, k), dtype=torch.int32, device=G.DEV)
+    codes = G.to_dev(q)
+    _lib.check(G.lib().matgptq_pack_master_device(codes.data_ptr(), n, k, out.data_ptr(), G.stream()))
+    return out
+
+
+@pytest.mark.parametrize("planes", (False, True))
+@pytest.mark.parametrize("bits,group,bf16", FORMATS)
+@pytest.mark.parametrize("n,k,m,rows,rows_planes", CASES)
+def test_few_rows(n, k, m, rows, rows_planes, bits, group, bf16, planes):
+    zeros = (n // 16 + bits) % 2 == 0
+    flags = 3 if bf16 else 1
+    most = 4 if bits <= (4 if planes else 6) else 2
+    elsewhere = m <= 4 and not planes and not bf16 and group == 128  # (with the fused prologues)
+    assert G.lib().matgptq_few_rows(bits, group, n, k, m, flags, int(planes)) == (0 if elsewhere else min(rows_planes if planes else rows, most))
+    q, st, zt, sd, zd = layer(bits, group, bf16, zeros, n, k, seed=n + k + bits)
+    x = torch.from_numpy(o.make_activations(m, k, seed=m, outlier_frac=0.01)).to(st.dtype)
+    y = run(bits, group, n, k, x.cuda(), packed_of(q, bits, planes), sd, zd, flags, planes).double().cpu().numpy()
+    xd = x.double().numpy()
+    ref = xd @ exact_weights(q, st, zt, bits, group).T
+    # one rounding of the result, and sums in fp32 of products of codes with up to 1024 (bf16: 128) added to them: their
+    # rounding errors stay below 2^-21 of the sum of the magnitudes
+    scale = np.repeat(st.double().numpy(), k if group == -1 else group, axis=1) * (1 << (8 - bits))
+    reach = np.abs(xd) @ (scale * ((128 if bf16 else 1024) + 2 * (1 << bits))).T
+    assert np.all(np.abs(y - ref) <= 2.0 ** (-8 if bf16 else -11) * np.abs(ref) + 2.0 ** -21 * reach + 2.0 ** -24)
+
+
+@pytest.mark.parametrize("planes", (False, True))
+@pytest.mark.parametrize("bits,group,bf16,zeros", [(4, 128, False, True), (3, -1, False, True), (8, 128, True, False), (6, -1, True, True)])
+def test_infinities_nan_and_the_largest_numbers(bits, group, bf16, zeros, planes):
+    # one wave's columns hold them: rows with one are what dequantised weights give, the others stay finite
+    n, k, m = 80, 2176, 11
+    q, st, zt, sd, zd = layer(bits, group, bf16, zeros, n, k, seed=bits)
+    x = torch.from_numpy(o.make_activations(m, k, seed=5)).to(st.dtype)
+    x[1, 300], x[4, 2100], x[5, 7], x[5, 1200] = float("inf"), float("-inf"), float("inf"), float("nan")
+    x[7, 640] = 3e38 if bf16 else 65504.0
+    w = (o.dequantize_bf16(q, st.float().numpy(), zt.float().numpy(), bits, group) if bf16
+         else o.dequantize(q, st.numpy(), zt.numpy(), bits, group)).astype(np.float64)
+    with np.errstate(invalid="ignore", over="ignore"):
+        ref = x.double().numpy() @ w.T
+        ref = torch.from_numpy(ref).to(st.dtype).double().numpy()
+    y = run(bits, group, n, k, x.cuda(), packed_of(q, bits, planes), sd, zd, 3 if bf16 else 1, planes).double().cpu().numpy()
+    assert G.lib().matgptq_few_rows(bits, group, n, k, m, 3 if bf16 else 1, int(planes)) == 1
+    for row, col in ((1, 300), (4, 2100), (5, 7)):
+        # (a weight the oracle rounds to nothing may be a rounding of scale * (zero - 128) here, and the product infinite)
+        some = w[:, col] != 0
+        assert np.count_nonzero(some) > 60 and np.array_equal(y[row][some], ref[row][some], equal_nan=True)
+    fine = [i for i in range(m) if i not in (1, 4, 5)]
+    assert np.all(np.isfinite(y[fine]) == np.isfinite(ref[fine]))
+    for row in fine:
+        ok = np.isfinite(ref[row])
+        assert np.max(np.abs(y[row][ok] - ref[row][ok]), initial=0) <= (1e-2 if bf16 else 2e-3) * np.max(np.abs(ref[row][ok]), initial=1e-30)
+
+
+def test_exact_on_integers():
+    # scales 0 and 1, integer activations: every sum is a whole number below 2^24
+    rng = np.random.default_rng(3)
+    n, k = 96, 4224
+    for bits in (2, 3, 4, 6, 8):
+        codes = rng.integers(0, 1 << bits, (n, k), dtype=np.uint8)
+        scales = np.round(rng.random((n, k // 128))).astype(np.float16)
+        pk, sd = G.pack_device(codes, bits, from_master=False), G.reorder_device(scales, n, k, 128)
+        w = o.dequantize_kernel_form(codes, scales, bits, 128)
+        for m in (5, 8, 16):
+            x = np.round(rng.standard_normal((m, k))).astype(np.float16)
+            y = G.gemm(bits, 128, n, k, G.to_dev(x), pk, sd, None).cpu().numpy()
+            assert np.array_equal(y.view(np.uint16), o.linear_f64(x, w).astype(np.float16).view(np.uint16)), (bits, m)

@@ -481,3 +481,24 @@ def test_midbatch_buffers_at_the_edges_of_the_rule():
     assert [buffers(8, g, 32 * 257, 2048, 16, 1, plain | forced(1, 0)) for g in (128, 32)] == [2, 1]
     assert [buffers(6, 128, 64 * 257, 2048, 16, z, plain | forced(2, 0)) for z in (0, 1)] == [2, 1]
     assert buffers(4, 128, 64 * 257, 2048, 16, 1, plain | forced(2, 0)) == 2
+
+
+def test_few_rows_at_the_edges_of_the_rule():
+    few = _lib.load().matgptq_few_rows
+    plain, bf16 = 1, 3
+    assert few(5, 128, 4096, 4096, 8, plain, 0) < 0 and few(4, 128, 4096, 4096, 0, plain, 0) < 0
+    assert few(4, 32, 4096, 4096, 8, plain, 0) == 0 and few(4, 128, 4096, 4096, 17, plain, 0) == 0
+    assert few(4, 128, 4096, 4096, 8, plain | (80 << 8), 0) == 0 and few(4, 128, 4096, 4096, 8, plain | (1 << 16), 0) == 0
+    # up to four rows of fp16 storage at group 128: the gemv kernel, as with a fused prologue
+    assert [few(4, g, 256, 1024, m, plain, 0) for g, m in ((128, 1), (128, 4), (128, 5), (-1, 1))] == [0, 0, 1, 1]
+    # one row: short walks on few row blocks, long ones of planes on many
+    assert [few(4, 128, 16 * n, 128 * k, 1, bf16, 0) for n, k in ((600, 16), (601, 16), (600, 17))] == [1, 0, 0]
+    assert [few(4, 128, 16 * n, 128 * k, 1, plain, 1) for n, k in ((600, 24), (600, 25), (1024, 41), (1025, 41), (1025, 40))] == [1, 0, 0, 1, 0]
+    assert [few(4, 128, 16 * n, 128 * k, 2, bf16, 0) for n, k in ((400, 24), (401, 24), (1024, 8), (1025, 8), (400, 25))] == [1, 0, 1, 0, 0]
+    assert [few(4, 128, 16 * n, 128 * k, 2, plain, 1) for n, k in ((600, 24), (601, 24), (600, 41), (601, 41))] == [1, 0, 0, 1]
+    # three and four rows: everything but long walks on few row blocks
+    assert [few(4, 128, 16 * n, 128 * k, 4, bf16, 0) for n, k in ((256, 64), (256, 65), (257, 65), (319, 65), (320, 65))] == [1, 0, 1, 1, 2]
+    # five and more: everything
+    assert [few(4, -1, 16 * n, 4096, 8, plain, 0) for n in (1, 319, 320, 512, 513, 636, 637)] == [1, 1, 2, 2, 2, 2, 4]
+    assert [few(4, 128, 16 * n, 4096, 9, plain, 0) for n in (318, 319, 636, 637)] == [1, 2, 2, 4]
+    assert [few(b, 128, 65536, 4096, 16, plain, p) for b, p in ((6, 0), (8, 0), (4, 1), (6, 1))] == [4, 2, 4, 2]
