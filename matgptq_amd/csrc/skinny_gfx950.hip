@@ -32,6 +32,8 @@
 //    codes have two register sets that are refilled behind the multiplication.  That pays where a wave alone on its
 //    SIMD waits for its copies, and where several rounds of workgroups keep the copies queued; the rule is in
 //    midbatch_plan.h;
+//  * walks of one tile (BUFS = 0: K up to 1024) have one buffer and one register set, nothing is requested behind the first
+//    tile, and more workgroups share a CU;
 //  * every load is branch-free (tiles beyond K, rows beyond M or N go through a zero-length
 //    buffer descriptor or an out-of-range offset);
 //  * the eight partial sums meet in LDS once, at the end; the threads add them and store four
@@ -69,7 +71,7 @@ skinny_kernel(const GemmArgs a, int n_tiles, int m_tiles) {
   using Fmt = TileFormat<BITS, MASTER>;
   constexpr int GPT = GROUP == 32 ? 4 : 1;
   constexpr int kStage = MB * 16 * 256;  // bytes of one activation buffer
-  constexpr int NS = 2;  // register sets of codes, scales, zeros
+  constexpr int NS = BUFS == 0 ? 1 : 2;  // register sets of codes, scales, zeros
   __shared__ __align__(16) unsigned char smem[skinny_lds_bytes(R, MB)];
   // (an array of its own: the compiler orders LDS copies and reads per variable)
   __shared__ __align__(16) unsigned char smem_odd[BUFS == 2 ? kWaves * kStage : 16];
@@ -223,8 +225,10 @@ skinny_kernel(const GemmArgs a, int n_tiles, int m_tiles) {
     __builtin_amdgcn_sched_barrier(0);
     __builtin_amdgcn_s_waitcnt(15 | (7 << 4) | (0 << 8) | (3 << 14));  // lgkmcnt(0)
     __builtin_amdgcn_sched_barrier(0);
-    dma(stage, kb + kWaves);
-    load_weights(wr[B ^ 1], sr[B ^ 1], zr[B ^ 1], kb + kWaves);
+    if constexpr (BUFS != 0) {
+      dma(stage, kb + kWaves);
+      load_weights(wr[(B ^ 1) % NS], sr[(B ^ 1) % NS], zr[(B ^ 1) % NS], kb + kWaves);
+    }
     if (kb < a.k_tiles) multiply(xf, wr[B], sr[B], zr[B]);
     __builtin_amdgcn_sched_barrier(0);
   };
@@ -232,7 +236,7 @@ skinny_kernel(const GemmArgs a, int n_tiles, int m_tiles) {
   // The same with two buffers: tile t in buffer and register set `btag`.  `moretag`: tile t + 2 is requested;
   // without it (the last two tiles) set 0 leaves set 1's requests in flight, set 1 none.
   constexpr int kTileLoads = 4 * MB + R * ((MASTER ? master_load_count(BITS) : tile_load_count(BITS)) + GPT * (ZP ? 2 : 1));
-  static_assert(BUFS == 1 || kTileLoads < 64, "vmcnt counts up to 63");
+  static_assert(BUFS != 2 || kTileLoads < 64, "vmcnt counts up to 63");
   auto tile_of_two = [&](int t, auto btag, auto moretag) {
     constexpr int B = decltype(btag)::value;
     constexpr bool kMore = decltype(moretag)::value;
@@ -265,7 +269,9 @@ skinny_kernel(const GemmArgs a, int n_tiles, int m_tiles) {
   __builtin_amdgcn_sched_barrier(0);
   dma(stage, wave);
   load_weights(wr[0], sr[0], zr[0], wave);
-  if constexpr (BUFS == 2) {
+  if constexpr (BUFS == 0) {
+    tile(0, Even{});
+  } else if constexpr (BUFS == 2) {
     dma(stage_odd, wave + kWaves);
     load_weights(wr[1], sr[1], zr[1], wave + kWaves);
     int t = 0;
@@ -312,10 +318,14 @@ skinny_kernel(const GemmArgs a, int n_tiles, int m_tiles) {
 }
 
 template <int GROUP, bool ZP, int R, int MB, bool MASTER>
-hipError_t launch_r(const GemmArgs& a, hipStream_t stream) {
+hipError_t launch_r(const GemmArgs& a, bool one, hipStream_t stream) {
   const int n_tiles = (a.row_blocks + R - 1) / R;
   const int m_tiles = (a.M + 16 * MB - 1) / (16 * MB);
   const dim3 grid(n_tiles * m_tiles), block(64 * kWaves);
+  if (one && a.k_tiles <= kWaves) {
+    hipLaunchKernelGGL((skinny_kernel<kBits, GROUP, ZP, R, MB, MASTER, 0>), grid, block, 0, stream, a, n_tiles, m_tiles);
+    return hipGetLastError();
+  }
   constexpr int kTwo = !MASTER && R <= 4 && MB <= 2 ? 2 : 1;
   if (kTwo == 2 && midbatch_two_buffers(kBits, kBf16, GROUP, ZP, R, MB, MASTER, a.k_tiles, a.M, a.row_blocks))
     hipLaunchKernelGGL((skinny_kernel<kBits, GROUP, ZP, R, MB, MASTER, kTwo>), grid, block, 0, stream, a, n_tiles, m_tiles);
@@ -325,30 +335,30 @@ hipError_t launch_r(const GemmArgs& a, hipStream_t stream) {
 }
 
 template <int GROUP, bool ZP, int MB, bool MASTER>
-hipError_t launch_rows(const GemmArgs& a, int r, hipStream_t s) {
+hipError_t launch_rows(const GemmArgs& a, int r, bool one, hipStream_t s) {
   // (four row blocks fit the register budget of two waves per SIMD up to 6 bits and with one
   // scale and zero per tile and row block; group 32 carries four; the master planes are eight
   // words per lane from 6 bits on)
   // (eight row blocks: pre-sliced codes up to 4 bits, 32 batch rows)
   if constexpr (GROUP != 32 && kBits <= 4 && !MASTER && MB == 2) {
-    if (r >= 8) return launch_r<GROUP, ZP, 8, MB, MASTER>(a, s);
+    if (r >= 8) return launch_r<GROUP, ZP, 8, MB, MASTER>(a, one, s);
   }
   if constexpr (GROUP != 32 && kBits <= (MASTER ? 4 : 6)) {
-    if (r >= 4) return launch_r<GROUP, ZP, 4, MB, MASTER>(a, s);
+    if (r >= 4) return launch_r<GROUP, ZP, 4, MB, MASTER>(a, one, s);
   }
-  if (r >= 2) return launch_r<GROUP, ZP, 2, MB, MASTER>(a, s);
-  return launch_r<GROUP, ZP, 1, MB, MASTER>(a, s);
+  if (r >= 2) return launch_r<GROUP, ZP, 2, MB, MASTER>(a, one, s);
+  return launch_r<GROUP, ZP, 1, MB, MASTER>(a, one, s);
 }
 
 template <int GROUP, bool ZP, bool MASTER>
-hipError_t launch_batch(const GemmArgs& a, int r, int mb, hipStream_t s) {
-  if (mb >= 4) return launch_rows<GROUP, ZP, 4, MASTER>(a, r, s);
-  return mb >= 2 ? launch_rows<GROUP, ZP, 2, MASTER>(a, r, s) : launch_rows<GROUP, ZP, 1, MASTER>(a, r, s);
+hipError_t launch_batch(const GemmArgs& a, int r, int mb, bool one, hipStream_t s) {
+  if (mb >= 4) return launch_rows<GROUP, ZP, 4, MASTER>(a, r, one, s);
+  return mb >= 2 ? launch_rows<GROUP, ZP, 2, MASTER>(a, r, one, s) : launch_rows<GROUP, ZP, 1, MASTER>(a, r, one, s);
 }
 
 template <int GROUP, bool ZP>
-hipError_t launch_storage(const GemmArgs& a, int r, int mb, bool master, hipStream_t s) {
-  return master ? launch_batch<GROUP, ZP, true>(a, r, mb, s) : launch_batch<GROUP, ZP, false>(a, r, mb, s);
+hipError_t launch_storage(const GemmArgs& a, int r, int mb, bool one, bool master, hipStream_t s) {
+  return master ? launch_batch<GROUP, ZP, true>(a, r, mb, one, s) : launch_batch<GROUP, ZP, false>(a, r, mb, one, s);
 }
 
 }  // namespace
@@ -361,14 +371,15 @@ hipError_t launch_storage(const GemmArgs& a, int r, int mb, bool master, hipStre
 #else
 #define MATGPTQ_LAUNCH_NAME MATGPTQ_CAT(launch_skinny_b, MATGPTQ_BITS)
 #endif
-// master: `a.packed` holds master-resident bit planes
-hipError_t MATGPTQ_LAUNCH_NAME(const GemmArgs& a, int group_size, int r, int mb, bool master, hipStream_t stream) {
+// one: walks of one tile take the kernel with one buffer and one register set; master: `a.packed` holds master-resident
+// bit planes
+hipError_t MATGPTQ_LAUNCH_NAME(const GemmArgs& a, int group_size, int r, int mb, bool one, bool master, hipStream_t stream) {
   const bool zp = a.zeros != nullptr;
   if (group_size == 128)
-    return zp ? launch_storage<128, true>(a, r, mb, master, stream) : launch_storage<128, false>(a, r, mb, master, stream);
+    return zp ? launch_storage<128, true>(a, r, mb, one, master, stream) : launch_storage<128, false>(a, r, mb, one, master, stream);
   if (group_size == 32)
-    return zp ? launch_storage<32, true>(a, r, mb, master, stream) : launch_storage<32, false>(a, r, mb, master, stream);
-  return zp ? launch_storage<-1, true>(a, r, mb, master, stream) : launch_storage<-1, false>(a, r, mb, master, stream);
+    return zp ? launch_storage<32, true>(a, r, mb, one, master, stream) : launch_storage<32, false>(a, r, mb, one, master, stream);
+  return zp ? launch_storage<-1, true>(a, r, mb, one, master, stream) : launch_storage<-1, false>(a, r, mb, one, master, stream);
 }
 
 }  // namespace matgptq
