@@ -65,16 +65,24 @@ class MatGPTQLinear(torch.nn.Module):
             self.register_buffer("matgptq_perm",
                                  perm.to(device=self.matgptq_qweight.device, dtype=torch.int64).reshape(-1))
 
-    @torch.no_grad()
     def forward(self, x: torch.Tensor) -> torch.Tensor:
+        # The product has no gradient.  Grad mode is switched off only where a tensor would ask for one: as a decorator the
+        # switch was 1.2 of the 8 us that a call on a few rows takes, which is all host time.
+        scales, zeros = self.matgptq_scales, self.matgptq_zeros
+        if torch.is_grad_enabled() and (x.requires_grad or scales.requires_grad or (zeros is not None and zeros.requires_grad)):
+            with torch.no_grad():
+                return self._product(x, scales, zeros)
+        return self._product(x, scales, zeros)
+
+    def _product(self, x: torch.Tensor, scales: torch.Tensor, zeros: Optional[torch.Tensor]) -> torch.Tensor:
         if self.matgptq_perm is not None:
             x = torch.index_select(x, -1, self.matgptq_perm)
-        if self.matgptq_zeros is not None:
+        if zeros is not None:
             return torch.ops.matgptq_cuda.matmul_matgptq_zp(
-                x, self.matgptq_qweight, self.matgptq_scales, self.matgptq_zeros,
+                x, self.matgptq_qweight, scales, zeros,
                 self.n_out_features, self.n_in_features, self.bitwidth, self.group_size, self.flag)
         return torch.ops.matgptq_cuda.matmul_matgptq(
-            x, self.matgptq_qweight, self.matgptq_scales,
+            x, self.matgptq_qweight, scales,
             self.n_out_features, self.n_in_features, self.bitwidth, self.group_size, self.flag)
 
     @torch.no_grad()
