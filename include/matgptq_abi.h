@@ -222,7 +222,7 @@ int matgptq_describe_plan(int bitwidth, int group_size, int64_t N, int64_t K, in
 /* Activation buffers (1 or 2) of the mid-batch kernel that matgptq_gemm would launch; 0 where it launches another one,
  * negative on an error. */
 int matgptq_midbatch_buffers(int bitwidth, int group_size, int64_t N, int64_t K, int64_t M, int has_zeros, uint32_t flags);
-/* Row blocks of 16 weight rows per workgroup (1, 2 or 4) of the few-rows kernel (up to 16 batch rows) where matgptq_gemm, or
+/* Row blocks of 16 weight rows per workgroup (1, 2, 4 or 8) of the few-rows kernel (up to 64 batch rows) where matgptq_gemm, or
  * with master != 0 matgptq_gemm_master, launches it; 0 where it launches another one, negative on an error. */
 int matgptq_few_rows(int bitwidth, int group_size, int64_t N, int64_t K, int64_t M, uint32_t flags, int master);
 

@@ -28,8 +28,8 @@ int check_problem(int bits, int group_size, int64_t N, int64_t K);  // pack_host
                                 bool stream_flavour, size_t smem, hipStream_t);                \
   hipError_t launch_prefill_b##B(const GemmArgs&, int group_size, int cfg, hipStream_t);          \
   hipError_t launch_skinny_b##B(const GemmArgs&, int group_size, int r, int mb, bool one, bool master, hipStream_t);   \
-  hipError_t launch_few_rows_b##B(const GemmArgs&, int group_size, int r, bool master, hipStream_t);          \
-  hipError_t launch_few_rows_b##B##_bf16(const GemmArgs&, int group_size, int r, bool master, hipStream_t);   \
+  hipError_t launch_few_rows_b##B(const GemmArgs&, int group_size, int r, int rows, bool master, hipStream_t);          \
+  hipError_t launch_few_rows_b##B##_bf16(const GemmArgs&, int group_size, int r, int rows, bool master, hipStream_t);   \
   hipError_t launch_gemv_b##B(const GemmArgs&, int group_size, int shape, int W, size_t lds_pad, bool master, hipStream_t);  \
   hipError_t launch_gemv_b##B##_bf16(const GemmArgs&, int group_size, int shape, int W, size_t lds_pad, bool master, hipStream_t); \
   hipError_t launch_gemv_prologue_b##B(const GemmArgs&, int kind, int shape, int W, const void* b, const void* w, void* out, \
@@ -556,23 +556,23 @@ hipError_t launch_skinny(int bits, bool bf16, const GemmArgs& a, int g, const Pl
 #undef MATGPTQ_CASE
 }
 
-hipError_t launch_few_rows(int bits, bool bf16, const GemmArgs& a, int g, int r, bool master, hipStream_t s) {
+hipError_t launch_few_rows(int bits, bool bf16, const GemmArgs& a, int g, FewRows f, bool master, hipStream_t s) {
 #define MATGPTQ_CASE(B) \
-  case B: return bf16 ? launch_few_rows_b##B##_bf16(a, g, r, master, s) : launch_few_rows_b##B(a, g, r, master, s);
+  case B: return bf16 ? launch_few_rows_b##B##_bf16(a, g, f.row_blocks, f.batch_rows, master, s) : launch_few_rows_b##B(a, g, f.row_blocks, f.batch_rows, master, s);
   switch (bits) {
     MATGPTQ_CASE(2)
     MATGPTQ_CASE(3)
     MATGPTQ_CASE(4)
     MATGPTQ_CASE(6)
-    default: return bf16 ? launch_few_rows_b8_bf16(a, g, r, master, s) : launch_few_rows_b8(a, g, r, master, s);
+    default: return bf16 ? launch_few_rows_b8_bf16(a, g, f.row_blocks, f.batch_rows, master, s) : launch_few_rows_b8(a, g, f.row_blocks, f.batch_rows, master, s);
   }
 #undef MATGPTQ_CASE
 }
 
-// Row blocks per workgroup of the few-rows kernel where a call without a forced variant takes it, else 0.
-int few_rows_of(int bits, int group_size, int64_t N, int64_t K, int64_t M, uint32_t flags, bool master) {
-  if ((flags & (MATGPTQ_FLAG_VARIANT_MASK | MATGPTQ_FLAG_FLAVOUR_MASK)) != 0 || M > kFewRowsMaxM) return 0;
-  return few_rows_row_blocks(bits, group_size, (flags & MATGPTQ_FLAG_BF16) != 0, master, (int)M, (int)(N / 16), (int)(K / 128));
+// Workgroup of the few-rows kernel where a call without a forced variant takes it, else no row blocks.
+FewRows few_rows_of(int bits, int group_size, int64_t N, int64_t K, int64_t M, uint32_t flags, bool master) {
+  if ((flags & (MATGPTQ_FLAG_VARIANT_MASK | MATGPTQ_FLAG_FLAVOUR_MASK)) != 0 || M > kFewRowsMaxM) return {0, 0};
+  return few_rows(bits, group_size, (flags & MATGPTQ_FLAG_BF16) != 0, master, (int)M, (int)(N / 16), (int)(K / 128));
 }
 
 }  // namespace
@@ -626,8 +626,8 @@ static int run_gemm(int bitwidth, int group_size, int64_t N, int64_t K, int64_t 
   if (!weights_dev || !scales_dev || !x_dev || !y_dev) return MATGPTQ_ENULL;
   Plan p;
   if (int e = make_plan(bitwidth, group_size, N, K, M, zeros_dev != nullptr, flags, &p)) return e;
-  const int few = few_rows_of(bitwidth, group_size, N, K, M, flags, master_planes);
-  if (master_planes && few == 0 && !plan_reads_planes(p, M)) return MATGPTQ_EVARIANT;
+  const FewRows few = few_rows_of(bitwidth, group_size, N, K, M, flags, master_planes);
+  if (master_planes && few.row_blocks == 0 && !plan_reads_planes(p, M)) return MATGPTQ_EVARIANT;
   GemmArgs a;
   a.packed = static_cast<const uint32_t*>(weights_dev);
   a.scales = static_cast<const uint16_t*>(scales_dev);
@@ -644,7 +644,7 @@ static int run_gemm(int bitwidth, int group_size, int64_t N, int64_t K, int64_t 
   const bool bf16 = (flags & MATGPTQ_FLAG_BF16) != 0;
   // (a forced variant on pre-sliced codes keeps the two buffers that matgptq_midbatch_buffers reports for it)
   const bool one_tile = master_planes || (flags & MATGPTQ_FLAG_VARIANT_MASK) == 0;
-  const hipError_t err = few != 0   ? launch_few_rows(bitwidth, bf16, a, group_size, few, master_planes, s)
+  const hipError_t err = few.row_blocks != 0 ? launch_few_rows(bitwidth, bf16, a, group_size, few, master_planes, s)
                          : p.gemv   ? launch_gemv(bitwidth, bf16, a, group_size, p, master_planes, s)
                          : p.decode ? launch_decode(bitwidth, bf16, a, group_size, p, s)
                          : p.skinny ? launch_skinny(bitwidth, bf16, a, group_size, p, one_tile, master_planes, s)
@@ -734,10 +734,12 @@ static int master_reads_planes(int bitwidth, int group_size, int64_t N, int64_t 
   Plan p;
   if (int e = make_plan(bitwidth, group_size, N, K, M, zp, *flags, &p)) return e;
   *direct = plan_reads_planes(p, M);
-  if (few_rows_of(bitwidth, group_size, N, K, M, *flags, true) != 0) {
+  const bool few = few_rows_of(bitwidth, group_size, N, K, M, *flags, true).row_blocks != 0;
+  if (few && M <= 16) {
     *direct = true;
     return MATGPTQ_OK;
   }
+  const uint32_t asked = *flags;
   const bool automatic = (*flags & MATGPTQ_FLAG_VARIANT_MASK) == 0 && ((*flags >> 16) & 3u) == 0;
   if (!*direct && automatic && M <= kGemvMaxM) {
     // the planner's own gemv shape for this problem has no instantiation on planes (four row blocks
@@ -757,6 +759,8 @@ static int master_reads_planes(int bitwidth, int group_size, int64_t N, int64_t 
       *direct = true;
     }
   }
+  // (a shape that needs the workspace keeps it, and multiplies the codes sliced there)
+  if (few && *direct) *flags = asked;
   return MATGPTQ_OK;
 }
 
@@ -900,7 +904,7 @@ int matgptq_midbatch_buffers(int bitwidth, int group_size, int64_t N, int64_t K,
 int matgptq_few_rows(int bitwidth, int group_size, int64_t N, int64_t K, int64_t M, uint32_t flags, int master) {
   if (int e = check_problem(bitwidth, group_size, N, K)) return e;
   if (M <= 0) return MATGPTQ_ESIZE;
-  return few_rows_of(bitwidth, group_size, N, K, M, flags, master != 0);
+  return few_rows_of(bitwidth, group_size, N, K, M, flags, master != 0).row_blocks;
 }
 
 int matgptq_pack_device(const uint8_t* codes_dev, int64_t N, int64_t K, int bitwidth,

@@ -1,4 +1,4 @@
-// Few-rows kernel: one to sixteen batch rows, one scale per tile of 128 columns or per row.
+// Few-rows kernel: one to 64 batch rows, one scale per tile of 128 columns or per row.
 // Compiled once per bitwidth with -DMATGPTQ_BITS=b.
 // Role of the reference's small-batch kernels (inference_lib/matgptq_cuda/csrc/matgptq_gemm.cu:337-953).
 //
@@ -6,7 +6,8 @@
 //    tile are copied with buffer_load ... lds into the wave's own buffer (256 contiguous bytes per 16 lanes, 16-byte chunk c
 //    of row r at position c ^ r), codes, scales and zeros go to registers.  Two buffers and two register sets: tile t + 2 is
 //    requested while t is multiplied and t + 1 is on its way.  Walks of one tile (K up to 1024) have one of each, half the
-//    registers, and more workgroups per CU.  Buffers hold 4, 8 or 16 batch rows.
+//    registers, and more workgroups per CU.  Buffers hold 4, 8, 16 or 32 batch rows; with 32 there is one buffer (64 KB for the
+//    eight waves), refilled as soon as its operands are in registers, and two register sets.
 //  * Codes are matrix operands as they are (raw_operand.h): a mask and an OR per pair of codes, no weight is formed.  The
 //    activations are the 16-row operand, the 16 weight rows the columns, so lane (n, q) ends with batch rows 4q .. 4q+3 of
 //    weight row n and applies that row's one scale to the four sums.  What the operand carries besides the code, and the zero
@@ -25,9 +26,11 @@
 //    8192 x 3584  4 bits fp16  M = 16  7.2 -> 6.7     1280 x 8192  4 bits fp16  M = 16  7.8 -> 7.0
 // and over 10000 random calls (every bitwidth and storage type, K = 256 .. 16384, M = 5 .. 16) 1.08 to 1.45 times faster on
 // the geometric mean of each format, slower by more than 1.5 % on one in a thousand.
-// Tried and taken back: activations loaded straight into the operand (16 rows x 64 bytes per load: 4096 x 14336 at M = 16
-// 13 -> 17 us), four buffers and everything requested at the start (28672 x 4096: within 3 % either way), sixteen waves
-// (ahead only below 5 rows on walks past 8192 columns), consecutive tiles per wave (2 % slower).
+// Seventeen to 64 batch rows: the rule in fewrows_plan.h says where and by how much.
+// Tried and taken back: 64 batch rows per workgroup (no faster than two workgroups of 32), activations loaded straight into
+// the operand (16 rows x 64 bytes per load: 4096 x 14336 at M = 16 13 -> 17 us), four buffers and everything requested at the
+// start (28672 x 4096: within 3 % either way), sixteen waves (ahead only below 5 rows on walks past 8192 columns), consecutive
+// tiles per wave (2 % slower).
 #include "fewrows_plan.h"
 #include "raw_operand.h"
 
@@ -49,28 +52,38 @@ constexpr int few_rows_min_waves(int bits, bool zp, int r, bool master, bool one
   return (one ? 1 : 2) * r * (words + 1 + (zp ? 1 : 0)) + 4 * r <= 64 ? 4 : 2;
 }
 
-// ROWS: batch rows held per tile, 8 or 16 (rows beyond M are never stored, whatever they hold)
+// ROWS: batch rows of a workgroup, 4, 8, 16 or 32 (rows beyond M are never stored, whatever they hold)
 // ONE: walks of one tile, which need one buffer and one register set
 template <int BITS, int GROUP, bool ZP, int R, int ROWS, bool MASTER, bool ONE>
-__global__ void __launch_bounds__(64 * kWaves, few_rows_min_waves(BITS, ZP, R, MASTER, ONE))
-few_rows_kernel(const GemmArgs a) {
+__global__ void __launch_bounds__(64 * kWaves, ROWS > 16 ? 2 : few_rows_min_waves(BITS, ZP, R, MASTER, ONE))
+few_rows_kernel(const GemmArgs a, int n_tiles, int m_tiles) {
   static_assert(GROUP == 128 || GROUP == -1, "one scale per tile or row");
   using Fmt = TileFormat<BITS, MASTER>;
   using Raw = RawOperand<BITS, MASTER>;
+  constexpr int MB = ROWS > 16 ? ROWS / 16 : 1;  // blocks of 16 batch rows
+  constexpr bool kTwo = !ONE && MB == 1;         // two buffers
+  constexpr int kSets = ONE ? 1 : 2;             // register sets
   constexpr int kStage = ROWS * 256;  // bytes of one activation buffer of a wave
   constexpr int kCopies = ROWS / 4;
-  constexpr int kSums = kWaves * R * 1024;  // the waves' sums reuse the first buffers
+  constexpr int kSums = kWaves * R * MB * 1024;  // the waves' sums reuse the first buffers
   constexpr float kMul = (float)(1 << (8 - BITS));
   __shared__ __align__(16) unsigned char smem_even[kWaves * kStage > kSums ? kWaves * kStage : kSums];
   // (an array of its own: the compiler orders LDS copies and reads per variable)
-  __shared__ __align__(16) unsigned char smem_odd[ONE ? 16 : kWaves * kStage];
+  __shared__ __align__(16) unsigned char smem_odd[kTwo ? kWaves * kStage : 16];
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r16 = lane & 15;
   const int q = lane >> 4;
-  const int rb_first = blockIdx.x * R;
+  // Workgroup ids go round-robin over the 8 XCDs: with several blocks of batch rows they are remapped so that the workgroups
+  // of one XCD walk those blocks of the same weight rows and share these in its L2.
+  const int total = n_tiles * m_tiles;
+  int lid = blockIdx.x;
+  if (m_tiles > 1 && (total & 7) == 0) lid = (blockIdx.x & 7) * (total >> 3) + (blockIdx.x >> 3);
+  const int nt = lid / m_tiles;
+  const int m0 = (lid - nt * m_tiles) * ROWS;
+  const int rb_first = nt * R;
 
   constexpr uint32_t tile_bytes = Fmt::kTileBytes;
   const uint32_t rb_bytes = (uint32_t)a.k_tiles * tile_bytes;
@@ -78,10 +91,13 @@ few_rows_kernel(const GemmArgs a) {
   const uint32_t aux_bytes = (uint32_t)a.row_blocks * a.G * 32;  // scales / zeros: [N/16][G][16] halves
   const uint32_t x_bytes = (uint32_t)a.M * (uint32_t)a.K * 2u;
 
-  float4v acc[R];
+  float4v acc[R][MB], xsum[MB];  // xsum: one scale per row with zero points, sums of all activations
 #pragma unroll
-  for (int rr = 0; rr < R; rr++) acc[rr] = float4v{0.f, 0.f, 0.f, 0.f};
-  float4v xsum = {0.f, 0.f, 0.f, 0.f};  // one scale per row with zero points: sums of all activations
+  for (int i = 0; i < MB; i++) {
+    xsum[i] = float4v{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int rr = 0; rr < R; rr++) acc[rr][i] = float4v{0.f, 0.f, 0.f, 0.f};
+  }
 
   const Raw raw;
   Frag centre[Raw::kOddOctets ? 2 : 1], ones;
@@ -97,7 +113,7 @@ few_rows_kernel(const GemmArgs a) {
   };
 
   // codes, scales and zeros of the tile in use and of the next one (scales and zeros as loaded)
-  uint32_t wr[ONE ? 1 : 2][R][Fmt::kWords], sr[ONE ? 1 : 2][R], zr[ONE ? 1 : 2][R];
+  uint32_t wr[kSets][R][Fmt::kWords], sr[kSets][R], zr[kSets][R];
   auto load_weights = [&](uint32_t (&w)[R][Fmt::kWords], uint32_t (&s)[R], uint32_t (&z)[R], int kb) {
 #pragma unroll
     for (int rr = 0; rr < R; rr++) {
@@ -119,12 +135,12 @@ few_rows_kernel(const GemmArgs a) {
   };
 
   // Copy of one tile's activations: instruction i moves rows 4i .. 4i+3 (lane l: row 4i + l/16, LDS position
-  // l%16, which holds chunk (l%16) ^ row of the row's 256 bytes).
+  // l%16, which holds chunk (l%16) ^ (row%16) of the row's 256 bytes).
   uint32_t copy_off[kCopies];
 #pragma unroll
   for (int i = 0; i < kCopies; i++) {
     const int row = 4 * i + q;
-    copy_off[i] = row < a.M ? (uint32_t)row * (uint32_t)a.K * 2u + (r16 ^ row) * 16 : x_bytes;
+    copy_off[i] = m0 + row < a.M ? (uint32_t)(m0 + row) * (uint32_t)a.K * 2u + (r16 ^ (row & 15)) * 16 : x_bytes;
   }
   auto copy_x = [&](unsigned char* to, int kb) {
     const BufRsrc xres = make_rsrc(a.x, kb < a.k_tiles ? x_bytes : 0u);
@@ -136,71 +152,90 @@ few_rows_kernel(const GemmArgs a) {
   };
 
   unsigned char* const stage_even = smem_even + wave * kStage;
-  unsigned char* const stage_odd = smem_odd + (ONE ? 0 : wave * kStage);
-  const int xrow = r16 & (ROWS - 1);
+  unsigned char* const stage_odd = smem_odd + (kTwo ? wave * kStage : 0);
+  const int xrow = ROWS < 16 ? r16 & (ROWS - 1) : r16;
   constexpr int kLoads = kCopies + R * ((MASTER ? master_load_count(BITS) : tile_load_count(BITS)) + (GROUP == -1 ? 0 : ZP ? 2 : 1));
   static_assert(kLoads < 64, "vmcnt counts up to 63");
-  // Tile t of the walk (K tile wave + 8 t) in buffer and register set `btag`.  `moretag`: tile t + 2 is requested;
-  // without it (the last two tiles) set 0 leaves set 1's requests in flight, set 1 none.
+  // Tile t of the walk (K tile wave + 8 t) in register set `btag`.  `moretag`: with two buffers tile t + 2 is requested
+  // (without it, on the last two tiles, set 0 leaves set 1's requests in flight, set 1 none), with one tile t + 1 as soon as
+  // the operands are in registers.
   auto tile = [&](int t, auto btag, auto moretag) {
     constexpr int B = decltype(btag)::value;
     constexpr bool kMore = decltype(moretag)::value;
-    constexpr int kYounger = !ONE && (kMore || B == 0) ? kLoads : 0;  // requests of the tile behind this one
+    constexpr int kYounger = kTwo && (kMore || B == 0) ? kLoads : 0;  // requests of the tile behind this one
     const int kb = wave + t * kWaves;
-    unsigned char* const buf = B == 0 ? stage_even : stage_odd;
+    unsigned char* const buf = kTwo && B == 1 ? stage_odd : stage_even;
     __builtin_amdgcn_sched_barrier(0);
     __builtin_amdgcn_s_waitcnt((kYounger & 15) | (7 << 4) | (15 << 8) | ((kYounger >> 4) << 14));
     __builtin_amdgcn_sched_barrier(0);
-    Frag xf[4];
+    Frag xf[4][MB];
 #pragma unroll
-    for (int j = 0; j < 4; j++) xf[j].v = *reinterpret_cast<const uint4*>(buf + xrow * 256 + (((4 * j + q) ^ xrow) * 16));
+    for (int j = 0; j < 4; j++)
+#pragma unroll
+      for (int i = 0; i < MB; i++)
+        xf[j][i].v = *reinterpret_cast<const uint4*>(buf + (i * 16 + xrow) * 256 + (((4 * j + q) ^ xrow) * 16));
     __builtin_amdgcn_sched_barrier(0);
     if constexpr (kMore) {
       __builtin_amdgcn_s_waitcnt(15 | (7 << 4) | (0 << 8) | (3 << 14));  // lgkmcnt(0): the buffer is free
       __builtin_amdgcn_sched_barrier(0);
-      copy_x(buf, kb + 2 * kWaves);
+      copy_x(buf, kb + (kTwo ? 2 : 1) * kWaves);
+      if constexpr (!kTwo) load_weights(wr[(B + 1) % kSets], sr[(B + 1) % kSets], zr[(B + 1) % kSets], kb + kWaves);
     }
     // (only the last tile of a walk can lie beyond K; its buffer may hold anything)
     if (kMore || kb < a.k_tiles) {
       const float4v zero4 = {0.f, 0.f, 0.f, 0.f};
-      float4v off = zero4, xs = zero4;
+      float4v off[MB], xs[MB];
 #pragma unroll
-      for (int j = 0; j < 4; j++) {
-        off = mma(xf[j], centre[Raw::kOddOctets ? (j & 1) : 0], off);
-        if constexpr (ZP) xs = mma(xf[j], ones, xs);
+      for (int i = 0; i < MB; i++) {
+        off[i] = zero4;
+        xs[i] = zero4;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+          off[i] = mma(xf[j][i], centre[Raw::kOddOctets ? (j & 1) : 0], off[i]);
+          if constexpr (ZP) xs[i] = mma(xf[j][i], ones, xs[i]);
+        }
+        if constexpr (ZP && GROUP == -1) xsum[i] += xs[i];
       }
-      if constexpr (ZP && GROUP == -1) xsum += xs;
 #pragma unroll
       for (int rr = 0; rr < R; rr++) {
-        float4v d = off;
-        if constexpr (GROUP == -1) {
-          d += acc[rr];
-        } else if constexpr (ZP) {
-          const float z = 128.0f / kMul - storage_to_float((uint16_t)zr[B][rr]) * (1.0f / kMul);
+        float4v d[MB];
+        float z = 0.f;
+        if constexpr (ZP && GROUP != -1) z = 128.0f / kMul - storage_to_float((uint16_t)zr[B][rr]) * (1.0f / kMul);
 #pragma unroll
-          for (int e = 0; e < 4; e++) d[e] = __builtin_fmaf(z, xs[e], d[e]);
+        for (int i = 0; i < MB; i++) {
+          d[i] = off[i];
+          if constexpr (GROUP == -1) {
+            d[i] += acc[rr][i];
+          } else if constexpr (ZP) {
+#pragma unroll
+            for (int e = 0; e < 4; e++) d[i][e] = __builtin_fmaf(z, xs[i][e], d[i][e]);
+          }
         }
         auto one = [&](auto jtag) {
           constexpr int J = decltype(jtag)::value;
           Frag codes;
           raw.template octet<J>(wr[B][rr], codes.u);
-          d = mma(xf[J], codes, d);
+#pragma unroll
+          for (int i = 0; i < MB; i++) d[i] = mma(xf[J][i], codes, d[i]);
         };
         one(std::integral_constant<int, 0>{});
         one(std::integral_constant<int, 1>{});
         one(std::integral_constant<int, 2>{});
         one(std::integral_constant<int, 3>{});
         if constexpr (GROUP == -1) {
-          acc[rr] = d;
+#pragma unroll
+          for (int i = 0; i < MB; i++) acc[rr][i] = d[i];
         } else {
           const float s = storage_to_float((uint16_t)sr[B][rr]);
 #pragma unroll
-          for (int e = 0; e < 4; e++) acc[rr][e] = __builtin_fmaf(s, d[e], acc[rr][e]);
+          for (int i = 0; i < MB; i++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) acc[rr][i][e] = __builtin_fmaf(s, d[i][e], acc[rr][i][e]);
         }
       }
     }
     __builtin_amdgcn_sched_barrier(0);
-    if constexpr (kMore) load_weights(wr[B], sr[B], zr[B], kb + 2 * kWaves);
+    if constexpr (kMore && kTwo) load_weights(wr[B], sr[B], zr[B], kb + 2 * kWaves);
   };
 
   const int walk = (a.k_tiles + kWaves - 1) / kWaves;  // tiles of the longest walk
@@ -211,6 +246,19 @@ few_rows_kernel(const GemmArgs a) {
   load_weights(wr[0], sr[0], zr[0], wave);
   if constexpr (ONE) {
     tile(0, Even{}, std::false_type{});
+  } else if constexpr (!kTwo) {
+    // (every tile but the last requests the next one, which lies beyond K for the waves with a shorter walk)
+    int t = 0;
+    for (; t + 2 < walk; t += 2) {
+      tile(t, Even{}, std::true_type{});
+      tile(t + 1, Odd{}, std::true_type{});
+    }
+    if (t + 1 < walk) {
+      tile(t, Even{}, std::true_type{});
+      tile(t + 1, Odd{}, std::false_type{});
+    } else {
+      tile(t, Even{}, std::false_type{});
+    }
   } else {
     copy_x(stage_odd, wave + kWaves);
     load_weights(wr[1], sr[1], zr[1], wave + kWaves);
@@ -229,14 +277,21 @@ few_rows_kernel(const GemmArgs a) {
 #pragma unroll
   for (int rr = 0; rr < R; rr++)
 #pragma unroll
-    for (int e = 0; e < 4; e++) finite = finite && __builtin_isfinite(acc[rr][e]);
+    for (int i = 0; i < MB; i++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) finite = finite && __builtin_isfinite(acc[rr][i][e]);
   const bool again = __builtin_amdgcn_ballot_w64(!finite) != 0;
   if (again) {
     const typename Fmt::Consts unpack;
-    const uint32_t x_off = xrow < a.M ? (uint32_t)xrow * (uint32_t)a.K * 2u + q * 16 : x_bytes;
     const BufRsrc xres = make_rsrc(a.x, x_bytes);
+    uint32_t x_off[MB];
 #pragma unroll
-    for (int rr = 0; rr < R; rr++) acc[rr] = float4v{0.f, 0.f, 0.f, 0.f};
+    for (int i = 0; i < MB; i++) {
+      const int row = m0 + i * 16 + xrow;
+      x_off[i] = row < a.M ? (uint32_t)row * (uint32_t)a.K * 2u + q * 16 : x_bytes;
+#pragma unroll
+      for (int rr = 0; rr < R; rr++) acc[rr][i] = float4v{0.f, 0.f, 0.f, 0.f};
+    }
     for (int kb = wave; kb < a.k_tiles; kb += kWaves) {
 #pragma unroll
       for (int rr = 0; rr < R; rr++) {
@@ -248,16 +303,20 @@ few_rows_kernel(const GemmArgs a) {
         const float z = ZP ? s * (storage_to_float(a.zeros[g]) - 128.0f) : __uint_as_float(opaque_vgpr(0u));
         auto one = [&](auto jtag) {
           constexpr int J = decltype(jtag)::value;
-          const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(xres, x_off, (uint32_t)kb * 256u + J * 64u, 0);
-          Frag x, aw;
-          x.v = make_uint4(v.x, v.y, v.z, v.w);
+          Frag aw;
           if constexpr (kBf16) {
             dequant_octet_bf16_fmt<Fmt, BITS, J>(w, unpack, s * kMul, z, aw);
           } else {
             const _Float16 s1 = (_Float16)(s * kMul), z1 = (_Float16)z;
             dequant_octet_fmt<Fmt, BITS, J, true>(w, unpack, half2v{z1, z1}, half2v{s1, s1}, aw);
           }
-          acc[rr] = mma(x, aw, acc[rr]);
+#pragma unroll
+          for (int i = 0; i < MB; i++) {
+            const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(xres, x_off[i], (uint32_t)kb * 256u + J * 64u, 0);
+            Frag x;
+            x.v = make_uint4(v.x, v.y, v.z, v.w);
+            acc[rr][i] = mma(x, aw, acc[rr][i]);
+          }
         };
         one(std::integral_constant<int, 0>{});
         one(std::integral_constant<int, 1>{});
@@ -266,7 +325,9 @@ few_rows_kernel(const GemmArgs a) {
       }
     }
 #pragma unroll
-    for (int rr = 0; rr < R; rr++) acc[rr] *= 1.0f / kMul;
+    for (int rr = 0; rr < R; rr++)
+#pragma unroll
+      for (int i = 0; i < MB; i++) acc[rr][i] *= 1.0f / kMul;
   }
 
   if (GROUP == -1 && !again) {  // the row's one scale and zero point
@@ -274,64 +335,77 @@ few_rows_kernel(const GemmArgs a) {
     for (int rr = 0; rr < R; rr++) {
       const int rb = rb_first + rr < a.row_blocks ? rb_first + rr : a.row_blocks - 1;
       const float s = storage_to_float(a.scales[(size_t)rb * 16 + r16]);
-      if constexpr (ZP) {
-        const float z = 128.0f / kMul - storage_to_float(a.zeros[(size_t)rb * 16 + r16]) * (1.0f / kMul);
+      const float z = ZP ? 128.0f / kMul - storage_to_float(a.zeros[(size_t)rb * 16 + r16]) * (1.0f / kMul) : 0.f;
 #pragma unroll
-        for (int e = 0; e < 4; e++) acc[rr][e] = __builtin_fmaf(z, xsum[e], acc[rr][e]);
-      }
-      // (a sum times scale 0 is +0, as a sum of products with it is)
+      for (int i = 0; i < MB; i++)
 #pragma unroll
-      for (int e = 0; e < 4; e++) acc[rr][e] = __builtin_fmaf(s, acc[rr][e], 0.f);
+        for (int e = 0; e < 4; e++) {
+          if constexpr (ZP) acc[rr][i][e] = __builtin_fmaf(z, xsum[i][e], acc[rr][i][e]);
+          // (a sum times scale 0 is +0, as a sum of products with it is)
+          acc[rr][i][e] = __builtin_fmaf(s, acc[rr][i][e], 0.f);
+        }
     }
   }
 
   // The waves' sums of every output meet in LDS (over the activation buffers: every wave has to be done with its
-  // own first), four batch rows 4q .. 4q+3 of weight row r16 per lane and row block.
+  // own first), four batch rows 4q .. 4q+3 of weight row r16 per lane, row block and batch block.
   __builtin_amdgcn_s_waitcnt(0 | (7 << 4) | (0 << 8) | (0 << 14));  // nothing in flight into LDS any more
   __syncthreads();
   float* const red = reinterpret_cast<float*>(smem_even);
 #pragma unroll
-  for (int rr = 0; rr < R; rr++) *reinterpret_cast<float4v*>(red + ((wave * R + rr) * 64 + lane) * 4) = acc[rr];
+  for (int rr = 0; rr < R; rr++)
+#pragma unroll
+    for (int i = 0; i < MB; i++) *reinterpret_cast<float4v*>(red + (((wave * R + rr) * MB + i) * 64 + lane) * 4) = acc[rr][i];
   __syncthreads();
-  for (int o = tid; o < R * 256; o += 64 * kWaves) {
+  for (int o = tid; o < R * MB * 256; o += 64 * kWaves) {
     float sum = red[o];
 #pragma unroll
-    for (int w = 1; w < kWaves; w++) sum += red[w * R * 256 + o];
-    const int l = (o >> 2) & 63;
-    const int rb = rb_first + (o >> 8), m = 4 * (l >> 4) + (o & 3);
+    for (int w = 1; w < kWaves; w++) sum += red[w * R * MB * 256 + o];
+    const int l = (o >> 2) & 63, ri = o >> 8;
+    const int rb = rb_first + ri / MB, m = m0 + (ri % MB) * 16 + 4 * (l >> 4) + (o & 3);
     if (rb < a.row_blocks && m < a.M) a.y[(size_t)m * a.N + (size_t)rb * 16 + (l & 15)] = float_to_storage(sum * kMul);
   }
 }
 
 template <int GROUP, bool ZP, int R, int ROWS, bool MASTER>
 hipError_t launch_r(const GemmArgs& a, hipStream_t stream) {
-  const dim3 grid((a.row_blocks + R - 1) / R), block(64 * kWaves);
+  const int n_tiles = (a.row_blocks + R - 1) / R, m_tiles = (a.M + ROWS - 1) / ROWS;
+  const dim3 grid(n_tiles * m_tiles), block(64 * kWaves);
   if (a.k_tiles <= kWaves)
-    hipLaunchKernelGGL((few_rows_kernel<kBits, GROUP, ZP, R, ROWS, MASTER, true>), grid, block, 0, stream, a);
+    hipLaunchKernelGGL((few_rows_kernel<kBits, GROUP, ZP, R, ROWS, MASTER, true>), grid, block, 0, stream, a, n_tiles, m_tiles);
   else
-    hipLaunchKernelGGL((few_rows_kernel<kBits, GROUP, ZP, R, ROWS, MASTER, false>), grid, block, 0, stream, a);
+    hipLaunchKernelGGL((few_rows_kernel<kBits, GROUP, ZP, R, ROWS, MASTER, false>), grid, block, 0, stream, a, n_tiles, m_tiles);
   return hipGetLastError();
 }
 
 template <int GROUP, bool ZP, int R, bool MASTER>
-hipError_t launch_batch(const GemmArgs& a, hipStream_t stream) {
-  if (a.M <= 4) return launch_r<GROUP, ZP, R, 4, MASTER>(a, stream);
-  return a.M <= 8 ? launch_r<GROUP, ZP, R, 8, MASTER>(a, stream) : launch_r<GROUP, ZP, R, 16, MASTER>(a, stream);
+hipError_t launch_batch(const GemmArgs& a, int rows, hipStream_t stream) {
+  if constexpr (R >= 2) {
+    if (rows > 16) return launch_r<GROUP, ZP, R, 32, MASTER>(a, stream);
+  }
+  if constexpr (R <= 4) {
+    if (a.M <= 4) return launch_r<GROUP, ZP, R, 4, MASTER>(a, stream);
+    return a.M <= 8 ? launch_r<GROUP, ZP, R, 8, MASTER>(a, stream) : launch_r<GROUP, ZP, R, 16, MASTER>(a, stream);
+  }
+  return hipErrorInvalidValue;
 }
 
 template <int GROUP, bool ZP, bool MASTER>
-hipError_t launch_rows(const GemmArgs& a, int r, hipStream_t s) {
-  // (four row blocks of 8-bit codes, or of six and eight planes, do not fit the registers)
-  if constexpr (kBits <= (MASTER ? 4 : 6)) {
-    if (r >= 4) return launch_batch<GROUP, ZP, 4, MASTER>(a, s);
+hipError_t launch_rows(const GemmArgs& a, int r, int rows, hipStream_t s) {
+  // (what the registers hold: few_rows_most_row_blocks)
+  if constexpr (few_rows_most_row_blocks(kBits, MASTER, 32) >= 8) {
+    if (r >= 8) return launch_batch<GROUP, ZP, 8, MASTER>(a, rows, s);
   }
-  if (r >= 2) return launch_batch<GROUP, ZP, 2, MASTER>(a, s);
-  return launch_batch<GROUP, ZP, 1, MASTER>(a, s);
+  if constexpr (few_rows_most_row_blocks(kBits, MASTER, 16) >= 4) {
+    if (r >= 4) return launch_batch<GROUP, ZP, 4, MASTER>(a, rows, s);
+  }
+  if (r >= 2) return launch_batch<GROUP, ZP, 2, MASTER>(a, rows, s);
+  return launch_batch<GROUP, ZP, 1, MASTER>(a, rows, s);
 }
 
 template <int GROUP, bool ZP>
-hipError_t launch_storage(const GemmArgs& a, int r, bool master, hipStream_t s) {
-  return master ? launch_rows<GROUP, ZP, true>(a, r, s) : launch_rows<GROUP, ZP, false>(a, r, s);
+hipError_t launch_storage(const GemmArgs& a, int r, int rows, bool master, hipStream_t s) {
+  return master ? launch_rows<GROUP, ZP, true>(a, r, rows, s) : launch_rows<GROUP, ZP, false>(a, r, rows, s);
 }
 
 }  // namespace
@@ -343,14 +417,14 @@ hipError_t launch_storage(const GemmArgs& a, int r, bool master, hipStream_t s) 
 #else
 #define MATGPTQ_LAUNCH_NAME MATGPTQ_CAT(launch_few_rows_b, MATGPTQ_BITS)
 #endif
-// M <= 16, group size 128 or -1.  r: row blocks of 16 weight rows per workgroup (1, 2 or 4); master: `a.packed` holds
-// master-resident bit planes
-hipError_t MATGPTQ_LAUNCH_NAME(const GemmArgs& a, int group_size, int r, bool master, hipStream_t stream) {
+// Group size 128 or -1.  r: row blocks of 16 weight rows per workgroup (1, 2, 4; 2, 4, 8 with 32 batch rows); rows: batch rows
+// per workgroup, 16 (fewer are taken where M is 4 or 8 at most) or 32; master: `a.packed` holds master-resident bit planes
+hipError_t MATGPTQ_LAUNCH_NAME(const GemmArgs& a, int group_size, int r, int rows, bool master, hipStream_t stream) {
   const bool zp = a.zeros != nullptr;
-  if (a.M > 16 || group_size == 32) return hipErrorInvalidValue;
+  if (group_size == 32) return hipErrorInvalidValue;
   if (group_size == 128)
-    return zp ? launch_storage<128, true>(a, r, master, stream) : launch_storage<128, false>(a, r, master, stream);
-  return zp ? launch_storage<-1, true>(a, r, master, stream) : launch_storage<-1, false>(a, r, master, stream);
+    return zp ? launch_storage<128, true>(a, r, rows, master, stream) : launch_storage<128, false>(a, r, rows, master, stream);
+  return zp ? launch_storage<-1, true>(a, r, rows, master, stream) : launch_storage<-1, false>(a, r, rows, master, stream);
 }
 
 }  // namespace matgptq

@@ -487,7 +487,7 @@ def test_few_rows_at_the_edges_of_the_rule():
     few = _lib.load().matgptq_few_rows
     plain, bf16 = 1, 3
     assert few(5, 128, 4096, 4096, 8, plain, 0) < 0 and few(4, 128, 4096, 4096, 0, plain, 0) < 0
-    assert few(4, 32, 4096, 4096, 8, plain, 0) == 0 and few(4, 128, 4096, 4096, 17, plain, 0) == 0
+    assert few(4, 32, 4096, 4096, 8, plain, 0) == 0 and few(4, 32, 256, 4096, 17, bf16, 0) == 0 and few(4, 128, 256, 1024, 65, bf16, 0) == 0
     assert few(4, 128, 4096, 4096, 8, plain | (80 << 8), 0) == 0 and few(4, 128, 4096, 4096, 8, plain | (1 << 16), 0) == 0
     # up to four rows of fp16 storage at group 128: the gemv kernel, as with a fused prologue
     assert [few(4, g, 256, 1024, m, plain, 0) for g, m in ((128, 1), (128, 4), (128, 5), (-1, 1))] == [0, 0, 1, 1]
@@ -502,3 +502,15 @@ def test_few_rows_at_the_edges_of_the_rule():
     assert [few(4, -1, 16 * n, 4096, 8, plain, 0) for n in (1, 319, 320, 512, 513, 636, 637)] == [1, 1, 2, 2, 2, 2, 4]
     assert [few(4, 128, 16 * n, 4096, 9, plain, 0) for n in (318, 319, 636, 637)] == [1, 2, 2, 4]
     assert [few(b, 128, 65536, 4096, 16, plain, p) for b, p in ((6, 0), (8, 0), (4, 1), (6, 1))] == [4, 2, 4, 2]
+    # seventeen and more: the smallest workgroup whose count does not exceed the CUs
+    of = lambda m, ks, ns, bits=4, flags=bf16, planes=0: [few(bits, -1, 16 * n, 128 * k, m, flags, planes) for k in ks for n in ns]
+    assert of(64, (3, 6, 8), (160, 161, 192, 193, 256, 257, 384, 385)) == [1, 1, 1, 0, 0, 0, 0, 0, 1, 1, 1, 2, 2, 2, 2, 0, 1, 0, 0, 0, 0, 2, 2, 0] and of(17, (9, 128), (128,)) == [1, 1]
+    assert of(32, (9, 17, 24, 25), (129, 256)) == [0, 0, 0, 0, 0, 0, 2, 2] and of(32, (16, 17), (257, 512)) == [0, 0, 2, 2]
+    assert of(17, (9, 17), (513, 1024, 1025, 4000)) == [4, 4, 0, 0, 4, 4, 8, 8] and of(17, (17,), (2048, 2049), flags=plain) == [8, 0]
+    assert of(17, (17,), (1024, 4000), bits=6, flags=plain) == [4, 4] and of(17, (17,), (513, 4000), bits=8) == [0, 0]
+    assert of(17, (17,), (513, 1025), planes=1) == [4, 0] and [of(17, (25,), (129, 513), bits=b, planes=1) for b in (4, 6)] == [[2, 4], [0, 0]]
+    assert of(33, (9,), (85, 86, 128, 129, 170, 171, 256, 257, 340, 341)) == [1, 0, 0, 2, 2, 0, 0, 4, 4, 0]
+    assert of(49, (9, 17), (64,)) == [0, 1] and of(49, (9,), (65, 256, 257, 512, 513)) == [0, 0, 4, 4, 0] and of(64, (17,), (128, 129, 256, 257)) == [0, 2, 2, 4]
+    assert of(49, (40, 41), (257,)) == [4, 4] and of(49, (40, 41), (257,), flags=plain) == [4, 0]
+    # fp16 storage with a scale per tile: below 32 rows
+    assert [few(4, 128, 256, 4096, m, plain, p) for m in (31, 32, 64) for p in (0, 1)] == [1, 1, 0, 0, 0, 0]
