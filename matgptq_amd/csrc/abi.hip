@@ -73,6 +73,7 @@ struct Plan {
   size_t pad;    // gemv: dynamic LDS to ask for at least (bounds the workgroups per CU)
   bool decode;
   bool skinny;   // mid-batch kernel (K split inside the workgroup), R row blocks per workgroup
+  bool sliced_only;  // mid-batch in place of a tile that planes are sliced for first: they still are
   int mb;        // mid-batch: blocks of 16 batch rows per workgroup
   int R, S, W;   // decode: row blocks per wave, slots and k-slices per workgroup
   int kc;        // decode: tiles of K staged in LDS at a time
@@ -108,6 +109,7 @@ int make_plan(int bits, int group_size, int64_t N, int64_t K, int64_t M, bool zp
   p->shape = 0;
   p->pad = 0;
   p->skinny = false;
+  p->sliced_only = false;
   p->mb = 2;
   p->cfg = 0;
   // default decode shape (measured on MI355X, M = 1, Llama-3-8B layers): eight waves per
@@ -224,6 +226,16 @@ int make_plan(int bits, int group_size, int64_t N, int64_t K, int64_t M, bool zp
         const double t_192 = rounds(wgs_192) * 1.5 / 1.09;
         const double t_128 = rounds(wgs_128);
         p->cfg = t_192 < t_128 && fits_192 ? 9 : 3;
+        // One round of 128 x 192 tiles, where 128 x 128 tiles need a second one, pays for every format but 3 bits of bf16
+        // storage at group size 32 with zero points (0.6), also for those that lose where rounds are many: 1.15 to 1.30, 550
+        // random calls.  Both widths in one launch where they take every slot once: 1.2 to 1.5 against 128 x 128, 1.03 to
+        // 1.13 against 128 x 192 alone (bf16 storage, and 6 bits without a scale per tile).
+        if (wgs_192 <= 512 && wgs_128 > 512 && !(bits == 3 && bf16 && g32zp)) {
+          int narrow = 0;
+          const int wide = prefill_mix_wide_tiles(row_blocks, m_tiles, &narrow);
+          const bool mix = (bf16 || (bits == 6 && group_size != 128)) && wide > 0 && wide * m_tiles <= 256;
+          p->cfg = mix ? 14 : 9;
+        }
         if (p->cfg == 3 && bf16 && bits == 8 && group_size != 32 && wgs_big <= 512) p->cfg = 11;
         // 6-bit codes on fp16 storage with one scale per tile or row: one register set refilled octet by
         // octet fits the 128 x 256 tile once the compiler is left to order the step itself (243 registers;
@@ -291,6 +303,9 @@ int make_plan(int bits, int group_size, int64_t N, int64_t K, int64_t M, bool zp
       // whose registers fit that tile (bf16 storage: all but 3 and 6 bits and group size 32 -
       // 8192 x 8192 at M = 1024 116 against 128 us at 4 bits, 127 against 148 at 8).
       const bool bf16 = (flags & MATGPTQ_FLAG_BF16) != 0;
+      const bool fixed_order = !bf16 && group_size == 128;
+      const int64_t wgs_192s = ((N + 191) / 192) * ((M + 127) / 128);
+      const double t_192s = 4.0 + kt * (wgs_192s > 192 ? 1.36 : 1.22);  // 128 x 192 tiles, K split
       if (wgs_128 <= 256) {
         const double wide_codes = bits == 8 ? 1.1 : 1.0;  // (8-bit codes: 24 against 22 us per 32 K tiles)
         const double t = 3.0 + kt * wide_codes * (0.66 + 0.32 * (double)wgs_128 / 256.0);
@@ -301,14 +316,12 @@ int make_plan(int bits, int group_size, int64_t N, int64_t K, int64_t M, bool zp
         const int64_t wgs_64s = ((N + 127) / 128) * ((M + 63) / 64);
         const double t6 = 4.5 + kt * (bits == 8 ? 1.2 : 1.0) * (bf16 ? 1.05 : 1.0) * (0.45 + 0.19 * (double)wgs_64s / 256.0);
         if (wgs_64s <= 256 && t6 < best) { best = t6; p->cfg = 16; }
-      } else if (wgs_big <= 256 && bits != 6 && !(bf16 && (bits == 3 || group_size == 32)) && !(group_size == 32 && zp)) {
+      } else if (bits != 6 && !(bf16 && (bits == 3 || group_size == 32)) && !(group_size == 32 && zp)) {
         const double t = 5.0 + kt * (wgs_big > 192 ? 1.65 : 1.4);
         if (t < best) { best = t; p->cfg = 11; }
         // the same with 128 x 192 tiles where those fill more of the CUs in their one round
         // (10240 x 8192 at M = 512: 216 workgroups, 91 us against 94 on 160 of the wider tile)
-        const int64_t wgs_192s = ((N + 191) / 192) * ((M + 127) / 128);
-        const double t3 = 4.0 + kt * (wgs_192s > 192 ? 1.36 : 1.22);
-        if (wgs_192s <= 256 && t3 < best) { best = t3; p->cfg = 13; }
+        if (wgs_192s <= 256 && t_192s < best) { best = t_192s; p->cfg = 13; }
       }
       for (int mb = 2; mb <= (M > 32 ? 4 : 2); mb <<= 1) {
         const int64_t m_tiles = (M + 16 * mb - 1) / (16 * mb);
@@ -339,6 +352,22 @@ int make_plan(int bits, int group_size, int64_t N, int64_t K, int64_t M, bool zp
           p->mb = mb;
           R = r;
         }
+      }
+      // Formats whose registers do not hold the 128 x 256 tile take the 128 x 192 tile with K split in place of the 128 x 128 tile:
+      // 1.24 to 1.30 over 2300 random calls, none slower.  (6-bit codes on fp16 storage with a scale per tile keep the order of
+      // their sums.)
+      if (!p->skinny && p->cfg == 3 && wgs_192s <= 256 && t_192s < best && !fixed_order) p->cfg = 13;
+      // The 64 x 128 tile on few of the CUs: workgroups of the mid-batch kernel a quarter or a half as large take more of them.
+      // Up to 96 of the tiles, 2000 random calls of 97 to 640 batch rows: 1.30 with 32 x 32 and, where 64 batch rows pad no more,
+      // 1.25 with 64 x 64 (8-bit codes, two row blocks at most, 0.93 that way, and 0.76 to 0.9 on walks of three tiles with
+      // 32 x 32: not those); more batch rows on fewer row blocks 0.76 to 1; 97 to 128 of the tiles 0.95 to 1.2.
+      // (fp16 storage with a scale per tile keeps the order of its sums.)
+      if (variant == 0 && !p->skinny && p->cfg == 16 && M > 96 && M <= 640 && !(bits == 8 && k_tiles <= 24) && !fixed_order &&
+          ((N + 127) / 128) * ((M + 63) / 64) <= 96) {
+        p->skinny = p->sliced_only = true;
+        const bool tall = r_max == 4 && ((M + 63) / 64) * 64 * 7 <= ((M + 31) / 32) * 32 * 8;
+        p->mb = tall ? 4 : 2;
+        R = tall ? 4 : 2;
       }
     }
   } else if (flavour == 0 && M > kGemvMaxM &&
@@ -611,7 +640,7 @@ const char* matgptq_strerror(int code) {
 // (the gemv kernel reads the planes in every batch size it is planned for: one to four rows, and five
 // to eight with one scale per tile or row)
 static bool plan_reads_planes(const Plan& p, int64_t M) {
-  return (p.gemv && M <= kGemvEightMaxM && (p.shape == 1 || p.shape == 2)) || p.skinny;
+  return (p.gemv && M <= kGemvEightMaxM && (p.shape == 1 || p.shape == 2)) || (p.skinny && !p.sliced_only);
 }
 
 // checks, plan, launch; `master_planes`: the weight operand is master-resident bit planes and

@@ -514,3 +514,20 @@ def test_few_rows_at_the_edges_of_the_rule():
     assert of(49, (40, 41), (257,)) == [4, 4] and of(49, (40, 41), (257,), flags=plain) == [4, 0]
     # fp16 storage with a scale per tile: below 32 rows
     assert [few(4, 128, 256, 4096, m, plain, p) for m in (31, 32, 64) for p in (0, 1)] == [1, 1, 0, 0, 0, 0]
+
+
+def test_planner_gives_the_wider_formats_192_rows_and_few_64_row_tiles_smaller_workgroups():
+    plan = lambda *a: _lib.describe_plan(*a).split(" zp")[1][2:]
+    # one round of 128 x 192 tiles with K split where the 128 x 256 tile spills; not 6 bits with the order of sums kept
+    assert [plan(6, g, 5984, 4096, 1024, True, f) for g, f in ((-1, 1), (32, 1), (128, 3), (128, 1))] == ["cfg13", "cfg13", "cfg13", "cfg3"]
+    assert plan(6, -1, 6160, 4096, 1024, True, 1) == "cfg3"
+    # one round of 128 x 192 tiles where 128 x 128 tiles need two, mixed with these where slots stay empty
+    assert [plan(6, g, 10240, 4096, 1024, True, f) for g, f in ((-1, 1), (32, 3), (128, 3), (128, 1))] == ["cfg14", "cfg14", "cfg14", "cfg9"]
+    assert plan(8, 32, 12288, 4096, 1024, True, 3) == "cfg9" and plan(8, 32, 12304, 4096, 1024, True, 3) == "cfg3"
+    assert plan(3, 32, 10240, 4096, 1024, True, 3) == "cfg3" and plan(3, 32, 10240, 4096, 1024, False, 3) == "cfg14"
+    # up to 96 tiles of 64 x 128: 32 x 32 or 64 x 64 of the mid-batch kernel; planes of more than 128 rows are sliced as before
+    assert plan(4, -1, 3072, 4096, 192, True, 1) == "R4 mb4"
+    assert [plan(4, 32, n, 4096, 192, True, 1) for n in (4096, 4112)] == ["R2 mb2", "cfg16"]
+    assert [plan(4, 32, 1024, 4096, m, True, 1) for m in (640, 641)] == ["R2 mb2", "cfg16"]
+    assert [plan(8, 32, 4096, k, 192, True, 1) for k in (3072, 3200)] == ["cfg16", "R2 mb2"]
+    assert _lib.load().matgptq_gemm_master_workspace_bytes(4, 32, 4096, 4096, 192, 1) == 4 * 4096 * 4096 // 8
