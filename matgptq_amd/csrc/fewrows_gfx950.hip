@@ -8,12 +8,11 @@
 //    requested while t is multiplied and t + 1 is on its way.  Walks of one tile (K up to 1024) have one of each, half the
 //    registers, and more workgroups per CU.  Buffers hold 4, 8, 16 or 32 batch rows; with 32 there is one buffer (64 KB for the
 //    eight waves), refilled as soon as its operands are in registers, and two register sets.
-//  * Codes are matrix operands as they are (raw_operand.h): a mask and an OR per pair of codes, no weight is formed.  The
-//    activations are the 16-row operand, the 16 weight rows the columns, so lane (n, q) ends with batch rows 4q .. 4q+3 of
-//    weight row n and applies that row's one scale to the four sums.  What the operand carries besides the code, and the zero
-//    point, multiply sums of activations only: two chains of four MFMAs against constants per tile, shared by the R row
-//    blocks, whose result is the start value of the code chain.  Per tile and row block that leaves some 30 vector
-//    instructions at 4 bits (the mid-batch kernel, which forms weights, has 50, on bf16 storage 66), and no rounded weight:
+//  * Codes are matrix operands as they are (raw_operand.h), no weight is formed: a mask, an OR and on fp16 storage a packed
+//    addition per pair of codes.  The activations are the 16-row operand, the 16 weight rows the columns, so lane (n, q) ends
+//    with batch rows 4q .. 4q+3 of weight row n and applies that row's one scale to the four sums.  The zero point, and what
+//    the operand of bf16 storage carries besides the code, multiply sums of activations only: chains of four MFMAs against
+//    constants per tile, shared by the R row blocks, whose result is the start value of the code chain.  No weight is rounded:
 //    the error against 64 bits is that of the result's rounding (fp16 2.1e-4, 2.8e-4 with rounded weights; bf16 1.7e-3, 2.2e-3).
 //  * What bounds it: the copies of the activations, which every workgroup repeats, and HBM.  On layers with one row block per
 //    CU and a long K the copies are most of the traffic of a CU (4096 x 14336 at M = 16: 458 KB beside 115 KB of codes).
@@ -100,11 +99,12 @@ few_rows_kernel(const GemmArgs a, int n_tiles, int m_tiles) {
   }
 
   const Raw raw;
-  Frag centre[Raw::kOddOctets ? 2 : 1], ones;
-  Raw::template centre<0>(centre[0]);
-  if constexpr (Raw::kOddOctets) Raw::template centre<1>(centre[1]);
+  Frag minus, ones;
 #pragma unroll
-  for (int i = 0; i < 4; i++) ones.u[i] = pow2_pair(0);
+  for (int i = 0; i < 4; i++) {
+    minus.u[i] = Raw::kOff;
+    ones.u[i] = pow2_pair(0);
+  }
   auto mma = [](const Frag& x, const Frag& w, float4v c) {
     if constexpr (kBf16)
       return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, x.h), __builtin_bit_cast(bf16x8, w.h), c, 0, 0, 0);
@@ -191,7 +191,7 @@ few_rows_kernel(const GemmArgs a, int n_tiles, int m_tiles) {
         xs[i] = zero4;
 #pragma unroll
         for (int j = 0; j < 4; j++) {
-          off[i] = mma(xf[j][i], centre[Raw::kOddOctets ? (j & 1) : 0], off[i]);
+          if constexpr (!Raw::kCentred) off[i] = mma(xf[j][i], minus, off[i]);
           if constexpr (ZP) xs[i] = mma(xf[j][i], ones, xs[i]);
         }
         if constexpr (ZP && GROUP == -1) xsum[i] += xs[i];

@@ -21,6 +21,8 @@ MORE_ROWS = [(128, 1024, 64, 1, 16), (2048, 1152, 17, 1, 16), (1360, 2176, 48, 1
              (2064, 2176, 50, 2, 32), (4160, 1152, 64, 4, 32)]
 FORMATS = [(2, 128, False), (3, 128, False), (4, 128, False), (6, 128, False), (8, 128, False), (2, -1, True), (3, -1, True),
            (4, 128, True), (6, 128, True), (8, -1, True), (8, 128, True), (4, -1, False)]
+# what the operand of bf16 storage carries besides the code (raw_operand.h; planes at 2 bits: 8)
+BF16_BASE = {2: 8, 3: 8, 4: 16, 6: 128, 8: 0}
 
 
 def layer(bits, group, bf16, zeros, n, k, seed):
@@ -66,39 +68,39 @@ def check(bits, group, bf16, planes, zeros, n, k, m, flags):
     y = run(bits, group, n, k, x.cuda(), packed_of(q, bits, planes), sd, zd, flags, planes).double().cpu().numpy()
     xd = x.double().numpy()
     ref = xd @ exact_weights(q, st, zt, bits, group).T
-    # one rounding of the result, and sums in fp32 of products of codes with up to 1024 (bf16: 128) added to them: their
-    # rounding errors stay below 2^-21 of the sum of the magnitudes
+    # one rounding of the result, and sums in fp32 whose rounding errors stay below 2^-21 of the sum of the magnitudes: code and
+    # zero point around the centre, 2^(b-1) each, on bf16 storage once more twice the base that the operand carries
     scale = np.repeat(st.double().numpy(), k if group == -1 else group, axis=1) * (1 << (8 - bits))
-    reach = np.abs(xd) @ (scale * ((128 if bf16 else 1024) + 2 * (1 << bits))).T
+    reach = np.abs(xd) @ (scale * ((1 << bits) + (2 * BF16_BASE[bits] + (1 << bits) if bf16 else 0))).T
     assert np.all(np.abs(y - ref) <= 2.0 ** (-8 if bf16 else -11) * np.abs(ref) + 2.0 ** -21 * reach + 2.0 ** -24)
 
 
-@pytest.mark.parametrize("planes", (False, True))
-@pytest.mark.parametrize("bits,group,bf16", FORMATS)
-@pytest.mark.parametrize("n,k,m,rows,rows_planes", CASES)
-def test_few_rows(n, k, m, rows, rows_planes, bits, group, bf16, planes):
-    zeros = (n // 16 + bits) % 2 == 0
+# (up to four rows of fp16 at group 128, pre-sliced, are the gemv kernel's, as with a fused prologue)
+@pytest.mark.parametrize("n,k,m,rows,bits,group,bf16,planes", [
+    (n, k, m, min(rows_planes if planes else rows, 4 if bits <= (4 if planes else 6) else 2), bits, group, bf16, planes)
+    for n, k, m, rows, rows_planes in CASES for bits, group, bf16 in FORMATS for planes in (False, True)
+    if m > 4 or planes or bf16 or group != 128])
+def test_few_rows(n, k, m, rows, bits, group, bf16, planes):
     flags = 3 if bf16 else 1
-    most = 4 if bits <= (4 if planes else 6) else 2
-    elsewhere = m <= 4 and not planes and not bf16 and group == 128  # (with the fused prologues)
-    assert G.lib().matgptq_few_rows(bits, group, n, k, m, flags, int(planes)) == (0 if elsewhere else min(rows_planes if planes else rows, most))
-    check(bits, group, bf16, planes, zeros, n, k, m, flags)
+    assert G.lib().matgptq_few_rows(bits, group, n, k, m, flags, int(planes)) == rows
+    check(bits, group, bf16, planes, (n // 16 + bits) % 2 == 0, n, k, m, flags)
 
 
-@pytest.mark.parametrize("planes", (False, True))
-@pytest.mark.parametrize("bits,group,bf16", FORMATS)
-@pytest.mark.parametrize("n,k,m,r,rows", MORE_ROWS)
-def test_few_rows_17_to_64(n, k, m, r, rows, bits, group, bf16, planes):
-    flags = 3 if bf16 else 1
-    few = G.lib().matgptq_few_rows(bits, group, n, k, m, flags, int(planes))
+def rows_expected(k, m, r, rows, bits, group, bf16, planes):
     if not bf16 and group == 128 and m >= 32:
-        assert few == 0
-        return
+        return 0
     most = 2 if bits > (4 if planes else 6) else 8 if rows == 32 and bits <= 4 and not planes else 4
     small_tiles = planes and bits > 4 and r == 2 and rows == 16 and 1024 < k and m <= 32
-    assert few == (0 if small_tiles else r if r <= most else 4 if r == 8 and most == 4 and not planes else 0)
-    if few:
-        check(bits, group, bf16, planes, (n // 16 + bits) % 2 == 0, n, k, m, flags)
+    return 0 if small_tiles else r if r <= most else 4 if r == 8 and most == 4 and not planes else 0
+
+
+@pytest.mark.parametrize("n,k,m,rows,bits,group,bf16,planes", [
+    (n, k, m, rows_expected(k, m, r, rows, *form, planes), *form, planes)
+    for n, k, m, r, rows in MORE_ROWS for form in FORMATS for planes in (False, True) if rows_expected(k, m, r, rows, *form, planes)])
+def test_few_rows_17_to_64(n, k, m, rows, bits, group, bf16, planes):
+    flags = 3 if bf16 else 1
+    assert G.lib().matgptq_few_rows(bits, group, n, k, m, flags, int(planes)) == rows
+    check(bits, group, bf16, planes, (n // 16 + bits) % 2 == 0, n, k, m, flags)
 
 
 @pytest.mark.parametrize("planes", (False, True))
@@ -133,16 +135,42 @@ def test_infinities_nan_and_the_largest_numbers(n, m, row_blocks, bits, group, b
         assert np.max(np.abs(y[row][ok] - ref[row][ok]), initial=0) <= (1e-2 if bf16 else 2e-3) * np.max(np.abs(ref[row][ok]), initial=1e-30)
 
 
-def test_exact_on_integers():
-    # scales 0 and 1, integer activations: every sum is a whole number below 2^24
+@pytest.mark.parametrize("planes", (False, True))
+@pytest.mark.parametrize("bits,group,bf16", [(b, g, bf16) for b in (2, 3, 4, 6, 8) for g in (128, -1) for bf16 in (False, True)])
+@pytest.mark.parametrize("n,k", [(96, 4224), (4112, 2176)])
+def test_exact_on_integers(n, k, bits, group, bf16, planes):
+    # scales 0 and 1, integer activations: every sum is a whole number below 2^24, and is rounded once
     rng = np.random.default_rng(3)
-    n, k = 96, 4224
-    for bits in (2, 3, 4, 6, 8):
-        codes = rng.integers(0, 1 << bits, (n, k), dtype=np.uint8)
-        scales = np.round(rng.random((n, k // 128))).astype(np.float16)
-        pk, sd = G.pack_device(codes, bits, from_master=False), G.reorder_device(scales, n, k, 128)
-        w = o.dequantize_kernel_form(codes, scales, bits, 128)
-        for m in (5, 8, 16):
-            x = np.round(rng.standard_normal((m, k))).astype(np.float16)
-            y = G.gemm(bits, 128, n, k, G.to_dev(x), pk, sd, None).cpu().numpy()
-            assert np.array_equal(y.view(np.uint16), o.linear_f64(x, w).astype(np.float16).view(np.uint16)), (bits, m)
+    dt = torch.bfloat16 if bf16 else torch.float16
+    q = rng.integers(0, 256, (n, k), dtype=np.uint8)
+    scales = torch.from_numpy(np.round(rng.random((n, 1 if group == -1 else k // 128)))).to(dt)
+    sd = G.reorder_device(scales.view(torch.float16).numpy(), n, k, group)
+    packed = packed_of(q, bits, planes)
+    w = torch.from_numpy(exact_weights(q, scales, torch.full_like(scales, 128), bits, group))
+    for m in (5, 8, 16, 27):
+        x = torch.from_numpy(np.round(rng.standard_normal((m, k)))).to(dt)
+        y = run(bits, group, n, k, x.cuda(), packed, sd, None, 3 if bf16 else 1, planes).cpu()
+        assert torch.equal(y, (x.double() @ w.T).to(dt)), m
+
+
+@pytest.mark.parametrize("planes", (False, True))
+@pytest.mark.parametrize("bits,group,bf16", FORMATS)
+@pytest.mark.parametrize("m", (11, 28))
+def test_a_column_of_outliers_leaves_rows_whose_weight_there_is_zero(m, bits, group, bf16, planes):
+    # (products with it are zero: nothing of its size may take part in the sums.  bf16: the base of the operand does, at 2^-21
+    # of its magnitude as above, which stays below the rounding of an output)
+    n, k, col = 272, 2176, 300
+    q, st, _, sd, _ = layer(bits, group, bf16, False, n, k, seed=bits)
+    q[:, col] = 128
+    x = torch.from_numpy(o.make_activations(m, k, seed=m)).to(st.dtype)
+    x[:, col] = 1e4 * x.float().std()
+    y = run(bits, group, n, k, x.cuda(), packed_of(q, bits, planes), sd, None, 3 if bf16 else 1, planes).double().cpu().numpy()
+    assert G.lib().matgptq_few_rows(bits, group, n, k, m, 3 if bf16 else 1, int(planes)) == 1
+    ref = x.double().numpy() @ exact_weights(q, st, torch.full_like(st, 128), bits, group).T
+    scale = np.repeat(st.double().numpy(), k if group == -1 else group, axis=1) * (1 << (8 - bits))
+    rest = np.abs(x.double().numpy())
+    rest[:, col] = 0
+    reach = rest @ (scale * (1 << bits)).T
+    if bf16:
+        reach += np.abs(x.double().numpy()) @ (scale * (2 * BF16_BASE[bits] + (1 << bits))).T
+    assert np.all(np.abs(y - ref) <= 2.0 ** (-8 if bf16 else -11) * np.abs(ref) + 2.0 ** -21 * reach + 2.0 ** -24)
