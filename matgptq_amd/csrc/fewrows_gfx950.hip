@@ -271,8 +271,26 @@ few_rows_kernel(const GemmArgs a, int n_tiles, int m_tiles) {
     if (t + 1 < walk) tile(t + 1, Odd{}, std::false_type{});
   }
 
-  // Infinities and NaN among the activations (and bf16 numbers beyond 2^120) have met `base` times themselves with the
-  // other sign and left NaN: such a wave forms its sums again, with dequantised weights as the other kernels do.
+  if constexpr (GROUP == -1) {  // the row's one scale and zero point
+#pragma unroll
+    for (int rr = 0; rr < R; rr++) {
+      const int rb = rb_first + rr < a.row_blocks ? rb_first + rr : a.row_blocks - 1;
+      const float s = storage_to_float(a.scales[(size_t)rb * 16 + r16]);
+      const float z = ZP ? 128.0f / kMul - storage_to_float(a.zeros[(size_t)rb * 16 + r16]) * (1.0f / kMul) : 0.f;
+#pragma unroll
+      for (int i = 0; i < MB; i++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          if constexpr (ZP) acc[rr][i][e] = __builtin_fmaf(z, xsum[i][e], acc[rr][i][e]);
+          // (a sum times scale 0 is +0, as a sum of products with it is)
+          acc[rr][i][e] = __builtin_fmaf(s, acc[rr][i][e], 0.f);
+        }
+    }
+  }
+
+  // Infinities and NaN among a row's activations (and bf16 numbers beyond 2^120) have met zero codes, `base` or the zero
+  // point with the other sign and left NaN: a wave with such sums forms them again, with dequantised weights as the
+  // other kernels do.  The sums of the other rows stay as they are: what a row gives does not depend on its neighbours.
   bool finite = true;
 #pragma unroll
   for (int rr = 0; rr < R; rr++)
@@ -280,8 +298,7 @@ few_rows_kernel(const GemmArgs a, int n_tiles, int m_tiles) {
     for (int i = 0; i < MB; i++)
 #pragma unroll
       for (int e = 0; e < 4; e++) finite = finite && __builtin_isfinite(acc[rr][i][e]);
-  const bool again = __builtin_amdgcn_ballot_w64(!finite) != 0;
-  if (again) {
+  if (__builtin_amdgcn_ballot_w64(!finite) != 0) {
     const typename Fmt::Consts unpack;
     const BufRsrc xres = make_rsrc(a.x, x_bytes);
     uint32_t x_off[MB];
@@ -289,13 +306,14 @@ few_rows_kernel(const GemmArgs a, int n_tiles, int m_tiles) {
     for (int i = 0; i < MB; i++) {
       const int row = m0 + i * 16 + xrow;
       x_off[i] = row < a.M ? (uint32_t)row * (uint32_t)a.K * 2u + q * 16 : x_bytes;
-#pragma unroll
-      for (int rr = 0; rr < R; rr++) acc[rr][i] = float4v{0.f, 0.f, 0.f, 0.f};
     }
-    for (int kb = wave; kb < a.k_tiles; kb += kWaves) {
 #pragma unroll
-      for (int rr = 0; rr < R; rr++) {
-        const int rb = rb_first + rr < a.row_blocks ? rb_first + rr : a.row_blocks - 1;
+    for (int rr = 0; rr < R; rr++) {
+      const int rb = rb_first + rr < a.row_blocks ? rb_first + rr : a.row_blocks - 1;
+      float4v again[MB];
+#pragma unroll
+      for (int i = 0; i < MB; i++) again[i] = float4v{0.f, 0.f, 0.f, 0.f};
+      for (int kb = wave; kb < a.k_tiles; kb += kWaves) {
         uint32_t w[Fmt::kWords];
         Fmt::load(make_rsrc(a.packed, w_bytes), (uint32_t)rb * rb_bytes + (uint32_t)kb * tile_bytes, lane, w);
         const size_t g = ((size_t)rb * a.G + (GROUP == -1 ? 0 : kb)) * 16 + r16;
@@ -315,7 +333,7 @@ few_rows_kernel(const GemmArgs a, int n_tiles, int m_tiles) {
             const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(xres, x_off[i], (uint32_t)kb * 256u + J * 64u, 0);
             Frag x;
             x.v = make_uint4(v.x, v.y, v.z, v.w);
-            acc[rr][i] = mma(x, aw, acc[rr][i]);
+            again[i] = mma(x, aw, again[i]);
           }
         };
         one(std::integral_constant<int, 0>{});
@@ -323,27 +341,11 @@ few_rows_kernel(const GemmArgs a, int n_tiles, int m_tiles) {
         one(std::integral_constant<int, 2>{});
         one(std::integral_constant<int, 3>{});
       }
-    }
-#pragma unroll
-    for (int rr = 0; rr < R; rr++)
-#pragma unroll
-      for (int i = 0; i < MB; i++) acc[rr][i] *= 1.0f / kMul;
-  }
-
-  if (GROUP == -1 && !again) {  // the row's one scale and zero point
-#pragma unroll
-    for (int rr = 0; rr < R; rr++) {
-      const int rb = rb_first + rr < a.row_blocks ? rb_first + rr : a.row_blocks - 1;
-      const float s = storage_to_float(a.scales[(size_t)rb * 16 + r16]);
-      const float z = ZP ? 128.0f / kMul - storage_to_float(a.zeros[(size_t)rb * 16 + r16]) * (1.0f / kMul) : 0.f;
 #pragma unroll
       for (int i = 0; i < MB; i++)
 #pragma unroll
-        for (int e = 0; e < 4; e++) {
-          if constexpr (ZP) acc[rr][i][e] = __builtin_fmaf(z, xsum[i][e], acc[rr][i][e]);
-          // (a sum times scale 0 is +0, as a sum of products with it is)
-          acc[rr][i][e] = __builtin_fmaf(s, acc[rr][i][e], 0.f);
-        }
+        for (int e = 0; e < 4; e++)
+          if (!__builtin_isfinite(acc[rr][i][e])) acc[rr][i][e] = again[i][e] * (1.0f / kMul);
     }
   }
 

@@ -105,6 +105,22 @@ def test_few_rows_17_to_64(n, k, m, rows, bits, group, bf16, planes):
 
 @pytest.mark.parametrize("planes", (False, True))
 @pytest.mark.parametrize("bits,group,bf16,zeros", [(4, 128, False, True), (3, -1, False, True), (8, 128, True, False), (6, -1, True, True)])
+@pytest.mark.parametrize("n,m", [(80, 11), (80, 28), (4112, 19)])
+def test_rows_keep_their_bits_whatever_their_neighbours_hold(n, m, bits, group, bf16, zeros, planes):
+    k = 2176
+    q, st, _, sd, zd = layer(bits, group, bf16, zeros, n, k, seed=bits)
+    packed = packed_of(q, bits, planes)
+    x = torch.from_numpy(o.make_activations(m, k, seed=5)).to(st.dtype)
+    alone = run(bits, group, n, k, x.cuda(), packed, sd, zd, 3 if bf16 else 1, planes)
+    x[3, 300], x[3, 2100], x[8, 7] = float("inf"), float("nan"), float("-inf")
+    y = run(bits, group, n, k, x.cuda(), packed, sd, zd, 3 if bf16 else 1, planes)
+    others = [i for i in range(m) if i not in (3, 8)]
+    assert torch.equal(y[others].view(torch.int16), alone[others].view(torch.int16))
+    assert torch.isnan(y[3]).all() and not torch.isfinite(y[8]).all()
+
+
+@pytest.mark.parametrize("planes", (False, True))
+@pytest.mark.parametrize("bits,group,bf16,zeros", [(4, 128, False, True), (3, -1, False, True), (8, 128, True, False), (6, -1, True, True)])
 @pytest.mark.parametrize("n,m,row_blocks", [(80, 11, 1), (80, 28, 1), (4112, 19, 2)])
 def test_infinities_nan_and_the_largest_numbers(n, m, row_blocks, bits, group, bf16, zeros, planes):
     # one wave's columns hold them: rows with one are what dequantised weights give, the others stay finite
