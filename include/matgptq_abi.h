@@ -81,6 +81,8 @@ size_t matgptq_packed_words(int bitwidth, int64_t N, int64_t K);
  *              or NULL: every zero is 128, which is the reference kernel's
  *              symmetric form  (c - 2^(b-1)) * scale * 2^(8-b)
  * x_dev        [M, K] fp16 row-major;  y_dev  [M, N] fp16 row-major
+ * x_dev has to lie on 16 bytes where M is more than 4 (the kernels copy it into LDS in pieces of that size; the torch
+ * operators copy other views first).
  * Any M >= 1 is accepted.  Graph-capturable: no allocation, no host read.
  * With flag bit 0 clear the call ends with hipStreamSynchronize(stream). */
 int matgptq_gemm(int bitwidth, int group_size, int64_t N, int64_t K, int64_t M,

@@ -598,9 +598,12 @@ hipError_t launch_few_rows(int bits, bool bf16, const GemmArgs& a, int g, FewRow
 #undef MATGPTQ_CASE
 }
 
-// Workgroup of the few-rows kernel where a call without a forced variant takes it, else no row blocks.
-FewRows few_rows_of(int bits, int group_size, int64_t N, int64_t K, int64_t M, uint32_t flags, bool master) {
+// Workgroup of the few-rows kernel where a call without a forced variant takes it, else no row blocks.  `x` (or nullptr: as if
+// aligned): the kernel copies the activations into LDS in pieces of 16 bytes; off those, the kernels that ran before it do,
+// of which the gemv kernel loads them into registers.
+FewRows few_rows_of(int bits, int group_size, int64_t N, int64_t K, int64_t M, const void* x, uint32_t flags, bool master) {
   if ((flags & (MATGPTQ_FLAG_VARIANT_MASK | MATGPTQ_FLAG_FLAVOUR_MASK)) != 0 || M > kFewRowsMaxM) return {0, 0};
+  if (reinterpret_cast<uintptr_t>(x) % 16 != 0) return {0, 0};
   return few_rows(bits, group_size, (flags & MATGPTQ_FLAG_BF16) != 0, master, (int)M, (int)(N / 16), (int)(K / 128));
 }
 
@@ -655,7 +658,7 @@ static int run_gemm(int bitwidth, int group_size, int64_t N, int64_t K, int64_t 
   if (!weights_dev || !scales_dev || !x_dev || !y_dev) return MATGPTQ_ENULL;
   Plan p;
   if (int e = make_plan(bitwidth, group_size, N, K, M, zeros_dev != nullptr, flags, &p)) return e;
-  const FewRows few = few_rows_of(bitwidth, group_size, N, K, M, flags, master_planes);
+  const FewRows few = few_rows_of(bitwidth, group_size, N, K, M, x_dev, flags, master_planes);
   if (master_planes && few.row_blocks == 0 && !plan_reads_planes(p, M)) return MATGPTQ_EVARIANT;
   GemmArgs a;
   a.packed = static_cast<const uint32_t*>(weights_dev);
@@ -755,7 +758,7 @@ int matgptq_gemm_prologue(int bitwidth, int group_size, int64_t N, int64_t K, in
 // workspace is given the mid-batch kernel instead (its largest shape for that batch size), which
 // costs 1.05 .. 1.4 times its time on pre-sliced codes but saves the slicing pass - 41 us for the
 // 117 M codes of a 28672 x 4096 layer, more than such a product takes.
-static int master_reads_planes(int bitwidth, int group_size, int64_t N, int64_t K, int64_t M, bool zp,
+static int master_reads_planes(int bitwidth, int group_size, int64_t N, int64_t K, int64_t M, bool zp, const void* x,
                                uint32_t* flags, bool* direct) {
   if (int e = check_problem(bitwidth, group_size, N, K)) return e;
   if (K % 128 != 0) return MATGPTQ_ESHAPE;  // the bit planes have whole tiles only
@@ -763,7 +766,7 @@ static int master_reads_planes(int bitwidth, int group_size, int64_t N, int64_t 
   Plan p;
   if (int e = make_plan(bitwidth, group_size, N, K, M, zp, *flags, &p)) return e;
   *direct = plan_reads_planes(p, M);
-  const bool few = few_rows_of(bitwidth, group_size, N, K, M, *flags, true).row_blocks != 0;
+  const bool few = few_rows_of(bitwidth, group_size, N, K, M, x, *flags, true).row_blocks != 0;
   if (few && M <= 16) {
     *direct = true;
     return MATGPTQ_OK;
@@ -800,7 +803,7 @@ size_t matgptq_gemm_master_workspace_bytes(int bitwidth, int group_size, int64_t
   for (int zp = 0; zp < 2; ++zp) {
     bool direct = false;
     uint32_t f = flags;
-    if (master_reads_planes(bitwidth, group_size, N, K, M, zp != 0, &f, &direct) != MATGPTQ_OK) return 0;
+    if (master_reads_planes(bitwidth, group_size, N, K, M, zp != 0, nullptr, &f, &direct) != MATGPTQ_OK) return 0;
     if (!direct) return matgptq_packed_words(bitwidth, N, K) * 4;
   }
   return 0;
@@ -811,7 +814,7 @@ static int gemm_master_impl(int bitwidth, int group_size, int64_t N, int64_t K, 
                             const void* x_dev, void* y_dev, void* workspace_dev, size_t workspace_bytes,
                             void* stream, uint32_t flags) {
   bool direct = false;
-  if (int e = master_reads_planes(bitwidth, group_size, N, K, M, zeros_dev != nullptr, &flags, &direct)) return e;
+  if (int e = master_reads_planes(bitwidth, group_size, N, K, M, zeros_dev != nullptr, x_dev, &flags, &direct)) return e;
   if (!planes_dev) return MATGPTQ_ENULL;
   if (direct)
     return run_gemm(bitwidth, group_size, N, K, M, planes_dev, scales_dev, zeros_dev, x_dev, y_dev, stream,
@@ -859,7 +862,7 @@ int matgptq_gemm_master_static(int bitwidth, int group_size, int64_t N, int64_t 
                                const void* x_dev, void* y_dev, void* stream, uint32_t flags) {
   bool direct = false;
   uint32_t plan_flags = flags;  // (gemm_master_impl decides again from the caller's flags, the same way)
-  if (int e = master_reads_planes(bitwidth, group_size, N, K, M, zeros_dev != nullptr, &plan_flags, &direct)) return e;
+  if (int e = master_reads_planes(bitwidth, group_size, N, K, M, zeros_dev != nullptr, x_dev, &plan_flags, &direct)) return e;
   void* ws = nullptr;
   size_t need = 0;
   if (!direct) {
@@ -933,7 +936,7 @@ int matgptq_midbatch_buffers(int bitwidth, int group_size, int64_t N, int64_t K,
 int matgptq_few_rows(int bitwidth, int group_size, int64_t N, int64_t K, int64_t M, uint32_t flags, int master) {
   if (int e = check_problem(bitwidth, group_size, N, K)) return e;
   if (M <= 0) return MATGPTQ_ESIZE;
-  return few_rows_of(bitwidth, group_size, N, K, M, flags, master != 0).row_blocks;
+  return few_rows_of(bitwidth, group_size, N, K, M, nullptr, flags, master != 0).row_blocks;
 }
 
 int matgptq_pack_device(const uint8_t* codes_dev, int64_t N, int64_t K, int bitwidth,

@@ -200,7 +200,7 @@ Tensor matmul_impl(const Tensor& input, const Tensor& weights, const Tensor& sca
               "matmul_matgptq: input must be (..., batch, n_in_features)");
   // the reference reads the input as if it were contiguous (bindings.cpp:171-186): a strided
   // view (a slice of a fused projection, a transposed batch) is compacted first
-  const Tensor input_c = input.contiguous();
+  Tensor input_c = input.contiguous();
   const int64_t groups = group_size == -1 ? 1 : n_in_features / group_size;
   TORCH_CHECK(scales.is_contiguous() && scales.numel() == n_out_features * groups,
               "matgptq_scales has the wrong size");
@@ -221,6 +221,8 @@ Tensor matmul_impl(const Tensor& input, const Tensor& weights, const Tensor& sca
   c10::hip::HIPGuardMasqueradingAsCUDA guard(dev);
   Tensor out = torch::empty({m, n_out_features}, input.options());
   if (m == 0) return out;
+  // (a view that starts off 16 bytes: most kernels copy the activations into LDS in pieces of that size)
+  if (reinterpret_cast<uintptr_t>(input_c.data_ptr()) % 16 != 0) input_c = input_c.clone();
   const uint32_t flags = (uint32_t)feature_flag | MATGPTQ_FLAG_ASYNC;
   int code;
   if (master) {

@@ -170,6 +170,25 @@ def test_exact_on_integers(n, k, bits, group, bf16, planes):
 
 
 @pytest.mark.parametrize("planes", (False, True))
+@pytest.mark.parametrize("bits,group,bf16", [(4, 128, False), (3, 128, True), (8, -1, False)])
+@pytest.mark.parametrize("off", (1, 4, 7))
+def test_activations_off_16_bytes(off, bits, group, bf16, planes):
+    n, k = 272, 1152
+    q, st, _, sd, zd = layer(bits, group, bf16, True, n, k, seed=bits)
+    packed, flags = packed_of(q, bits, planes), 3 if bf16 else 1
+    op = torch.ops.matgptq_cuda.matmul_matgptq_master if planes else torch.ops.matgptq_cuda.matmul_matgptq_zp
+    for m in (1, 3, 6, 8, 16, 24, 64, 300):
+        x = torch.from_numpy(o.make_activations(m, k, seed=m)).to(st.dtype).cuda()
+        view = torch.cat((x.new_zeros(off), x.reshape(-1)))[off:].view(m, k)
+        assert view.data_ptr() % 16 == 2 * off
+        call = lambda t: op(t, packed.view(torch.uint32), sd.view(st.dtype), zd.view(st.dtype), n, k, bits, group, flags)
+        assert torch.equal(call(view), call(x)), m
+        if m <= 8:  # without the operator's copy: the gemv kernel, which loads them into registers
+            assert torch.equal(run(bits, group, n, k, view, packed, sd, zd, flags, planes),
+                               run(bits, group, n, k, x, packed, sd, zd, flags | (101 << 8), planes)), m
+
+
+@pytest.mark.parametrize("planes", (False, True))
 @pytest.mark.parametrize("bits,group,bf16", FORMATS)
 @pytest.mark.parametrize("m", (11, 28))
 def test_a_column_of_outliers_leaves_rows_whose_weight_there_is_zero(m, bits, group, bf16, planes):
