@@ -217,8 +217,7 @@ int matgptq_gemm_master_static(int bitwidth, int group_size, int64_t N, int64_t 
                                const void *planes_dev, const void *scales_dev, const void *zeros_dev,
                                const void *x_dev, void *y_dev, void *stream, uint32_t flags);
 
-/* Human-readable name of the kernel variant matgptq_gemm would launch; where matgptq_few_rows() is not 0 that kernel runs
- * instead, and the name is the one of the forced variant next to it. */
+/* Human-readable name of the kernel variant matgptq_gemm would launch. */
 int matgptq_describe_plan(int bitwidth, int group_size, int64_t N, int64_t K, int64_t M,
                           int has_zeros, uint32_t flags, char *buf, size_t buf_len);
 /* Activation buffers (1 or 2) of the mid-batch kernel that matgptq_gemm would launch; 0 where it launches another one,

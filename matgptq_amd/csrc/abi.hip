@@ -373,7 +373,7 @@ int make_plan(int bits, int group_size, int64_t N, int64_t K, int64_t M, bool zp
   } else if (flavour == 0 && M > kGemvMaxM &&
              !(bits == 8 && group_size != 32 && !(flags & MATGPTQ_FLAG_BF16) && row_blocks >= 1024)) {
     // Five to sixteen batch rows.  Automatic calls at group sizes 128 and -1 run the few-rows kernel in front of this plan
-    // (few_rows_of), so these lines and the eight-row ones below decide group size 32 and what the plan's name says.
+    // (few_rows_of), so these lines and the eight-row ones below decide group size 32 and activations off 16 bytes.
     // Every decode workgroup stages the whole batch of activations (scaled copies, written by the vector
     // ALU), which grows with M and K, while the mid-batch kernel copies them into LDS
     // asynchronously.  Measured on MI355X (Llama-3-8B layers, 2, 4 and 8 bits, M = 5 .. 16, weights
@@ -906,7 +906,11 @@ int matgptq_describe_plan(int bitwidth, int group_size, int64_t N, int64_t K, in
   if (M <= 0) return MATGPTQ_ESIZE;
   Plan p;
   if (int e = make_plan(bitwidth, group_size, N, K, M, has_zeros != 0, flags, &p)) return e;
-  if (p.gemv)
+  const FewRows few = few_rows_of(bitwidth, group_size, N, K, M, nullptr, flags, false);
+  if (few.row_blocks != 0)
+    snprintf(buf, buf_len, "fewrows b%d g%d zp%d R%d rows%d", bitwidth, group_size, has_zeros ? 1 : 0, few.row_blocks,
+             few_rows_held(few, (int)M));
+  else if (p.gemv)
     snprintf(buf, buf_len, "gemv b%d g%d zp%d T%d R%d W%d pad%zu", bitwidth, group_size, has_zeros ? 1 : 0,
              kGemvShapes[p.shape][0], p.R, p.W, p.pad);
   else if (p.decode)
@@ -927,7 +931,7 @@ int matgptq_midbatch_buffers(int bitwidth, int group_size, int64_t N, int64_t K,
   if (M <= 0) return MATGPTQ_ESIZE;
   Plan p;
   if (int e = make_plan(bitwidth, group_size, N, K, M, has_zeros != 0, flags, &p)) return e;
-  if (!p.skinny) return 0;
+  if (!p.skinny || few_rows_of(bitwidth, group_size, N, K, M, nullptr, flags, false).row_blocks != 0) return 0;
   if ((flags & MATGPTQ_FLAG_VARIANT_MASK) == 0 && K / 128 <= 8) return 1;
   return midbatch_two_buffers(bitwidth, (flags & MATGPTQ_FLAG_BF16) != 0, group_size, has_zeros != 0, p.R, p.mb, false,
                               (int)(K / 128), (int)M, (int)(N / 16)) ? 2 : 1;

@@ -13,6 +13,9 @@ struct FewRows {
   int row_blocks, batch_rows;
 };
 
+// Batch rows that a workgroup really holds for a call of M.
+constexpr int few_rows_held(FewRows f, int M) { return M <= 4 ? 4 : M <= 8 ? 8 : f.batch_rows; }
+
 // Most row blocks of 16 weight rows per workgroup that the registers hold, by the format and the batch rows per workgroup.
 constexpr int few_rows_most_row_blocks(int bits, bool master, int rows) {
   if (bits > (master ? 4 : 6)) return 2;

@@ -18,13 +18,13 @@ LLAMA70B = {"qkv": (10240, 8192), "o": (8192, 8192), "gate_up": (57344, 8192), "
 # take four row blocks per workgroup on the layer with many rows at four batch rows: `{r}`)
 SMALL_BATCH_PLANS = {
     "qkv": {2: "gemv b{b} g128 zp1 T4 R1 W8 pad0", 4: "gemv b{b} g128 zp1 T4 R2 W8 pad0",
-            8: "gemv b{b} g128 zp1 T4 R2 W8 pad0", 16: "midbatch b{b} g128 zp1 R2 mb1"},
+            8: "fewrows b{b} g128 zp1 R2 rows8", 16: "fewrows b{b} g128 zp1 R2 rows16"},
     "o": {2: "gemv b{b} g128 zp1 T4 R1 W8 pad0", 4: "gemv b{b} g128 zp1 T4 R1 W8 pad0",
-          8: "gemv b{b} g128 zp1 T4 R1 W8 pad0", 16: "midbatch b{b} g128 zp1 R1 mb1"},
+          8: "fewrows b{b} g128 zp1 R1 rows8", 16: "fewrows b{b} g128 zp1 R1 rows16"},
     "gate_up": {2: "gemv b{b} g128 zp1 T4 R1 W8 pad0", 4: "gemv b{b} g128 zp1 T4 R{r} W8 pad0",
-                8: "midbatch b{b} g128 zp1 R4 mb1", 16: "midbatch b{b} g128 zp1 R4 mb1"},
+                8: "fewrows b{b} g128 zp1 R4 rows8", 16: "fewrows b{b} g128 zp1 R4 rows16"},
     "down": {2: "gemv b{b} g128 zp1 T4 R1 W16 pad0", 4: "gemv b{b} g128 zp1 T4 R1 W16 pad0",
-             8: "gemv b{b} g128 zp1 T4 R1 W16 pad0", 16: "midbatch b{b} g128 zp1 R1 mb1"},
+             8: "fewrows b{b} g128 zp1 R1 rows8", 16: "fewrows b{b} g128 zp1 R1 rows16"},
 }
 
 

@@ -50,9 +50,9 @@ def test_gemv_group_sizes_32_and_per_row(b, zp, g):
     lay = G.Layer(n, k, b, g, seed=60 + b, zero_points=zp)
     for m in (1, 2, 3, 4):
         x = o.make_activations(m, k, seed=m + b, outlier_frac=0.01)
-        assert _lib.describe_plan(b, g, n, k, m, zp).startswith("gemv")
         G.assert_close_to_oracle(lay.run(x), x, lay.w, f"default b={b} g={g} zp={zp} M={m}")
         for shape in (1, 2):
+            assert _lib.describe_plan(b, g, n, k, m, zp, gemv_flags(shape)).startswith("gemv")
             for waves in (0, 1, 3, 16):
                 y = lay.run(x, flags=gemv_flags(shape, waves))
                 G.assert_close_to_oracle(y, x, lay.w, f"b={b} g={g} zp={zp} M={m} shape={shape} W={waves}")
@@ -87,7 +87,7 @@ def test_gemv_group_sizes_agree_with_the_decode_kernel():
         lay = G.Layer(n, k, b, g, seed=11)
         for m in (1, 3):
             x = o.make_activations(m, k, seed=m)
-            a = lay.run(x).astype(np.float64)
+            a = lay.run(x, flags=gemv_flags(1)).astype(np.float64)
             c = lay.run(x, flags=1 | (1 << 16)).astype(np.float64)  # burst flavour: the decode kernel
             assert _lib.describe_plan(b, g, n, k, m, True, 1 | (1 << 16)).startswith("decode")
             assert np.max(np.abs(a - c)) <= 2.0 ** -9 * np.max(np.abs(c))
@@ -104,9 +104,8 @@ def test_gemv_five_to_eight_batch_rows(b, zp, g):
     lay = G.Layer(n, k, b, g, seed=40 + b, zero_points=zp)
     for m in (5, 6, 7, 8):
         x = o.make_activations(m, k, seed=m + b, outlier_frac=0.01)
-        assert _lib.describe_plan(b, g, n, k, m, zp).startswith("gemv")
-        G.assert_close_to_oracle(lay.run(x), x, lay.w, f"default b={b} g={g} zp={zp} M={m}")
         for shape in (1, 2):
+            assert _lib.describe_plan(b, g, n, k, m, zp, gemv_flags(shape)).startswith("gemv")
             for waves in (0, 1, 3, 16):
                 if shape == 2 and waves == 16:  # more LDS than a CU has
                     with pytest.raises(_lib.MatGPTQError, match="variant"):
@@ -146,8 +145,8 @@ def test_gemv_five_to_eight_batch_rows_exact_in_the_reference_test_regime():
 
 
 def test_gemv_is_not_taken_outside_its_domain():
-    assert _lib.describe_plan(4, 128, 4096, 4096, 9, True).split()[0] in ("decode-burst", "midbatch")
-    assert _lib.describe_plan(4, 128, 28672, 4096, 5, True).split()[0] in ("decode-burst", "midbatch")
+    assert _lib.describe_plan(4, 128, 4096, 4096, 9, True).startswith("fewrows")
+    assert _lib.describe_plan(4, 128, 28672, 4096, 5, True).startswith("fewrows")
     assert _lib.describe_plan(4, 32, 4096, 4096, 5, True).split()[0].startswith(("decode", "midbatch"))
     with pytest.raises(_lib.MatGPTQError, match="variant"):  # group 32: shapes 1 and 2 only
         G.Layer(32, 256, 4, 32, seed=1).run(o.make_activations(1, 256, seed=1), flags=gemv_flags(0))

@@ -99,9 +99,9 @@ def test_midbatch_kernel_reads_the_planes_itself(b, g, m):
     planes = planes_device(q)
     sc, zr = G.reorder_device(s, n, k, g), G.reorder_device(z, n, k, g)
     x = o.make_activations(m, k, seed=m)
-    # (five to eight batch rows of a layer this small go to the gemv kernel: the mid-batch kernel is
-    # forced for them)
-    flags = 1 | (82 << 8) if 5 <= m <= 8 and g != 32 else 1
+    # (up to sixteen batch rows go to the few-rows kernel but for group 32: the mid-batch kernel is forced for them)
+    flags = 1 | (82 << 8) if m <= 16 and g != 32 else 1
+    assert G.lib().matgptq_few_rows(b, g, n, k, m, flags, 1) == 0
     assert _lib.describe_plan(b, g, n, k, m, True, flags).startswith("midbatch")
     for zeros in (zr, None):
         y, need = gemm_master(b, g, n, k, G.to_dev(x), planes, sc, zeros, flags=flags, workspace=None)
@@ -123,13 +123,15 @@ def test_gemv_kernel_reads_the_planes_at_five_to_eight_rows(b, g, m, n):
     planes = planes_device(q)
     sc, zr = G.reorder_device(s, n, k, g), G.reorder_device(z, n, k, g)
     x = o.make_activations(m, k, seed=m)
-    assert _lib.describe_plan(b, g, n, k, m, True).startswith("gemv")
+    flags = 1 | ((102 if n // 16 >= 320 else 101) << 8)  # (forced: the few-rows kernel takes these calls)
+    assert _lib.describe_plan(b, g, n, k, m, True, flags).startswith("gemv")
+    assert G.lib().matgptq_few_rows(b, g, n, k, m, flags, 1) == 0
     for zeros in (zr, None):
-        y, need = gemm_master(b, g, n, k, G.to_dev(x), planes, sc, zeros, workspace=None)
+        y, need = gemm_master(b, g, n, k, G.to_dev(x), planes, sc, zeros, flags=flags, workspace=None)
         assert need == 0
         zz = z if zeros is not None else np.full_like(z, 128)
         G.assert_close_to_oracle(y, x, o.dequantize(q, s, zz, b, g), f"planes, gemv b={b} g={g} M={m}")
-        y2 = G.gemm(b, g, n, k, G.to_dev(x), G.pack_device(q, b, True), sc, zeros).cpu().numpy()
+        y2 = G.gemm(b, g, n, k, G.to_dev(x), G.pack_device(q, b, True), sc, zeros, flags=flags).cpu().numpy()
         # (the pre-sliced 2-bit tiles pair their octets differently and the 6- and 8-bit ones multiply their two
         # code segments apart: another order of the fp32 sums, so close, not identical)
         assert np.max(np.abs(y.astype(np.float64) - y2)) <= 2.0 ** -9 * np.max(np.abs(y2.astype(np.float64)))
@@ -281,7 +283,8 @@ def test_master_gemm_in_a_graph():
 @pytest.mark.parametrize("b,m", [(3, 3), (2, 4), (3, 4), (2, 3)])
 def test_three_and_four_rows_on_many_row_layers_read_the_planes(b, m):
     # the pre-sliced plan here is the gemv kernel with four row blocks per workgroup, which is not built
-    # for planes: on planes the two-row-block shape serves the call, without a workspace
+    # for planes: on planes the few-rows kernel serves the call, and where the activations lie off 16 bytes the
+    # gemv kernel's two-row-block shape, both without a workspace
     n, k, g = 16384, 512, 128
     assert "R4" in _lib.describe_plan(b, g, n, k, m, True)
     q, s, z = o.make_layer(n, k, g, seed=b * 7 + m)
@@ -292,4 +295,9 @@ def test_three_and_four_rows_on_many_row_layers_read_the_planes(b, m):
         y, need = gemm_master(b, g, n, k, G.to_dev(x), planes, sc, zeros, workspace=None)
         assert need == 0
         zz = z if zeros is not None else np.full_like(z, 128)
-        G.assert_close_to_oracle(y, x, o.dequantize(q, s, zz, b, g), f"planes, gemv R2 b={b} M={m}")
+        G.assert_close_to_oracle(y, x, o.dequantize(q, s, zz, b, g), f"planes b={b} M={m}")
+        two, _ = gemm_master(b, g, n, k, G.to_dev(x), planes, sc, zeros, flags=1 | (102 << 8), workspace=None)
+        view = torch.cat((torch.zeros(3, dtype=torch.float16), torch.from_numpy(x).reshape(-1))).to(G.DEV)[3:].view(m, k)
+        off, need = gemm_master(b, g, n, k, view, planes, sc, zeros, workspace=None)
+        assert need == 0 and np.array_equal(off, two)
+        G.assert_close_to_oracle(two, x, o.dequantize(q, s, zz, b, g), f"planes, gemv R2 b={b} M={m}")

@@ -154,14 +154,15 @@ def test_error_codes():
 
 
 def test_describe_plan_regimes():
-    # batch 1..4: the gemv kernel; five rows on: decode / mid-batch, or the gemv kernel again (below)
+    # batch 1..4: the gemv kernel; five rows on: few rows, at group 32 mid-batch
     assert _lib.describe_plan(4, 128, 4096, 4096, 1) == "gemv b4 g128 zp0 T4 R1 W8 pad0"
     assert _lib.describe_plan(4, 128, 4096, 14336, 1, True) == "gemv b4 g128 zp1 T4 R1 W16 pad0"
     assert _lib.describe_plan(4, 128, 4096, 4096, 4, True) == "gemv b4 g128 zp1 T4 R1 W8 pad0"
     assert _lib.describe_plan(4, 128, 28672, 4096, 4, True) == "gemv b4 g128 zp1 T4 R2 W8 pad0"
     assert _lib.describe_plan(4, 128, 4096, 4096, 1, True, 1 | (1 << 16)).startswith("decode-burst")
     assert _lib.describe_plan(4, 32, 4096, 4096, 1) == "gemv b4 g32 zp0 T4 R1 W8 pad0"
-    assert _lib.describe_plan(4, -1, 4096, 4096, 4) == "gemv b4 g-1 zp0 T4 R1 W8 pad0"
+    assert _lib.describe_plan(4, -1, 4096, 14336, 4) == "gemv b4 g-1 zp0 T4 R1 W16 pad0"
+    assert _lib.describe_plan(4, -1, 4096, 4096, 4) == "fewrows b4 g-1 zp0 R1 rows4"
     assert _lib.describe_plan(2, 128, 28672, 4096, 1, True) == "gemv b2 g128 zp1 T4 R2 W8 pad0"
     assert _lib.describe_plan(3, 128, 28672, 4096, 4, True) == "gemv b3 g128 zp1 T4 R4 W8 pad0"
     assert _lib.describe_plan(3, 128, 6144, 4096, 4, True) == "gemv b3 g128 zp1 T4 R2 W8 pad0"
@@ -172,26 +173,28 @@ def test_describe_plan_regimes():
     assert _lib.describe_plan(2, 128, 28672, 4096, 2, True) == "gemv b2 g128 zp1 T4 R2 W8 pad0"
     assert _lib.describe_plan(4, 128, 28672, 4096, 3, True) == "gemv b4 g128 zp1 T4 R2 W8 pad0"
     assert _lib.describe_plan(4, 32, 4096, 4096, 5).startswith(("decode", "midbatch"))
-    # five to sixteen rows: the mid-batch kernel, except at 8 bits on fp16 storage with one scale per
-    # tile or row, on layers with many rows (two row blocks per workgroup only)
+    # five to sixteen rows: the mid-batch kernel at group 32, else the few-rows kernel, with as many row blocks per workgroup
+    # as leave about 160 workgroups
     assert _lib.describe_plan(4, 32, 28672, 4096, 8, True) == "midbatch b4 g32 zp1 R2 mb1"
     assert _lib.describe_plan(4, 32, 28672, 4096, 5, True) == "midbatch b4 g32 zp1 R2 mb1"
     assert _lib.describe_plan(8, 32, 28672, 4096, 8, True) == "midbatch b8 g32 zp1 R2 mb1"
     assert _lib.describe_plan(6, 32, 28672, 4096, 16, True) == "midbatch b6 g32 zp1 R2 mb1"
-    assert _lib.describe_plan(8, 128, 28672, 4096, 8, True, 3) == "midbatch b8 g128 zp1 R2 mb1"  # bf16
-    assert _lib.describe_plan(8, 128, 28672, 4096, 5, True).startswith("decode")
-    assert _lib.describe_plan(8, -1, 28672, 4096, 16, False).startswith("decode")
-    assert _lib.describe_plan(4, 128, 28672, 4096, 5, True) == "midbatch b4 g128 zp1 R4 mb1"
-    # five to eight rows on layers with at most 512 row blocks: the gemv kernel's instantiation for eight
-    # batch rows (one scale per tile or row; two row blocks per workgroup from 320 row blocks on)
-    assert _lib.describe_plan(8, 128, 4096, 4096, 5, True) == "gemv b8 g128 zp1 T4 R1 W8 pad0"
-    assert _lib.describe_plan(4, 128, 4096, 14336, 8, True) == "gemv b4 g128 zp1 T4 R1 W16 pad0"
-    assert _lib.describe_plan(4, -1, 6144, 4096, 6, False) == "gemv b4 g-1 zp0 T4 R2 W8 pad0"
-    assert _lib.describe_plan(4, 128, 8192, 28672, 8, True) == "gemv b4 g128 zp1 T4 R2 W15 pad0"  # (LDS: fifteen waves)
-    assert _lib.describe_plan(6, 128, 8192, 8192, 8, True) == "midbatch b6 g128 zp1 R2 mb1"
-    assert _lib.describe_plan(6, 128, 6144, 4096, 8, True) == "gemv b6 g128 zp1 T4 R2 W8 pad0"
-    assert _lib.describe_plan(4, 128, 10240, 8192, 8, True).startswith("midbatch")
-    assert _lib.describe_plan(4, 128, 4096, 4096, 9, True) == "midbatch b4 g128 zp1 R1 mb1"
+    assert _lib.describe_plan(8, 128, 28672, 4096, 8, True, 3) == "fewrows b8 g128 zp1 R2 rows8"  # bf16
+    assert _lib.describe_plan(8, 128, 28672, 4096, 5, True) == "fewrows b8 g128 zp1 R2 rows8"
+    assert _lib.describe_plan(8, -1, 28672, 4096, 16, False) == "fewrows b8 g-1 zp0 R2 rows16"
+    assert _lib.describe_plan(4, 128, 28672, 4096, 5, True) == "fewrows b4 g128 zp1 R4 rows8"
+    assert _lib.describe_plan(8, 128, 4096, 4096, 5, True) == "fewrows b8 g128 zp1 R1 rows8"
+    assert _lib.describe_plan(4, 128, 4096, 14336, 8, True) == "fewrows b4 g128 zp1 R1 rows8"
+    assert _lib.describe_plan(4, -1, 6144, 4096, 6, False) == "fewrows b4 g-1 zp0 R2 rows8"
+    assert _lib.describe_plan(4, 128, 10240, 8192, 8, True) == "fewrows b4 g128 zp1 R4 rows8"
+    assert _lib.describe_plan(4, 128, 4096, 4096, 9, True) == "fewrows b4 g128 zp1 R1 rows16"
+    # fewer and more rows: only where it was measured ahead
+    assert _lib.describe_plan(4, 128, 256, 1024, 2, True, 3) == "fewrows b4 g128 zp1 R1 rows4"
+    assert _lib.describe_plan(4, 128, 4096, 1024, 17, True) == "fewrows b4 g128 zp1 R1 rows16"
+    assert _lib.describe_plan(4, -1, 28672, 4096, 30, True) == "fewrows b4 g-1 zp1 R8 rows32"
+    # the gemv kernel's instantiation for eight batch rows, forced (fifteen waves: LDS)
+    assert _lib.describe_plan(4, -1, 6144, 4096, 6, False, 1 | (102 << 8)) == "gemv b4 g-1 zp0 T4 R2 W8 pad0"
+    assert _lib.describe_plan(4, 128, 8192, 28672, 8, True, 1 | (102 << 8)) == "gemv b4 g128 zp1 T4 R2 W15 pad0"
     assert _lib.describe_plan(8, 32, 4096, 4096, 5, True) == "midbatch b8 g32 zp1 R1 mb1"
     assert _lib.describe_plan(4, 128, 8192, 8192, 2048).startswith("prefill")
     with pytest.raises(RuntimeError):
@@ -200,10 +203,9 @@ def test_describe_plan_regimes():
         _lib.describe_plan(4, 128, 4096, 4096, 1, True, 1 | (100 << 8) | (17 << 18))  # more than 16 waves
     with pytest.raises(RuntimeError):
         _lib.describe_plan(4, 128, 4096, 4096, 1, True, 1 | (100 << 8) | (41 << 23))  # more LDS than a CU has
-    assert _lib.describe_plan(8, 128, 28672, 4096, 16, True).startswith("decode")
-    assert _lib.describe_plan(4, 128, 28672, 4096, 16, True) == "midbatch b4 g128 zp1 R4 mb1"
+    assert _lib.describe_plan(8, 128, 28672, 4096, 16, True) == "fewrows b8 g128 zp1 R2 rows16"
+    assert _lib.describe_plan(4, 128, 28672, 4096, 16, True) == "fewrows b4 g128 zp1 R4 rows16"
     # small layers: the mid-batch kernel (K split inside the workgroup) from a few rows on
-    assert _lib.describe_plan(4, 128, 4096, 4096, 16, True).startswith("midbatch")
     assert _lib.describe_plan(4, 32, 4096, 14336, 5, True).startswith("midbatch")
     assert _lib.describe_plan(3, 32, 16, 1024, 17).startswith("midbatch")
     assert _lib.describe_plan(4, 128, 4096, 4096, 128, True) == "midbatch b4 g128 zp1 R4 mb2"
@@ -342,11 +344,11 @@ def test_planner_takes_64_row_split_tiles_where_128_row_ones_leave_half_of_the_c
 def test_planner_gives_eight_row_blocks_to_32_batch_rows_on_layers_with_many_rows():
     # the mid-batch kernel with eight row blocks and 32 batch rows per workgroup where that leaves 200 workgroups
     assert _lib.describe_plan(4, 128, 28672, 4096, 32, True) == "midbatch b4 g128 zp1 R8 mb2"
-    assert _lib.describe_plan(2, 128, 28672, 4096, 24, True) == "midbatch b2 g128 zp1 R8 mb2"
-    assert _lib.describe_plan(4, 128, 28672, 4096, 32, True, 3) == "midbatch b4 g128 zp1 R8 mb2"  # bf16 storage
+    assert _lib.describe_plan(2, 128, 28672, 4096, 32, True) == "midbatch b2 g128 zp1 R8 mb2"
+    assert _lib.describe_plan(4, 128, 28672, 4096, 32, True, 3) == "fewrows b4 g128 zp1 R8 rows32"  # bf16 storage
     assert _lib.describe_plan(4, 128, 10240, 8192, 32, True) == "midbatch b4 g128 zp1 R4 mb2"     # 80 workgroups only
     assert _lib.describe_plan(6, 128, 28672, 4096, 32, True) == "midbatch b6 g128 zp1 R4 mb2"     # registers
-    assert _lib.describe_plan(4, 128, 28672, 4096, 16, True) == "midbatch b4 g128 zp1 R4 mb1"
+    assert _lib.describe_plan(4, 128, 28672, 4096, 31, True) == "fewrows b4 g128 zp1 R8 rows32"   # below 32 rows
 
 
 def test_planner_keeps_group_32_with_zero_points_off_the_largest_ring_tile():
@@ -413,9 +415,8 @@ def test_header_is_plain_c(tmp_path):
 
 
 def test_planner_answers_every_valid_shape_within_its_kernels_domains():
-    # seeded random problems: a plan for each, the gemv kernel only up to eight batch rows (five to
-    # eight: one scale per tile or row, at most 512 row blocks, waves within the LDS of a CU), the
-    # mid-batch kernel from five rows on, the large-batch tiles from seventeen
+    # seeded random problems: a plan for each, the gemv kernel only up to four batch rows, the few-rows kernel up to 64
+    # with one scale per tile or row, the mid-batch kernel from five rows on, the large-batch tiles from seventeen
     import random
     import re
     rnd = random.Random(7)
@@ -433,19 +434,14 @@ def test_planner_answers_every_valid_shape_within_its_kernels_domains():
         kind = plan.split()[0]
         seen.add(kind)
         if kind == "gemv":
-            assert m <= 8, plan
-            w, r, t = (int(re.search(rf" {c}(\d+)", plan).group(1)) for c in "WRT")
-            assert 1 <= w <= 16, plan
-            if m > 4:
-                assert g != 32 and n // 16 <= 512, plan
-                assert w * (8 * (t * 256 + 16) + 256 + 64 * t + r * 1024) <= 160 * 1024, plan
+            assert m <= 4 and 1 <= int(re.search(r" W(\d+)", plan).group(1)) <= 16, plan
         elif kind == "midbatch":
             assert m > 4, plan
+        elif kind == "fewrows":
+            assert g != 32 and m <= 64, plan
         elif kind == "prefill":
             assert m > 16, plan
-        else:
-            assert kind.startswith("decode") and m <= 16, plan
-    assert {"gemv", "midbatch", "prefill"} <= seen
+    assert seen == {"gemv", "fewrows", "midbatch", "prefill"}
 
 
 def test_midbatch_buffers_at_the_edges_of_the_rule():
@@ -455,7 +451,7 @@ def test_midbatch_buffers_at_the_edges_of_the_rule():
     def forced(row_blocks_sel, batch_sel):
         return (80 + row_blocks_sel + 3 * batch_sel) << 8
 
-    assert buffers(4, 128, 4096, 4096, 1, 1, plain) == 0        # another kernel
+    assert [buffers(4, 128, 4096, 4096, m, 1, plain) for m in (1, 16, 128, 2048)] == [0, 0, 1, 0]  # 0: another kernel
     assert buffers(5, 128, 4096, 4096, 16, 1, plain) < 0 and buffers(4, 128, 4096, 4096, 0, 1, plain) < 0
     # a walk of one tile: every format and shape that has the second buffer at all (up to 32 batch rows, four row blocks)
     for bits, flags in ((2, plain), (4, bf16), (6, plain), (8, bf16)):
