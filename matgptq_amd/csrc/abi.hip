@@ -27,14 +27,14 @@ int check_problem(int bits, int group_size, int64_t N, int64_t K);  // pack_host
   hipError_t launch_decode_b##B(const GemmArgs&, int group_size, int R, int S, int W, int kc,  \
                                 bool stream_flavour, size_t smem, hipStream_t);                \
   hipError_t launch_prefill_b##B(const GemmArgs&, int group_size, int cfg, hipStream_t);          \
-  hipError_t launch_skinny_b##B(const GemmArgs&, int group_size, int r, int mb, bool one, bool master, hipStream_t);   \
+  hipError_t launch_skinny_b##B(const GemmArgs&, int group_size, int r, int mb, bool master, hipStream_t);   \
   hipError_t launch_few_rows_b##B(const GemmArgs&, int group_size, int r, int rows, bool master, hipStream_t);          \
   hipError_t launch_few_rows_b##B##_bf16(const GemmArgs&, int group_size, int r, int rows, bool master, hipStream_t);   \
   hipError_t launch_gemv_b##B(const GemmArgs&, int group_size, int shape, int W, size_t lds_pad, bool master, hipStream_t);  \
   hipError_t launch_gemv_b##B##_bf16(const GemmArgs&, int group_size, int shape, int W, size_t lds_pad, bool master, hipStream_t); \
   hipError_t launch_gemv_prologue_b##B(const GemmArgs&, int kind, int shape, int W, const void* b, const void* w, void* out, \
                                        float eps, hipStream_t);                                                            \
-  hipError_t launch_skinny_b##B##_bf16(const GemmArgs&, int group_size, int r, int mb, bool one, bool master, hipStream_t); \
+  hipError_t launch_skinny_b##B##_bf16(const GemmArgs&, int group_size, int r, int mb, bool master, hipStream_t); \
   hipError_t launch_decode_b##B##_bf16(const GemmArgs&, int group_size, int R, int S, int W,   \
                                        int kc, bool stream_flavour, size_t smem, hipStream_t); \
   hipError_t launch_prefill_b##B##_bf16(const GemmArgs&, int group_size, int cfg, hipStream_t);
@@ -572,15 +572,15 @@ hipError_t launch_gemv(int bits, bool bf16, const GemmArgs& a, int g, const Plan
 #undef MATGPTQ_CASE
 }
 
-hipError_t launch_skinny(int bits, bool bf16, const GemmArgs& a, int g, const Plan& p, bool one, bool master, hipStream_t s) {
+hipError_t launch_skinny(int bits, bool bf16, const GemmArgs& a, int g, const Plan& p, bool master, hipStream_t s) {
 #define MATGPTQ_CASE(B) \
-  case B: return bf16 ? launch_skinny_b##B##_bf16(a, g, p.R, p.mb, one, master, s) : launch_skinny_b##B(a, g, p.R, p.mb, one, master, s);
+  case B: return bf16 ? launch_skinny_b##B##_bf16(a, g, p.R, p.mb, master, s) : launch_skinny_b##B(a, g, p.R, p.mb, master, s);
   switch (bits) {
     MATGPTQ_CASE(2)
     MATGPTQ_CASE(3)
     MATGPTQ_CASE(4)
     MATGPTQ_CASE(6)
-    default: return bf16 ? launch_skinny_b8_bf16(a, g, p.R, p.mb, one, master, s) : launch_skinny_b8(a, g, p.R, p.mb, one, master, s);
+    default: return bf16 ? launch_skinny_b8_bf16(a, g, p.R, p.mb, master, s) : launch_skinny_b8(a, g, p.R, p.mb, master, s);
   }
 #undef MATGPTQ_CASE
 }
@@ -674,12 +674,10 @@ static int run_gemm(int bitwidth, int group_size, int64_t N, int64_t K, int64_t 
   a.row_blocks = (int)(N / 16);
   hipStream_t s = static_cast<hipStream_t>(stream);
   const bool bf16 = (flags & MATGPTQ_FLAG_BF16) != 0;
-  // (a forced variant on pre-sliced codes keeps the two buffers that matgptq_midbatch_buffers reports for it)
-  const bool one_tile = master_planes || (flags & MATGPTQ_FLAG_VARIANT_MASK) == 0;
   const hipError_t err = few.row_blocks != 0 ? launch_few_rows(bitwidth, bf16, a, group_size, few, master_planes, s)
                          : p.gemv   ? launch_gemv(bitwidth, bf16, a, group_size, p, master_planes, s)
                          : p.decode ? launch_decode(bitwidth, bf16, a, group_size, p, s)
-                         : p.skinny ? launch_skinny(bitwidth, bf16, a, group_size, p, one_tile, master_planes, s)
+                         : p.skinny ? launch_skinny(bitwidth, bf16, a, group_size, p, master_planes, s)
                                     : launch_prefill(bitwidth, bf16, a, group_size, p, s);
   if (err != hipSuccess) return MATGPTQ_ELAUNCH;
   // K = 128 t + 64: the kernels above have multiplied the t tiles; a second launch adds the last 64 columns
@@ -932,7 +930,6 @@ int matgptq_midbatch_buffers(int bitwidth, int group_size, int64_t N, int64_t K,
   Plan p;
   if (int e = make_plan(bitwidth, group_size, N, K, M, has_zeros != 0, flags, &p)) return e;
   if (!p.skinny || few_rows_of(bitwidth, group_size, N, K, M, nullptr, flags, false).row_blocks != 0) return 0;
-  if ((flags & MATGPTQ_FLAG_VARIANT_MASK) == 0 && K / 128 <= 8) return 1;
   return midbatch_two_buffers(bitwidth, (flags & MATGPTQ_FLAG_BF16) != 0, group_size, has_zeros != 0, p.R, p.mb, false,
                               (int)(K / 128), (int)M, (int)(N / 16)) ? 2 : 1;
 }

@@ -9,7 +9,8 @@ namespace matgptq {
 // the empty tile that the loop of pairs ends with; what they cost is registers (two sets of codes stay live) and, over
 // 64 KB, the second workgroup of a CU.  One against two buffers on some 15000 random calls (M = 5..128, K = 256..8192, all bitwidths,
 // groups and storage types; mean gain, share that lost more than 1.5 %):
-//  * walks of one tile: 13 %, none (8192 x 1024 at 4 bits, M = 16 / 32 / 64: 4.29 -> 3.98 / 5.28 -> 4.77 / 6.30 -> 5.69 us);
+//  * walks of one tile have nothing to fetch ahead: one buffer and one register set, the next workgroup of the CU instead
+//    (64 rows per workgroup 1.27 to 1.36 times faster than with two, 32 rows 1.03 to 1.08);
 //  * one row block and 16 batch rows: two or three tiles 6.7 %, 0.1 %; longer walks 5 %, 1 % (4096 x 4096 at M = 12:
 //    5.53 -> 5.28 us) without group 32 with zero points (0 to 2 %, 7 %: four scales and zeros per tile in two sets) and
 //    without even walks at 6 bits (2.5 %, 17 %);
@@ -26,7 +27,7 @@ inline bool midbatch_two_buffers(int bits, bool bf16, int group_size, bool zeros
   if (master || r > 4 || mb > 2) return false;
   const int walk = (k_tiles + 7) / 8;
   const int workgroups = ((row_blocks + r - 1) / r) * ((M + 16 * mb - 1) / (16 * mb));
-  if (walk <= 1) return true;
+  if (walk <= 1) return false;
   if (r > 1)
     return mb == 1 && !bf16 && workgroups > 256 && !(group_size == 32 && bits == 8) && !(r == 4 && bits == 6 && zeros);
   if (M > 32 && k_tiles > 32) return false;  // (several blocks of batch rows and a long walk)

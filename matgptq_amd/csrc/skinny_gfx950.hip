@@ -318,11 +318,11 @@ skinny_kernel(const GemmArgs a, int n_tiles, int m_tiles) {
 }
 
 template <int GROUP, bool ZP, int R, int MB, bool MASTER>
-hipError_t launch_r(const GemmArgs& a, bool one, hipStream_t stream) {
+hipError_t launch_r(const GemmArgs& a, hipStream_t stream) {
   const int n_tiles = (a.row_blocks + R - 1) / R;
   const int m_tiles = (a.M + 16 * MB - 1) / (16 * MB);
   const dim3 grid(n_tiles * m_tiles), block(64 * kWaves);
-  if (one && a.k_tiles <= kWaves) {
+  if (a.k_tiles <= kWaves) {
     hipLaunchKernelGGL((skinny_kernel<kBits, GROUP, ZP, R, MB, MASTER, 0>), grid, block, 0, stream, a, n_tiles, m_tiles);
     return hipGetLastError();
   }
@@ -335,30 +335,30 @@ hipError_t launch_r(const GemmArgs& a, bool one, hipStream_t stream) {
 }
 
 template <int GROUP, bool ZP, int MB, bool MASTER>
-hipError_t launch_rows(const GemmArgs& a, int r, bool one, hipStream_t s) {
+hipError_t launch_rows(const GemmArgs& a, int r, hipStream_t s) {
   // (four row blocks fit the register budget of two waves per SIMD up to 6 bits and with one
   // scale and zero per tile and row block; group 32 carries four; the master planes are eight
   // words per lane from 6 bits on)
   // (eight row blocks: pre-sliced codes up to 4 bits, 32 batch rows)
   if constexpr (GROUP != 32 && kBits <= 4 && !MASTER && MB == 2) {
-    if (r >= 8) return launch_r<GROUP, ZP, 8, MB, MASTER>(a, one, s);
+    if (r >= 8) return launch_r<GROUP, ZP, 8, MB, MASTER>(a, s);
   }
   if constexpr (GROUP != 32 && kBits <= (MASTER ? 4 : 6)) {
-    if (r >= 4) return launch_r<GROUP, ZP, 4, MB, MASTER>(a, one, s);
+    if (r >= 4) return launch_r<GROUP, ZP, 4, MB, MASTER>(a, s);
   }
-  if (r >= 2) return launch_r<GROUP, ZP, 2, MB, MASTER>(a, one, s);
-  return launch_r<GROUP, ZP, 1, MB, MASTER>(a, one, s);
+  if (r >= 2) return launch_r<GROUP, ZP, 2, MB, MASTER>(a, s);
+  return launch_r<GROUP, ZP, 1, MB, MASTER>(a, s);
 }
 
 template <int GROUP, bool ZP, bool MASTER>
-hipError_t launch_batch(const GemmArgs& a, int r, int mb, bool one, hipStream_t s) {
-  if (mb >= 4) return launch_rows<GROUP, ZP, 4, MASTER>(a, r, one, s);
-  return mb >= 2 ? launch_rows<GROUP, ZP, 2, MASTER>(a, r, one, s) : launch_rows<GROUP, ZP, 1, MASTER>(a, r, one, s);
+hipError_t launch_batch(const GemmArgs& a, int r, int mb, hipStream_t s) {
+  if (mb >= 4) return launch_rows<GROUP, ZP, 4, MASTER>(a, r, s);
+  return mb >= 2 ? launch_rows<GROUP, ZP, 2, MASTER>(a, r, s) : launch_rows<GROUP, ZP, 1, MASTER>(a, r, s);
 }
 
 template <int GROUP, bool ZP>
-hipError_t launch_storage(const GemmArgs& a, int r, int mb, bool one, bool master, hipStream_t s) {
-  return master ? launch_batch<GROUP, ZP, true>(a, r, mb, one, s) : launch_batch<GROUP, ZP, false>(a, r, mb, one, s);
+hipError_t launch_storage(const GemmArgs& a, int r, int mb, bool master, hipStream_t s) {
+  return master ? launch_batch<GROUP, ZP, true>(a, r, mb, s) : launch_batch<GROUP, ZP, false>(a, r, mb, s);
 }
 
 }  // namespace
@@ -371,15 +371,14 @@ hipError_t launch_storage(const GemmArgs& a, int r, int mb, bool one, bool maste
 #else
 #define MATGPTQ_LAUNCH_NAME MATGPTQ_CAT(launch_skinny_b, MATGPTQ_BITS)
 #endif
-// one: walks of one tile take the kernel with one buffer and one register set; master: `a.packed` holds master-resident
-// bit planes
-hipError_t MATGPTQ_LAUNCH_NAME(const GemmArgs& a, int group_size, int r, int mb, bool one, bool master, hipStream_t stream) {
+// master: `a.packed` holds master-resident bit planes
+hipError_t MATGPTQ_LAUNCH_NAME(const GemmArgs& a, int group_size, int r, int mb, bool master, hipStream_t stream) {
   const bool zp = a.zeros != nullptr;
   if (group_size == 128)
-    return zp ? launch_storage<128, true>(a, r, mb, one, master, stream) : launch_storage<128, false>(a, r, mb, one, master, stream);
+    return zp ? launch_storage<128, true>(a, r, mb, master, stream) : launch_storage<128, false>(a, r, mb, master, stream);
   if (group_size == 32)
-    return zp ? launch_storage<32, true>(a, r, mb, one, master, stream) : launch_storage<32, false>(a, r, mb, one, master, stream);
-  return zp ? launch_storage<-1, true>(a, r, mb, one, master, stream) : launch_storage<-1, false>(a, r, mb, one, master, stream);
+    return zp ? launch_storage<32, true>(a, r, mb, master, stream) : launch_storage<32, false>(a, r, mb, master, stream);
+  return zp ? launch_storage<-1, true>(a, r, mb, master, stream) : launch_storage<-1, false>(a, r, mb, master, stream);
 }
 
 }  // namespace matgptq

@@ -453,12 +453,12 @@ def test_midbatch_buffers_at_the_edges_of_the_rule():
 
     assert [buffers(4, 128, 4096, 4096, m, 1, plain) for m in (1, 16, 128, 2048)] == [0, 0, 1, 0]  # 0: another kernel
     assert buffers(5, 128, 4096, 4096, 16, 1, plain) < 0 and buffers(4, 128, 4096, 4096, 0, 1, plain) < 0
-    # a walk of one tile: every format and shape that has the second buffer at all (up to 32 batch rows, four row blocks)
+    # a walk of one tile has nothing to fetch ahead; up to 32 batch rows and four row blocks have the second buffer at all
     for bits, flags in ((2, plain), (4, bf16), (6, plain), (8, bf16)):
-        assert buffers(bits, 128, 256, 1024, 16, 1, flags | forced(1, 0)) == 2
-        assert buffers(bits, 32, 256, 1024, 30, 1, flags | forced(0, 1)) == 2
-    assert buffers(4, 128, 256, 1024, 60, 1, plain | forced(0, 2)) == 1   # 64 batch rows
-    assert buffers(4, 128, 256, 1024, 30, 1, plain | (91 << 8)) == 1      # eight row blocks
+        assert [buffers(bits, 128, 256, k, 16, 1, flags | forced(0, 0)) for k in (1024, 1152)] == [1, 2]
+        assert [buffers(bits, 32, 256, k, 30, 1, flags | forced(0, 1)) for k in (1024, 1152)] == [1, 2]
+    assert buffers(4, 128, 256, 1152, 60, 1, plain | forced(0, 2)) == 1   # 64 batch rows
+    assert buffers(4, 128, 256, 1152, 30, 1, plain | (91 << 8)) == 1      # eight row blocks
     # one row block, 16 batch rows: 3 | 4 tiles with zero points at group 32, 5 | 6 at 6 bits
     one = forced(0, 0)
     assert [buffers(4, 32, 256, k, 16, 1, plain | one) for k in (3072, 3200)] == [2, 1]
