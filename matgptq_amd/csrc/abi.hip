@@ -373,7 +373,8 @@ int make_plan(int bits, int group_size, int64_t N, int64_t K, int64_t M, bool zp
   } else if (flavour == 0 && M > kGemvMaxM &&
              !(bits == 8 && group_size != 32 && !(flags & MATGPTQ_FLAG_BF16) && row_blocks >= 1024)) {
     // Five to sixteen batch rows.  Automatic calls at group sizes 128 and -1 run the few-rows kernel in front of this plan
-    // (few_rows_of), so these lines and the eight-row ones below decide group size 32 and activations off 16 bytes.
+    // (few_rows_of), so these lines and the eight-row ones below decide group size 32, activations off 16 bytes, and the short
+    // walks of 8-bit codes that few_rows_small leaves to the decode kernel.
     // Every decode workgroup stages the whole batch of activations (scaled copies, written by the vector
     // ALU), which grows with M and K, while the mid-batch kernel copies them into LDS
     // asynchronously.  Measured on MI355X (Llama-3-8B layers, 2, 4 and 8 bits, M = 5 .. 16, weights

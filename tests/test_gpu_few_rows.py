@@ -12,7 +12,7 @@ from tests import _gpu_util as G
 pytestmark = pytest.mark.gpu
 
 # (N, K, M, row blocks per workgroup of 4-bit codes, of 4-bit planes)
-CASES = [(16, 128, 1, 1, 1), (48, 1024, 2, 1, 1), (304, 1152, 2, 1, 1), (48, 8192, 4, 1, 1), (5136, 384, 3, 2, 2), (32, 2048, 5, 1, 1),
+CASES = [(16, 128, 1, 1, 1), (48, 1024, 2, 1, 1), (304, 1152, 2, 1, 1), (48, 7680, 4, 1, 1), (5136, 384, 3, 2, 2), (32, 2048, 5, 1, 1),
          (5136, 1152, 8, 2, 2), (8208, 2944, 7, 2, 2), (10256, 3072, 8, 4, 4), (80, 4224, 9, 1, 1), (5136, 896, 16, 2, 2),
          (10256, 1024, 13, 4, 4), (10288, 2176, 16, 4, 4)]
 # (N, K, M, row blocks and batch rows per workgroup of 4-bit codes)
@@ -91,7 +91,7 @@ def rows_expected(k, m, r, rows, bits, group, bf16, planes):
         return 0
     most = 2 if bits > (4 if planes else 6) else 8 if rows == 32 and bits <= 4 and not planes else 4
     small_tiles = planes and bits > 4 and r == 2 and rows == 16 and 1024 < k and m <= 32
-    return 0 if small_tiles else r if r <= most else 4 if r == 8 and most == 4 and not planes else 0
+    return 0 if small_tiles or r > most else r
 
 
 @pytest.mark.parametrize("n,k,m,rows,bits,group,bf16,planes", [
