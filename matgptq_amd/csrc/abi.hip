@@ -28,8 +28,8 @@ int check_problem(int bits, int group_size, int64_t N, int64_t K);  // pack_host
                                 bool stream_flavour, size_t smem, hipStream_t);                \
   hipError_t launch_prefill_b##B(const GemmArgs&, int group_size, int cfg, hipStream_t);          \
   hipError_t launch_skinny_b##B(const GemmArgs&, int group_size, int r, int mb, bool master, hipStream_t);   \
-  hipError_t launch_few_rows_b##B(const GemmArgs&, int group_size, int r, int rows, bool master, hipStream_t);          \
-  hipError_t launch_few_rows_b##B##_bf16(const GemmArgs&, int group_size, int r, int rows, bool master, hipStream_t);   \
+  hipError_t launch_few_rows_b##B(const GemmArgs&, int group_size, int r, int held, bool master, hipStream_t);          \
+  hipError_t launch_few_rows_b##B##_bf16(const GemmArgs&, int group_size, int r, int held, bool master, hipStream_t);   \
   hipError_t launch_gemv_b##B(const GemmArgs&, int group_size, int shape, int W, size_t lds_pad, bool master, hipStream_t);  \
   hipError_t launch_gemv_b##B##_bf16(const GemmArgs&, int group_size, int shape, int W, size_t lds_pad, bool master, hipStream_t); \
   hipError_t launch_gemv_prologue_b##B(const GemmArgs&, int kind, int shape, int W, const void* b, const void* w, void* out, \
@@ -588,13 +588,13 @@ hipError_t launch_skinny(int bits, bool bf16, const GemmArgs& a, int g, const Pl
 
 hipError_t launch_few_rows(int bits, bool bf16, const GemmArgs& a, int g, FewRows f, bool master, hipStream_t s) {
 #define MATGPTQ_CASE(B) \
-  case B: return bf16 ? launch_few_rows_b##B##_bf16(a, g, f.row_blocks, f.batch_rows, master, s) : launch_few_rows_b##B(a, g, f.row_blocks, f.batch_rows, master, s);
+  case B: return bf16 ? launch_few_rows_b##B##_bf16(a, g, f.row_blocks, few_rows_held(f, a.M), master, s) : launch_few_rows_b##B(a, g, f.row_blocks, few_rows_held(f, a.M), master, s);
   switch (bits) {
     MATGPTQ_CASE(2)
     MATGPTQ_CASE(3)
     MATGPTQ_CASE(4)
     MATGPTQ_CASE(6)
-    default: return bf16 ? launch_few_rows_b8_bf16(a, g, f.row_blocks, f.batch_rows, master, s) : launch_few_rows_b8(a, g, f.row_blocks, f.batch_rows, master, s);
+    default: return bf16 ? launch_few_rows_b8_bf16(a, g, f.row_blocks, few_rows_held(f, a.M), master, s) : launch_few_rows_b8(a, g, f.row_blocks, few_rows_held(f, a.M), master, s);
   }
 #undef MATGPTQ_CASE
 }
@@ -765,12 +765,12 @@ static int master_reads_planes(int bitwidth, int group_size, int64_t N, int64_t 
   Plan p;
   if (int e = make_plan(bitwidth, group_size, N, K, M, zp, *flags, &p)) return e;
   *direct = plan_reads_planes(p, M);
-  const bool few = few_rows_of(bitwidth, group_size, N, K, M, x, *flags, true).row_blocks != 0;
-  if (few && M <= 16) {
+  // (the few-rows kernel reads them, and where the activations' address keeps a call from it the ways below all end without
+  // the workspace too)
+  if (few_rows_of(bitwidth, group_size, N, K, M, x, *flags, true).row_blocks != 0) {
     *direct = true;
     return MATGPTQ_OK;
   }
-  const uint32_t asked = *flags;
   const bool automatic = (*flags & MATGPTQ_FLAG_VARIANT_MASK) == 0 && ((*flags >> 16) & 3u) == 0;
   if (!*direct && automatic && M <= kGemvMaxM) {
     // the planner's own gemv shape for this problem has no instantiation on planes (four row blocks
@@ -790,8 +790,6 @@ static int master_reads_planes(int bitwidth, int group_size, int64_t N, int64_t 
       *direct = true;
     }
   }
-  // (a shape that needs the workspace keeps it, and multiplies the codes sliced there)
-  if (few && *direct) *flags = asked;
   return MATGPTQ_OK;
 }
 

@@ -377,45 +377,46 @@ few_rows_kernel(const GemmArgs a, int n_tiles, int m_tiles) {
   }
 }
 
-template <int GROUP, bool ZP, int R, int ROWS, bool MASTER>
-hipError_t launch_r(const GemmArgs& a, hipStream_t stream) {
-  const int n_tiles = (a.row_blocks + R - 1) / R, m_tiles = (a.M + ROWS - 1) / ROWS;
-  const dim3 grid(n_tiles * m_tiles), block(64 * kWaves);
-  if (a.k_tiles <= kWaves)
-    hipLaunchKernelGGL((few_rows_kernel<kBits, GROUP, ZP, R, ROWS, MASTER, true>), grid, block, 0, stream, a, n_tiles, m_tiles);
-  else
-    hipLaunchKernelGGL((few_rows_kernel<kBits, GROUP, ZP, R, ROWS, MASTER, false>), grid, block, 0, stream, a, n_tiles, m_tiles);
-  return hipGetLastError();
-}
-
-template <int GROUP, bool ZP, int R, bool MASTER>
-hipError_t launch_batch(const GemmArgs& a, int rows, hipStream_t stream) {
-  if constexpr (R >= 2) {
-    if (rows > 16) return launch_r<GROUP, ZP, R, 32, MASTER>(a, stream);
-  }
-  if constexpr (R <= 4) {
-    if (a.M <= 4) return launch_r<GROUP, ZP, R, 4, MASTER>(a, stream);
-    return a.M <= 8 ? launch_r<GROUP, ZP, R, 8, MASTER>(a, stream) : launch_r<GROUP, ZP, R, 16, MASTER>(a, stream);
+template <int GROUP, bool ZP, int R, int ROWS, bool MASTER, bool ONE>
+hipError_t launch_walk(const GemmArgs& a, hipStream_t stream) {
+  if constexpr (few_rows_built(kBits, GROUP, kBf16, MASTER, R, ROWS, ONE)) {
+    const int n_tiles = (a.row_blocks + R - 1) / R, m_tiles = (a.M + ROWS - 1) / ROWS;
+    const dim3 grid(n_tiles * m_tiles), block(64 * kWaves);
+    hipLaunchKernelGGL((few_rows_kernel<kBits, GROUP, ZP, R, ROWS, MASTER, ONE>), grid, block, 0, stream, a, n_tiles, m_tiles);
+    return hipGetLastError();
   }
   return hipErrorInvalidValue;
 }
 
+template <int GROUP, bool ZP, int R, int ROWS, bool MASTER>
+hipError_t launch_r(const GemmArgs& a, hipStream_t stream) {
+  return a.k_tiles <= kWaves ? launch_walk<GROUP, ZP, R, ROWS, MASTER, true>(a, stream)
+                             : launch_walk<GROUP, ZP, R, ROWS, MASTER, false>(a, stream);
+}
+
+template <int GROUP, bool ZP, int R, bool MASTER>
+hipError_t launch_batch(const GemmArgs& a, int held, hipStream_t stream) {
+  switch (held) {
+    case 4: return launch_r<GROUP, ZP, R, 4, MASTER>(a, stream);
+    case 8: return launch_r<GROUP, ZP, R, 8, MASTER>(a, stream);
+    case 16: return launch_r<GROUP, ZP, R, 16, MASTER>(a, stream);
+    default: return launch_r<GROUP, ZP, R, 32, MASTER>(a, stream);
+  }
+}
+
 template <int GROUP, bool ZP, bool MASTER>
-hipError_t launch_rows(const GemmArgs& a, int r, int rows, hipStream_t s) {
-  // (what the registers hold: few_rows_most_row_blocks)
-  if constexpr (few_rows_most_row_blocks(kBits, MASTER, 32) >= 8) {
-    if (r >= 8) return launch_batch<GROUP, ZP, 8, MASTER>(a, rows, s);
+hipError_t launch_rows(const GemmArgs& a, int r, int held, hipStream_t s) {
+  switch (r) {
+    case 1: return launch_batch<GROUP, ZP, 1, MASTER>(a, held, s);
+    case 2: return launch_batch<GROUP, ZP, 2, MASTER>(a, held, s);
+    case 4: return launch_batch<GROUP, ZP, 4, MASTER>(a, held, s);
+    default: return launch_batch<GROUP, ZP, 8, MASTER>(a, held, s);
   }
-  if constexpr (few_rows_most_row_blocks(kBits, MASTER, 16) >= 4) {
-    if (r >= 4) return launch_batch<GROUP, ZP, 4, MASTER>(a, rows, s);
-  }
-  if (r >= 2) return launch_batch<GROUP, ZP, 2, MASTER>(a, rows, s);
-  return launch_batch<GROUP, ZP, 1, MASTER>(a, rows, s);
 }
 
 template <int GROUP, bool ZP>
-hipError_t launch_storage(const GemmArgs& a, int r, int rows, bool master, hipStream_t s) {
-  return master ? launch_rows<GROUP, ZP, true>(a, r, rows, s) : launch_rows<GROUP, ZP, false>(a, r, rows, s);
+hipError_t launch_storage(const GemmArgs& a, int r, int held, bool master, hipStream_t s) {
+  return master ? launch_rows<GROUP, ZP, true>(a, r, held, s) : launch_rows<GROUP, ZP, false>(a, r, held, s);
 }
 
 }  // namespace
@@ -427,14 +428,14 @@ hipError_t launch_storage(const GemmArgs& a, int r, int rows, bool master, hipSt
 #else
 #define MATGPTQ_LAUNCH_NAME MATGPTQ_CAT(launch_few_rows_b, MATGPTQ_BITS)
 #endif
-// Group size 128 or -1.  r: row blocks of 16 weight rows per workgroup (1, 2, 4; 2, 4, 8 with 32 batch rows); rows: batch rows
-// per workgroup, 16 (fewer are taken where M is 4 or 8 at most) or 32; master: `a.packed` holds master-resident bit planes
-hipError_t MATGPTQ_LAUNCH_NAME(const GemmArgs& a, int group_size, int r, int rows, bool master, hipStream_t stream) {
+// Group size 128 or -1.  r: row blocks of 16 weight rows and held: batch rows per workgroup, as few_rows and few_rows_held give
+// them; master: `a.packed` holds master-resident bit planes
+hipError_t MATGPTQ_LAUNCH_NAME(const GemmArgs& a, int group_size, int r, int held, bool master, hipStream_t stream) {
   const bool zp = a.zeros != nullptr;
   if (group_size == 32) return hipErrorInvalidValue;
   if (group_size == 128)
-    return zp ? launch_storage<128, true>(a, r, rows, master, stream) : launch_storage<128, false>(a, r, rows, master, stream);
-  return zp ? launch_storage<-1, true>(a, r, rows, master, stream) : launch_storage<-1, false>(a, r, rows, master, stream);
+    return zp ? launch_storage<128, true>(a, r, held, master, stream) : launch_storage<128, false>(a, r, held, master, stream);
+  return zp ? launch_storage<-1, true>(a, r, held, master, stream) : launch_storage<-1, false>(a, r, held, master, stream);
 }
 
 }  // namespace matgptq

@@ -117,6 +117,14 @@ inline int few_rows_small(int bits, int group_size, bool bf16, bool master, int 
   return 1;
 }
 
+// The instantiations that the two rules can ask for (and no others are built): `held` as few_rows_held gives it, `one`: walks of
+// one tile.
+constexpr bool few_rows_built(int bits, int group_size, bool bf16, bool master, int r, int held, bool one) {
+  if (held == 32) return !one && r >= 2 && r <= few_rows_most_row_blocks(bits, master, 32);
+  if (held == 4) return r <= 2 && (bf16 || master || group_size != 128);
+  return r <= 4 && r <= few_rows_most_row_blocks(bits, master, 16);
+}
+
 // The workgroup for M batch rows.  `master`: the codes are master-resident planes.
 inline FewRows few_rows(int bits, int group_size, bool bf16, bool master, int M, int row_blocks, int k_tiles) {
   if (group_size == 32 || M > kFewRowsMaxM) return {0, 0};

@@ -524,6 +524,34 @@ def test_few_rows_at_the_edges_of_the_rule():
     assert [few(4, 128, 256, 4096, m, plain, p) for m in (31, 32, 64) for p in (0, 1)] == [1, 1, 0, 0, 0, 0]
 
 
+def test_few_rows_instantiations_are_those_that_the_rule_asks_for(tmp_path):
+    # the rule over all formats, 1 to 64 batch rows, up to 8300 row blocks and the walks at its lines: every workgroup that it
+    # returns is built, and every one that is built is returned for some call
+    import subprocess
+    source, program = tmp_path / "few.cpp", tmp_path / "few"
+    source.write_text(r'''
+#include "fewrows_plan.h"
+#include <cstdio>
+#include <initializer_list>
+using namespace matgptq;
+static bool seen[9][2][2][2][9][33][2];
+int main() {
+  for (int b : {2, 3, 4, 6, 8}) for (int g = 0; g < 2; g++) for (int bf = 0; bf < 2; bf++) for (int pl = 0; pl < 2; pl++) {
+    for (int m = 1; m <= 64; m++) for (int rb = 1; rb <= 8300; rb += rb < 1100 ? 1 : 7)
+      for (int kt : {1, 2, 4, 5, 8, 9, 10, 16, 17, 24, 25, 33, 41, 51, 56, 57, 61, 80, 112, 224}) {
+        const FewRows f = few_rows(b, g ? 128 : -1, bf, pl, m, rb, kt);
+        if (f.row_blocks) seen[b][g][bf][pl][f.row_blocks][few_rows_held(f, m)][kt <= kFewRowsWaves] = true;
+      }
+    for (int r : {1, 2, 4, 8}) for (int held : {4, 8, 16, 32}) for (int one = 0; one < 2; one++)
+      if (seen[b][g][bf][pl][r][held][one] != few_rows_built(b, g ? 128 : -1, bf, pl, r, held, one))
+        std::printf("b%d g%d bf%d planes%d r%d held%d one%d\n", b, g ? 128 : -1, bf, pl, r, held, one);
+  }
+}
+''')
+    subprocess.run(["g++", "-O2", "-std=c++17", f"-I{ROOT}/matgptq_amd/csrc", str(source), "-o", str(program)], check=True)
+    assert subprocess.run([str(program)], check=True, capture_output=True, text=True).stdout == ""
+
+
 def test_planner_gives_the_wider_formats_192_rows_and_few_64_row_tiles_smaller_workgroups():
     plan = lambda *a: _lib.describe_plan(*a).split(" zp")[1][2:]
     # one round of 128 x 192 tiles with K split where the 128 x 256 tile spills; not 6 bits with the order of sums kept
