@@ -207,7 +207,7 @@ int make_plan(int bits, int group_size, int64_t N, int64_t K, int64_t M, bool zp
       // (M = 2048, 4 bits: 8192 x 8192 228 against 256 us on 128 x 128 tiles, 8192 x 28672 761 against 870,
       // 57344 x 8192 1542 against 1611 on 128 x 192).  At 3 and 6 bits, with group size 32, and at 8 bits
       // with a scale and zero per tile it spills (8 bits, 8192 x 8192: 511 us): those take the
-      // 128 x 128 tile or, except at 6 bits, the 128 x 192 tile where its rounds pay.  8-bit codes fit
+      // 128 x 128 tile or the 128 x 192 tile where its rounds pay (at 6 bits: one in place of two).  8-bit codes fit
       // the 128 x 256 tile again once eight waves halve K between them, up to two rounds of one such
       // workgroup per CU (8192 x 8192, M = 2048: 243 against 270 us; 8192 x 28672: 889 against 1018).
       // Group size 32 with zero points keeps four scales and four zeros per tile and row block in
@@ -227,9 +227,9 @@ int make_plan(int bits, int group_size, int64_t N, int64_t K, int64_t M, bool zp
         const double t_128 = rounds(wgs_128);
         p->cfg = t_192 < t_128 && fits_192 ? 9 : 3;
         // One round of 128 x 192 tiles, where 128 x 128 tiles need a second one, pays for every format but 3 bits of bf16
-        // storage at group size 32 with zero points (0.6), also for those that lose where rounds are many: 1.15 to 1.30, 550
-        // random calls.  Both widths in one launch where they take every slot once: 1.2 to 1.5 against 128 x 128, 1.03 to
-        // 1.13 against 128 x 192 alone (bf16 storage, and 6 bits without a scale per tile).
+        // storage at group size 32 with zero points (0.6), also for those that lose where rounds are many: 1.17 over 1535
+        // random calls, none slower.  Both widths in one launch where they take every slot once: 1.27 over 3041 against 128 x 128
+        // or 128 x 192 tiles, 1.03 to 1.13 against the latter alone (bf16 storage, and 6 bits without a scale per tile).
         if (wgs_192 <= 512 && wgs_128 > 512 && !(bits == 3 && bf16 && g32zp)) {
           int narrow = 0;
           const int wide = prefill_mix_wide_tiles(row_blocks, m_tiles, &narrow);
@@ -354,14 +354,14 @@ int make_plan(int bits, int group_size, int64_t N, int64_t K, int64_t M, bool zp
         }
       }
       // Formats whose registers do not hold the 128 x 256 tile take the 128 x 192 tile with K split in place of the 128 x 128 tile:
-      // 1.24 to 1.30 over 2300 random calls, none slower.  (6-bit codes on fp16 storage with a scale per tile keep the order of
-      // their sums.)
+      // 1.26 over 2358 random calls, none slower.  (6-bit codes on fp16 storage with a scale per tile stay where they were: their
+      // results are left bit for bit as they were, which nothing depends on.)
       if (!p->skinny && p->cfg == 3 && wgs_192s <= 256 && t_192s < best && !fixed_order) p->cfg = 13;
       // The 64 x 128 tile on few of the CUs: workgroups of the mid-batch kernel a quarter or a half as large take more of them.
-      // Up to 96 of the tiles, 2000 random calls of 97 to 640 batch rows: 1.30 with 32 x 32 and, where 64 batch rows pad no more,
-      // 1.25 with 64 x 64 (8-bit codes, two row blocks at most, 0.93 that way, and 0.76 to 0.9 on walks of three tiles with
+      // Up to 96 of the tiles, 2090 random calls of 97 to 640 batch rows: 1.33 with 32 x 32 (2 % lost more than 2 %) and, where 64
+      // batch rows pad no more, 1.21 with 64 x 64 (8-bit codes, two row blocks at most, 0.93 that way, and 0.76 to 0.9 on walks of three tiles with
       // 32 x 32: not those); more batch rows on fewer row blocks 0.76 to 1; 97 to 128 of the tiles 0.95 to 1.2.
-      // (fp16 storage with a scale per tile keeps the order of its sums.)
+      // (Not fp16 storage with a scale per tile, as above.)
       if (variant == 0 && !p->skinny && p->cfg == 16 && M > 96 && M <= 640 && !(bits == 8 && k_tiles <= 24) && !fixed_order &&
           ((N + 127) / 128) * ((M + 63) / 64) <= 96) {
         p->skinny = p->sliced_only = true;

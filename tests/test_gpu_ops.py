@@ -336,6 +336,24 @@ def test_resident_master_codes_switch_bitwidth_at_run_time():
         plain.set_bitwidth(torch.nn.Module(), 4)
 
 
+@pytest.mark.parametrize("watched", ("nothing", "input", "scales", "zeros"))
+def test_module_products_have_no_gradient(watched):
+    # (the module switches grad mode off only where a tensor would ask for one)
+    n, k, g = 64, 256, 128
+    q, s, z = o.make_layer(n, k, g, seed=2)
+    perm = torch.from_numpy(np.random.default_rng(0).permutation(k))
+    lin = MatGPTQLinear(torch.from_numpy(o.slice_codes(q, 4)).cuda(), torch.from_numpy(s).cuda(), 4, g, zeros=torch.from_numpy(z).cuda(),
+                        perm=perm)
+    x = torch.from_numpy(o.make_activations(3, k, seed=1)).cuda()
+    with torch.no_grad():
+        want = lin(x)
+    t = {"input": x, "scales": lin.matgptq_scales, "zeros": lin.matgptq_zeros}.get(watched)
+    if t is not None:
+        t.requires_grad_(True)
+    y = lin(x)
+    assert torch.is_grad_enabled() and not y.requires_grad and y.grad_fn is None and torch.equal(y, want)
+
+
 def test_strided_input_is_accepted():
     # the reference never checks the layout of its input (bindings.cpp:146-191)
     n, k, b = 64, 512, 4

@@ -1,5 +1,6 @@
 """Formats and sizes on the lines of the rules that choose between 128 x 128 tiles, 128 x 192 tiles (with K split, alone, or mixed
-with the narrower ones in one launch), 64 x 128 tiles and the mid-batch kernel, against the 128 x 128 tile forced."""
+with the narrower ones in one launch), 64 x 128 tiles and the mid-batch kernel, against the product in 64 bits and against the
+128 x 128 tile forced."""
 import numpy as np
 import pytest
 import torch
@@ -34,6 +35,12 @@ def test_plan_lines(bits, group, bf16, zeros, n, k, m, plan):
     # both form the same rounded weights and round each result once; their sums in fp32, in other orders, differ by less than
     # 2^-20 of the sum of the magnitudes
     spread = lambda t: np.repeat(t.double().numpy(), k if group == -1 else group, axis=1)
-    w = np.abs(spread(st) * (o.slice_codes(q, bits).astype(np.float64) * (1 << (8 - bits)) - spread(zt)))
-    reach = x.double().abs() @ torch.from_numpy(w).cuda().T
+    w = torch.from_numpy(spread(st) * (o.slice_codes(q, bits).astype(np.float64) * (1 << (8 - bits)) - spread(zt))).cuda()
+    reach = x.double().abs() @ w.abs().T
+    # against weights that are not rounded: half a step of each weight besides, and (fp16 storage) of scale times zero point
+    shift = torch.from_numpy(spread(st) * np.abs(spread(zt) - 128.0)).cuda()
+    half = 2.0 ** (-8 if bf16 else -11)
+    weights = half * reach if bf16 else half * (reach + x.double().abs() @ shift.T)
+    exact = x.double() @ w.T
+    assert torch.all((y - exact).abs() <= half * exact.abs() + weights + 2.0 ** -20 * reach + 2.0 ** -24)
     assert torch.all((y - ref).abs() <= 2.0 ** (-7 if bf16 else -10) * ref.abs() + 2.0 ** -20 * reach + 2.0 ** -24)
