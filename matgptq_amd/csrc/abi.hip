@@ -227,8 +227,8 @@ int make_plan(int bits, int group_size, int64_t N, int64_t K, int64_t M, bool zp
         const double t_128 = rounds(wgs_128);
         p->cfg = t_192 < t_128 && fits_192 ? 9 : 3;
         // One round of 128 x 192 tiles, where 128 x 128 tiles need a second one, pays for every format but 3 bits of bf16
-        // storage at group size 32 with zero points (0.6), also for those that lose where rounds are many: 1.17 over 1535
-        // random calls, none slower.  Both widths in one launch where they take every slot once: 1.27 over 3041 against 128 x 128
+        // storage at group size 32 with zero points (0.6), also for those that lose where rounds are many: 1.19 over 724
+        // random calls, none slower.  Both widths in one launch where they take every slot once: 1.27 over 1323 against 128 x 128
         // or 128 x 192 tiles, 1.03 to 1.13 against the latter alone (bf16 storage, and 6 bits without a scale per tile).
         if (wgs_192 <= 512 && wgs_128 > 512 && !(bits == 3 && bf16 && g32zp)) {
           int narrow = 0;
@@ -354,15 +354,16 @@ int make_plan(int bits, int group_size, int64_t N, int64_t K, int64_t M, bool zp
         }
       }
       // Formats whose registers do not hold the 128 x 256 tile take the 128 x 192 tile with K split in place of the 128 x 128 tile:
-      // 1.26 over 2358 random calls, none slower.  (6-bit codes on fp16 storage with a scale per tile stay where they were: their
+      // 1.27 over 1267 random calls, none slower.  (6-bit codes on fp16 storage with a scale per tile stay where they were: their
       // results are left bit for bit as they were, which nothing depends on.)
       if (!p->skinny && p->cfg == 3 && wgs_192s <= 256 && t_192s < best && !fixed_order) p->cfg = 13;
       // The 64 x 128 tile on few of the CUs: workgroups of the mid-batch kernel a quarter or a half as large take more of them.
-      // Up to 96 of the tiles, 2090 random calls of 97 to 640 batch rows: 1.33 with 32 x 32 (2 % lost more than 2 %) and, where 64
-      // batch rows pad no more, 1.21 with 64 x 64 (8-bit codes, two row blocks at most, 0.93 that way, and 0.76 to 0.9 on walks of three tiles with
+      // Up to 96 of the tiles, 960 random calls of 97 to 640 batch rows: 1.32 with 32 x 32 (but for 6 bits with zero points at
+      // group size 32 on 9 and 10 K tiles, 0.89 to 1.1) and, where 64 batch rows pad no more, 1.24 with 64 x 64 (8-bit codes, two row blocks at most, 0.93 that way, and 0.76 to 0.9 on walks of three tiles with
       // 32 x 32: not those); more batch rows on fewer row blocks 0.76 to 1; 97 to 128 of the tiles 0.95 to 1.2.
       // (Not fp16 storage with a scale per tile, as above.)
-      if (variant == 0 && !p->skinny && p->cfg == 16 && M > 96 && M <= 640 && !(bits == 8 && k_tiles <= 24) && !fixed_order &&
+      if (variant == 0 && !p->skinny && p->cfg == 16 && M > 96 && M <= 640 && !(bits == 8 && k_tiles <= 24) &&
+          !(bits == 6 && group_size == 32 && zp && (k_tiles == 9 || k_tiles == 10)) && !fixed_order &&
           ((N + 127) / 128) * ((M + 63) / 64) <= 96) {
         p->skinny = p->sliced_only = true;
         const bool tall = r_max == 4 && ((M + 63) / 64) * 64 * 7 <= ((M + 31) / 32) * 32 * 8;

@@ -17,15 +17,14 @@
 //  * What bounds it: the copies of the activations, which every workgroup repeats, and HBM.  On layers with one row block per
 //    CU and a long K the copies are most of the traffic of a CU (4096 x 14336 at M = 16: 458 KB beside 115 KB of codes).
 //
-// Measured against what ran before, weights cold, us (mid-batch kernel; * gemv kernel, which stages activations through
+// Measured against what ran before, weights from HBM, us (mid-batch kernel; * gemv kernel, which stages activations through
 // registers once per wave and row block):
-//   28672 x 4096  3 bits bf16  M = 8  17.9 -> 12.7    4 bits fp16  M = 8  16.1 -> 14.2,  M = 16  16.9 -> 15.5
-//    4096 x 14336 3 bits bf16  M = 8  11.1* -> 9.4    4 bits fp16  M = 16 13.2 -> 12.9
-//    4096 x 4096  3 bits bf16  M = 8   5.4* -> 4.5    4 bits fp16  M = 16  5.8 -> 5.4
-//    8192 x 3584  4 bits fp16  M = 16  7.2 -> 6.7     1280 x 8192  4 bits fp16  M = 16  7.8 -> 7.0
-// and over 10000 random calls (every bitwidth and storage type, K = 256 .. 16384, M = 5 .. 16) 1.08 to 1.45 times faster on
-// the geometric mean of each format, slower by more than 1.5 % on one in a thousand.
-// Seventeen to 64 batch rows: the rule in fewrows_plan.h says where and by how much.
+//   28672 x 4096  3 bits bf16  M = 8  20.6 -> 14.9    4 bits fp16  M = 8  19.6 -> 14.8,  M = 16  19.7 -> 15.6
+//    4096 x 14336 3 bits bf16  M = 8  11.3* -> 9.4    4 bits fp16  M = 16 14.5 -> 12.7
+//    4096 x 4096  3 bits bf16  M = 8   5.6* -> 4.6    4 bits fp16  M = 16  6.0 -> 5.4,   M = 24   7.4 -> 5.9
+//    8192 x 3584  4 bits fp16  M = 16  7.7 -> 6.4     1280 x 8192  4 bits fp16  M = 16  8.5 -> 7.7
+//    6144 x 4096  4 bits bf16  M = 32  9.4 -> 8.4     1024 x 4096  4 bits bf16  M = 64  7.4 -> 5.1
+// The rule in fewrows_plan.h says for which calls and by how much over random ones.
 // Tried and taken back: 64 batch rows per workgroup (no faster than two workgroups of 32), activations loaded straight into
 // the operand (16 rows x 64 bytes per load: 4096 x 14336 at M = 16 13 -> 17 us), four buffers and everything requested at the
 // start (28672 x 4096: within 3 % either way), sixteen waves (ahead only below 5 rows on walks past 8192 columns), consecutive
@@ -75,15 +74,12 @@ few_rows_kernel(const GemmArgs a, int n_tiles, int m_tiles) {
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r16 = lane & 15;
   const int q = lane >> 4;
-  // Workgroup ids go round-robin over the 8 XCDs: remapped so that the workgroups of one XCD are neighbours, which walk the
-  // blocks of batch rows of the same weight rows and share these in its L2.  With several blocks of batch rows 1.08 to 1.1 on counts
-  // that are not a multiple of 8 (17 to 64 rows, geometric mean).  With a single one, 9 to 16 batch rows on up to 100 row blocks of
-  // four K tiles took, in us, remapped 2.36 where the count is a multiple of 8 and 2.83 where it is not, as they come 2.81 and 2.43.
-  // (Why is not known; the mid-batch kernel shows the first of the two.)
-  const int total = n_tiles * m_tiles;
+  // Workgroup ids go round-robin over the 8 XCDs: with several blocks of batch rows they are remapped so that the workgroups
+  // of one XCD walk those blocks of the same weight rows and share these in its L2 (against ids as they come: two blocks of
+  // batch rows 1.05, three 1.08, four 1.12 on the geometric mean of 10000 random calls; a single one the same either way).
   int lid = blockIdx.x;
-  if (m_tiles > 1 || (total & 7) == 0) {
-    const int xcd = blockIdx.x & 7, rest = total & 7;
+  if (m_tiles > 1) {
+    const int total = n_tiles * m_tiles, xcd = blockIdx.x & 7, rest = total & 7;
     lid = xcd * (total >> 3) + (xcd < rest ? xcd : rest) + (blockIdx.x >> 3);
   }
   const int nt = lid / m_tiles;
@@ -119,8 +115,8 @@ few_rows_kernel(const GemmArgs a, int n_tiles, int m_tiles) {
   };
 
   // codes, scales and zeros of the tile in use and of the next one (scales and zeros as loaded).  Codes have the policy of data
-  // that is read once also where workgroups for other batch rows read them again: with the default one 17 to 64 rows take 1 %
-  // longer and one block of rows 5 % (geometric means over 35000 random calls).
+  // that is read once also where workgroups for other batch rows read them again: with the default one, one block of batch rows
+  // takes 6 % longer, two the same, three and four 1 and 2 % less (geometric means over 13000 random calls).
   uint32_t wr[kSets][R][Fmt::kWords], sr[kSets][R], zr[kSets][R];
   auto load_weights = [&](uint32_t (&w)[R][Fmt::kWords], uint32_t (&s)[R], uint32_t (&z)[R], int kb) {
 #pragma unroll

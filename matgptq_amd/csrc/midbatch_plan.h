@@ -10,7 +10,7 @@ namespace matgptq {
 // 64 KB, the second workgroup of a CU.  One against two buffers on some 15000 random calls (M = 5..128, K = 256..8192, all bitwidths,
 // groups and storage types; mean gain, share that lost more than 1.5 %):
 //  * walks of one tile have nothing to fetch ahead: one buffer and one register set, the next workgroup of the CU instead
-//    (64 rows per workgroup 1.27 to 1.36 times faster than with two, 32 rows 1.03 to 1.08);
+//    (1.07 to 1.14 times faster than with two, planes 1.18 to 1.25, over 10300 random calls of 5 to 96 batch rows, none slower);
 //  * one row block and 16 batch rows: two or three tiles 6.7 %, 0.1 %; longer walks 5 %, 1 % (4096 x 4096 at M = 12:
 //    5.53 -> 5.28 us) without group 32 with zero points (0 to 2 %, 7 %: four scales and zeros per tile in two sets) and
 //    without even walks at 6 bits (2.5 %, 17 %);

@@ -443,7 +443,7 @@ def test_planner_answers_every_valid_shape_within_its_kernels_domains():
         elif kind == "prefill":
             assert m > 16, plan
         else:
-            assert kind == "decode-burst" and b == 8 and n > 32000 and k <= 256 and 4 < m <= 16, plan
+            assert kind == "decode-burst" and b == 8 and n > 40000 and k <= 256 and 4 < m <= 16, plan
     assert seen == {"gemv", "fewrows", "midbatch", "decode-burst", "prefill"}
 
 
@@ -492,10 +492,10 @@ def test_few_rows_at_the_edges_of_the_rule():
     assert [few(4, g, 256, 1024, m, plain, 0) for g, m in ((128, 1), (128, 4), (128, 5), (-1, 1))] == [0, 0, 1, 1]
     # one and two rows: short walks on few row blocks, long ones of planes on many
     at = lambda m, flags, planes, *sizes: [few(4, 128, 16 * n, 128 * k, m, flags, planes) for n, k in sizes]
-    assert at(1, bf16, 0, (256, 10), (257, 10), (256, 11), (257, 4), (257, 5), (512, 8), (513, 8), (257, 9)) == [1, 0, 0, 0, 1, 1, 0, 0]
+    assert at(1, bf16, 0, (256, 4), (257, 4), (257, 5), (512, 8), (513, 8), (256, 9)) == [1, 0, 1, 1, 0, 0]
     assert at(1, plain, 1, (600, 16), (601, 16), (256, 24), (257, 17), (256, 25)) == [1, 0, 1, 0, 0]
-    assert at(1, plain, 1, (1024, 51), (1025, 50), (1025, 51), (1025, 80), (1025, 81)) == [0, 0, 1, 1, 0]
-    assert at(2, bf16, 0, (400, 24), (401, 24), (400, 25), (800, 8), (801, 8)) == [1, 0, 0, 1, 0]
+    assert at(1, plain, 1, (1024, 51), (1025, 50), (1025, 51), (1025, 64), (1025, 65)) == [0, 0, 1, 1, 0]
+    assert at(2, bf16, 0, (400, 24), (401, 24), (400, 25), (640, 8), (641, 8)) == [1, 0, 0, 1, 0]
     assert at(2, plain, 1, (600, 24), (601, 24), (1024, 8), (1025, 8)) == [1, 0, 1, 0]
     assert at(2, plain, 1, (800, 51), (801, 50), (801, 51), (801, 120), (801, 121)) == [0, 0, 1, 1, 0]
     # three and four rows: everything but long walks on few row blocks and 9 to 16 K tiles on many
@@ -505,7 +505,7 @@ def test_few_rows_at_the_edges_of_the_rule():
     assert at(4, plain, 1, (320, 60), (320, 61), (2200, 9), (2201, 9), (2201, 17)) == [2, 0, 2, 0, 2]
     # five and more: everything but many rows of one or two K tiles at 8 bits of fp16 storage
     many = lambda n, k, bits=8, flags=plain, planes=0: few(bits, 128, 16 * n, 128 * k, 9, flags, planes)
-    assert [many(2000, 2), many(2001, 2), many(2001, 3), many(2001, 2, 6), many(2001, 2, 8, bf16), many(2001, 2, 8, plain, 1)] == [2, 0, 2, 4, 2, 2]
+    assert [many(2500, 2), many(2501, 2), many(2501, 3), many(2501, 2, 6), many(2501, 2, 8, bf16), many(2501, 2, 8, plain, 1)] == [2, 0, 2, 4, 2, 2]
     assert [few(4, -1, 16 * n, 4096, 8, plain, 0) for n in (1, 319, 320, 512, 513, 636, 637)] == [1, 1, 2, 2, 2, 2, 4]
     assert [few(4, 128, 16 * n, 4096, 9, plain, 0) for n in (318, 319, 636, 637)] == [1, 2, 2, 4]
     assert [few(b, 128, 65536, 4096, 16, plain, p) for b, p in ((6, 0), (8, 0), (4, 1), (6, 1))] == [4, 2, 4, 2]
@@ -514,9 +514,9 @@ def test_few_rows_at_the_edges_of_the_rule():
     assert of(64, (3, 6, 8), (160, 161, 192, 193, 256, 257, 384, 385)) == [1, 1, 1, 0, 0, 0, 0, 0, 1, 1, 1, 2, 2, 2, 2, 0, 1, 0, 0, 0, 0, 2, 2, 0] and of(17, (9, 128), (128,)) == [1, 1]
     assert of(32, (9, 17, 24, 25), (129, 256)) == [0, 0, 0, 0, 0, 0, 2, 2] and of(32, (16, 17), (257, 512)) == [0, 0, 2, 2]
     assert of(17, (9, 17, 25), (513, 1024, 1025, 2048, 4000)) == [4, 4, 0, 0, 0, 4, 4, 8, 8, 0, 4, 4, 8, 8, 8] and of(17, (25,), (2048, 2049), flags=plain) == [8, 0]
-    assert of(17, (17, 32, 33), (1024, 4000), bits=6, flags=plain) == [4, 0, 4, 0, 4, 4] and of(22, (25,), (129,), bits=6) == [0] and of(23, (25,), (129,), bits=6) == [2]
-    assert of(64, (1,), (120, 121, 192), flags=plain) == [1, 0, 0] and of(64, (1,), (192,)) == [1] and of(17, (17,), (513, 4000), bits=8) == [0, 0]
-    assert of(17, (17,), (513, 1025), planes=1) == [4, 0] and [of(m, (25,), (129, 513), bits=b, planes=1) for m, b in ((20, 4), (21, 4), (21, 6))] == [[0, 4], [2, 4], [0, 0]]
+    assert of(17, (17, 24, 25), (1024, 4000), bits=6, flags=plain) == [4, 0, 4, 0, 4, 4]
+    assert of(64, (1,), (140, 141, 192), flags=plain) == [1, 0, 0] and of(64, (1,), (192,)) == [1] and of(17, (17,), (513, 4000), bits=8) == [0, 0]
+    assert of(17, (17,), (513, 1025), planes=1) == [4, 0] and [of(17, (25,), (129, 513), bits=b, planes=1) for b in (4, 6)] == [[2, 4], [0, 0]]
     assert of(33, (9,), (85, 86, 128, 129, 170, 171, 256, 257, 340, 341)) == [1, 0, 0, 2, 2, 0, 0, 4, 4, 0]
     assert of(49, (9, 17), (64,)) == [0, 1] and of(49, (9,), (65, 256, 257, 512, 513)) == [0, 0, 4, 4, 0] and of(64, (17,), (128, 129, 256, 257)) == [0, 2, 2, 4]
     assert of(49, (40, 41), (257,)) == [4, 4] and of(49, (40, 41), (257,), flags=plain) == [4, 0]
@@ -566,4 +566,5 @@ def test_planner_gives_the_wider_formats_192_rows_and_few_64_row_tiles_smaller_w
     assert [plan(4, 32, n, 4096, 192, True, 1) for n in (4096, 4112)] == ["R2 mb2", "cfg16"]
     assert [plan(4, 32, 1024, 4096, m, True, 1) for m in (640, 641)] == ["R2 mb2", "cfg16"]
     assert [plan(8, 32, 4096, k, 192, True, 1) for k in (3072, 3200)] == ["cfg16", "R2 mb2"]
+    assert [plan(6, 32, 4096, k, 192, zp, 1) for k, zp in ((1280, True), (1280, False), (1408, True))] == ["cfg16", "R2 mb2", "R2 mb2"]
     assert _lib.load().matgptq_gemm_master_workspace_bytes(4, 32, 4096, 4096, 192, 1) == 4 * 4096 * 4096 // 8
