@@ -14,8 +14,10 @@
 //    the operand of bf16 storage carries besides the code, multiply sums of activations only: chains of four MFMAs against
 //    constants per tile, shared by the R row blocks, whose result is the start value of the code chain.  No weight is rounded:
 //    the error against 64 bits is that of the result's rounding (fp16 2.1e-4, 2.8e-4 with rounded weights; bf16 1.7e-3, 2.2e-3).
-//  * What bounds it: the copies of the activations, which every workgroup repeats, and HBM.  On layers with one row block per
-//    CU and a long K the copies are most of the traffic of a CU (4096 x 14336 at M = 16: 458 KB beside 115 KB of codes).
+//  * What bounds it: no unit alone.  28672 x 4096, 3 bits bf16, M = 8 (13.8 us): HBM 3.4 TB/s, vector issue 0.41, L2 5.6 TB/s;
+//    4096 x 14336 (9.7 us): 2.6, 0.29, 8.6.  It is the chain of a wave (copy, operands, products, sums) over the few tiles of
+//    its walk, and the copies of the activations, which every workgroup repeats: on layers with one row block per CU and a long K
+//    most of the traffic of a CU (4096 x 14336 at M = 16: 458 KB beside 115 KB of codes).
 //
 // Measured against what ran before, weights from HBM, us (mid-batch kernel; * gemv kernel, which stages activations through
 // registers once per wave and row block):
