@@ -600,11 +600,12 @@ hipError_t launch_few_rows(int bits, bool bf16, const GemmArgs& a, int g, FewRow
 #undef MATGPTQ_CASE
 }
 
-// Workgroup of the few-rows kernel where a call without a forced variant takes it, else no row blocks.  `x` (or nullptr: as if
-// aligned): the kernel copies the activations into LDS in pieces of 16 bytes; off those, the kernels that ran before it do,
-// of which the gemv kernel loads them into registers.
+// Workgroup of the few-rows kernel where a call takes it that forces no variant and asks the gemv kernel for no waves or LDS,
+// else no row blocks.  `x` (or nullptr: as if aligned): the kernel copies the activations into LDS in pieces of 16 bytes; off
+// those, the kernels that ran before it do, of which the gemv kernel loads them into registers.
 FewRows few_rows_of(int bits, int group_size, int64_t N, int64_t K, int64_t M, const void* x, uint32_t flags, bool master) {
-  if ((flags & (MATGPTQ_FLAG_VARIANT_MASK | MATGPTQ_FLAG_FLAVOUR_MASK)) != 0 || M > kFewRowsMaxM) return {0, 0};
+  constexpr uint32_t gemv_bits = 31u << MATGPTQ_FLAG_GEMV_WAVES_SHIFT | 63u << MATGPTQ_FLAG_GEMV_LDS_SHIFT;
+  if ((flags & (MATGPTQ_FLAG_VARIANT_MASK | MATGPTQ_FLAG_FLAVOUR_MASK | gemv_bits)) != 0 || M > kFewRowsMaxM) return {0, 0};
   if (reinterpret_cast<uintptr_t>(x) % 16 != 0) return {0, 0};
   return few_rows(bits, group_size, (flags & MATGPTQ_FLAG_BF16) != 0, master, (int)M, (int)(N / 16), (int)(K / 128));
 }

@@ -488,6 +488,10 @@ def test_few_rows_at_the_edges_of_the_rule():
     assert few(5, 128, 4096, 4096, 8, plain, 0) < 0 and few(4, 128, 4096, 4096, 0, plain, 0) < 0
     assert few(4, 32, 4096, 4096, 8, plain, 0) == 0 and few(4, 32, 256, 4096, 17, bf16, 0) == 0 and few(4, 128, 256, 1024, 65, bf16, 0) == 0
     assert few(4, 128, 4096, 4096, 8, plain | (80 << 8), 0) == 0 and few(4, 128, 4096, 4096, 8, plain | (1 << 16), 0) == 0
+    # waves or LDS asked of the gemv kernel keep a call with it, and the plan shows them
+    plan = lambda flags: _lib.describe_plan(4, -1, 256, 1024, 2, False, flags)
+    assert plan(plain).startswith("fewrows") and plan(plain | (3 << 18)).startswith("gemv") and "W3" in plan(plain | (3 << 18))
+    assert few(4, -1, 256, 1024, 2, plain | (1 << 23), 0) == 0 and few(4, -1, 256, 1024, 2, plain | (31 << 18), 1) == 0
     # up to four rows of fp16 storage at group 128: the gemv kernel, as with a fused prologue
     assert [few(4, g, 256, 1024, m, plain, 0) for g, m in ((128, 1), (128, 4), (128, 5), (-1, 1))] == [0, 0, 1, 1]
     # one and two rows: short walks on few row blocks, long ones of planes on many
