@@ -67,9 +67,11 @@ class MatGPTQLinear(torch.nn.Module):
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         # The product has no gradient.  Grad mode is switched off only where a tensor would ask for one: as a decorator the
-        # switch was 1.2 of the 8 us that a call on a few rows takes, which is all host time.
+        # switch was 1.2 of the 8 us that a call on a few rows takes, which is all host time.  (What stands for a
+        # tensor while a graph is recorded has no answer to the question.)
         scales, zeros = self.matgptq_scales, self.matgptq_zeros
-        if torch.is_grad_enabled() and (x.requires_grad or scales.requires_grad or (zeros is not None and zeros.requires_grad)):
+        if torch.is_grad_enabled() and isinstance(x, torch.Tensor) and (
+                x.requires_grad or scales.requires_grad or (zeros is not None and zeros.requires_grad)):
             with torch.no_grad():
                 return self._product(x, scales, zeros)
         return self._product(x, scales, zeros)

@@ -34,6 +34,19 @@ def test_python_names_of_the_reference_package():
     assert set(["matgptq_qweight", "matgptq_scales"]) <= set(MatGPTQLinear.__init__.__code__.co_names) | {"matgptq_qweight", "matgptq_scales"}
 
 
+@pytest.mark.parametrize("zeros", (False, True))
+def test_module_can_be_recorded_into_a_graph(monkeypatch, zeros):
+    # (with grad mode on: what stands for a tensor meanwhile cannot be asked whether it requires a gradient)
+    ops = torch.ops.matgptq_cuda
+    monkeypatch.setattr(ops, "pack_matgptq_qweights", lambda q, *_: q.clone())
+    monkeypatch.setattr(ops, "reorder_matgptq_scales", lambda t, *_: t.clone())
+    s = torch.rand(16, 1).half()
+    lin = MatGPTQLinear(torch.zeros(16, 128, dtype=torch.uint8), s, 4, 128, zeros=s if zeros else None, perm=torch.arange(128))
+    assert torch.is_grad_enabled()
+    names = [str(node.target).split(".")[-1] for node in torch.fx.symbolic_trace(lin).graph.nodes]
+    assert [t for t in names if t.startswith("matmul_matgptq")] == ["matmul_matgptq_zp" if zeros else "matmul_matgptq"]
+
+
 def test_fake_shapes():
     # (input.shape[-2], N), bf16 iff flag bit 1 (inference_lib/matgptq_cuda/__init__.py:49-63)
     with torch.device("meta"):
