@@ -221,8 +221,9 @@ Tensor matmul_impl(const Tensor& input, const Tensor& weights, const Tensor& sca
   c10::hip::HIPGuardMasqueradingAsCUDA guard(dev);
   Tensor out = torch::empty({m, n_out_features}, input.options());
   if (m == 0) return out;
-  // (a view that starts off 16 bytes: most kernels copy the activations into LDS in pieces of that size)
-  if (reinterpret_cast<uintptr_t>(input_c.data_ptr()) % 16 != 0) input_c = input_c.clone();
+  // (a view that starts off 16 bytes: from five rows on the kernels copy the activations into LDS in pieces of that size;
+  // up to four rows the gemv kernel loads such views into registers, and a copy would be a second launch)
+  if (m > 4 && reinterpret_cast<uintptr_t>(input_c.data_ptr()) % 16 != 0) input_c = input_c.clone();
   const uint32_t flags = (uint32_t)feature_flag | MATGPTQ_FLAG_ASYNC;
   int code;
   if (master) {
