@@ -753,7 +753,7 @@ int matgptq_gemm_prologue(int bitwidth, int group_size, int64_t N, int64_t K, in
   return MATGPTQ_OK;
 }
 
-// does the GEMM at this shape read the planes itself (gemv and mid-batch kernels), or does it need
+// does the GEMM at this shape read the planes itself (gemv, few-rows and mid-batch kernels), or does it need
 // the pre-sliced tensor in a workspace first?
 // `flags` comes back with the plan to take: up to 128 batch rows a shape whose own plan needs the
 // workspace is given the mid-batch kernel instead (its largest shape for that batch size), which

@@ -558,7 +558,8 @@ int main() {
 
 def test_planner_gives_the_wider_formats_192_rows_and_few_64_row_tiles_smaller_workgroups():
     plan = lambda *a: _lib.describe_plan(*a).split(" zp")[1][2:]
-    # one round of 128 x 192 tiles with K split where the 128 x 256 tile spills; not 6 bits with the order of sums kept
+    # one round of 128 x 192 tiles with K split where the 128 x 256 tile spills; not 6 bits of fp16 storage at group 128, which are
+    # left as they were
     assert [plan(6, g, 5984, 4096, 1024, True, f) for g, f in ((-1, 1), (32, 1), (128, 3), (128, 1))] == ["cfg13", "cfg13", "cfg13", "cfg3"]
     assert plan(6, -1, 6160, 4096, 1024, True, 1) == "cfg3"
     # one round of 128 x 192 tiles where 128 x 128 tiles need two, mixed with these where slots stay empty
